@@ -108,7 +108,8 @@ class HIPEvaluator:
 
     def last_dag_shape(self):
         """Product-DAG launch of the last call: (parts per tile, tail tiles,
-        kernel: 0 / 1 the record kernel on 64 / 32-environment tiles, else the
+        kernel: 0 the pair kernel, or the segment kernel on 64-environment
+        tiles, 1 the segment kernel on narrower ones, else the
         run interpreter's environments per tile)."""
         p, t, k = C.c_int(), C.c_int64(), C.c_int()
         _lib.check(self.lib.ace_last_dag_shape(self.ctx, C.byref(p), C.byref(t), C.byref(k)))
@@ -135,8 +136,8 @@ class HIPEvaluator:
         _lib.check(self.lib.ace_set_pool_shape(self.ctx, int(chunk), int(envs_per_wave)))
 
     def set_kernel(self, mode: int = 0):
-        """Product-DAG kernel: 0 the record-segment kernel where the basis
-        allows it (default), 1 the run interpreter always, 2 the per-record
+        """Product-DAG kernel: 0 the pair kernel or the record-segment
+        kernel, whichever takes the basis (default), 1 the run interpreter always, 2 the per-record
         dispatch kernel over the same records (comparison)."""
         _lib.check(self.lib.ace_set_kernel(self.ctx, int(mode)))
 

@@ -4,7 +4,8 @@
 // launchers one unit calls in another.
 //
 // Units: acehip.hip (context, product DAG, energy entry points),
-// ace_pool.hip (1p basis and pooling), ace_force.hip (adjoint force
+// ace_pairs.hip (pair kernel: the product DAG of Invariant bases of
+// order 3 and 4), ace_pool.hip (1p basis and pooling), ace_force.hip (adjoint force
 // kernels), ace_basis.hip (basis-level evaluate / evaluate_d,
 // adjoint_EVAL_D), ace_surr.hip (learned-surrogate support).
 #pragma once
@@ -24,6 +25,7 @@
 #include "../../include/acehip.h"
 #include "host_util.hpp"
 #include "pack_host.hpp"
+#include "pairs_host.hpp"
 
 #define ACE_LMAX 10
 #define ACE_NPMAX ((ACE_LMAX + 1) * (ACE_LMAX + 2) / 2)
@@ -243,6 +245,19 @@ constexpr int FF_MAXE = 16;
 constexpr int FF_MAXE_WIDE = 32;
 constexpr size_t FF_LDS = 40 * 1024;
 
+// The pair kernel (ace_pairs.hip): most pooled values whose A+ and G rows fit
+// the LDS (1024 bytes per value and the constant, 160 KB), and the columns
+// above which a panel is cut (columns of one panel run one after another, so
+// the longest bounds a round; every cut repeats the panel's rows).
+constexpr int PAIR_MAX_POOL = 159;
+constexpr int PAIR_CAP = 96;
+struct PairDev {
+    acehost::PairProgram host;
+    DevBuf<uint32_t> words;
+    DevBuf<double> coef;
+    DevBuf<int32_t> seq[acehost::PAIR_MAXP + 2];
+};
+
 struct ForceFlatTab {
     int8_t nrl[ACE_LMAX + 1];  // n bound per l
     int16_t nq;  // number of (l, m, n) entries (their G slots in staging order: ace_ctx::ffq)
@@ -266,6 +281,9 @@ struct ace_ctx {
     int rec_et = 0;
     int seg_et = 0;
     bool force_interp = false;
+    // pair kernel programs (energy + forces, energy only) of bases it takes
+    bool pairs_ok = false;
+    PairDev pairs[2];
     // rec_dispatch: the record kernel that switches per record (ace_set_kernel
     // mode 2) instead of the segment kernel
     bool rec_dispatch = false;
@@ -296,6 +314,7 @@ struct ace_ctx {
     DevBuf<BtRec> bt_rec;
     DevBuf<int32_t> bt_rowo;  // [nB][BT_ROWO] record ranges per order
     DevBuf<int32_t> ffq;  // G slots of the flat force kernel's staged (l, m, n) entries
+    DevBuf<int32_t> ffk;  // their pooled functions (the pair kernel's G rows)
     DevBuf<int16_t> kidx;
     int nrl[ACE_LMAX + 1] = {0};  // n bound per l over the pooled functions
     // flat force kernel (Invariant, one species, nr <= 16): slot table and the
@@ -372,6 +391,10 @@ struct Workspace {
     double* Epart = nullptr;
     int32_t* nbr_env = nullptr;
     size_t nbr_cap = 0;  // entries nbr_env holds
+    // G layout: 0 the slots of the programs; P >= 1 the pair kernel's shares
+    // [part][npool][estride], P of them (P + 1 for environments from genv_hi on)
+    int gparts = 0;
+    int64_t genv_hi = 0;
 };
 
 // The context's own buffers (as sized by their last ensure).
@@ -436,6 +459,13 @@ int validate_inputs(ace_ctx* ctx, int64_t nenv, const int32_t* off, int64_t nnbr
 // (device count env_count): energies, and the adjoint G with forces.
 int launch_dag_listed(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, bool forces, double* E_out,
                       const int32_t* env_list, const int32_t* env_count);
+// ace_pairs.hip: the pair programs at context creation (sets pairs_ok), their
+// coefficients, and the launch: energies, and with forces the G shares of P
+// workgroups per tile of 32 environments (P + 1 for the last nhi tiles).
+int pairs_create(ace_ctx* ctx, const std::vector<int32_t>& pool);
+int pairs_set_coeffs(ace_ctx* ctx, const std::vector<double>& leaf);
+int launch_pairs(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, bool forces, int P, int64_t nhi,
+                 const Workspace& ws, double* E_out);
 // ace_pool.hip: A+[k][env] into ws.Aplus (stride estride); with nbr_map
 // also the neighbour -> environment map ws.nbr_env (flat force kernel).
 int launch_pool_any(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* off, const double* xyz,

@@ -17,6 +17,23 @@ namespace {
 // ---------------------------------------------------------------------------
 // k_force: +dE/dr_j = Re sum_k G[k] grad(R_n Y_lm)(r_j)
 
+// The pair kernel's G: parts shares of every row (one more from env_hi on),
+// stride apart; parts = 0: the programs' slots.
+struct GParts {
+    int parts;
+    int64_t env_hi, stride;
+    __device__ __forceinline__ double2 sum(const double2* __restrict__ p, int64_t env) const {
+        double2 g = *p;
+        const int n = env >= env_hi ? parts + 1 : parts;
+        for (int q = 1; q < n; ++q) {
+            const double2 v = p[(int64_t)q * stride];
+            g.x += v.x;
+            g.y += v.y;
+        }
+        return g;
+    }
+};
+
 // The NC components of G[k] for one environment: sums over k's slots.  With
 // class-split programs (gcls set) a slot holds one complex value of class
 // gcls[slot] (read once), and component p is sum_slots cls_u[class][p] * value.
@@ -25,9 +42,13 @@ __device__ __forceinline__ void gather_g(const int32_t* __restrict__ gslot_ptr,
                                          const int32_t* __restrict__ gslot_list,
                                          const int32_t* __restrict__ gcls, const double2* __restrict__ cls_u,
                                          const double2* __restrict__ Gbuf, int64_t estride, int64_t env, int k,
-                                         double2 (&g)[NC]) {
+                                         const GParts& gp, double2 (&g)[NC]) {
 #pragma unroll
     for (int p = 0; p < NC; ++p) g[p] = make_double2(0.0, 0.0);
+    if (NC == 1 && gp.parts > 0) {
+        g[0] = gp.sum(Gbuf + (int64_t)k * estride + env, env);
+        return;
+    }
     for (int s = gslot_ptr[k]; s < gslot_ptr[k + 1]; ++s) {
         const int slot = gslot_list[s];
         if (NC > 1 && gcls) {
@@ -95,7 +116,7 @@ __global__ __launch_bounds__(64) void k_force_lds(RadialParams rp, int64_t nenv,
                                                const int32_t* __restrict__ gslot_list,
                                                const int32_t* __restrict__ gcls,
                                                const double2* __restrict__ cls_u,
-                                               const double2* __restrict__ Gbuf, int64_t estride,
+                                               const double2* __restrict__ Gbuf, int64_t estride, GParts gp,
                                                double* __restrict__ dE) {
     constexpr int NP = (L + 1) * (L + 2) / 2;
     constexpr int NC = PROP == 0 ? 1 : 3;
@@ -108,7 +129,7 @@ __global__ __launch_bounds__(64) void k_force_lds(RadialParams rp, int64_t nenv,
     if (env >= nenv) return;
     for (int k = lane; k < npool; k += 64) {
         double2 g[NC];
-        gather_g<NC>(gslot_ptr, gslot_list, gcls, cls_u, Gbuf, estride, env, k, g);
+        gather_g<NC>(gslot_ptr, gslot_list, gcls, cls_u, Gbuf, estride, env, k, gp, g);
 #pragma unroll
         for (int p = 0; p < NC; ++p) Gs[k * NC + p] = g[p];
     }
@@ -218,7 +239,7 @@ __global__ __launch_bounds__(64) void k_force(RadialParams rp, ForceTab ft, int6
                                                const int32_t* __restrict__ gslot_list,
                                                const int32_t* __restrict__ gcls,
                                                const double2* __restrict__ cls_u,
-                                               const double2* __restrict__ Gbuf, int64_t estride,
+                                               const double2* __restrict__ Gbuf, int64_t estride, GParts gp,
                                                double* __restrict__ dE) {
     constexpr int NP = (L + 1) * (L + 2) / 2;
     constexpr int NC = PROP == 0 ? 1 : 3;
@@ -234,7 +255,7 @@ __global__ __launch_bounds__(64) void k_force(RadialParams rp, ForceTab ft, int6
         const int mu = max(0, pool[4 * k]), n = pool[4 * k + 1] - 1, l = pool[4 * k + 2], m = pool[4 * k + 3];
         const int d = mu * ft.spstride + ft.off[idxp(l, m)] + n * NC;
         double2 g[NC];
-        gather_g<NC>(gslot_ptr, gslot_list, gcls, cls_u, Gbuf, estride, env, k, g);
+        gather_g<NC>(gslot_ptr, gslot_list, gcls, cls_u, Gbuf, estride, env, k, gp, g);
 #pragma unroll
         for (int p = 0; p < NC; ++p) Gd[d + p] = g[p];
     }
@@ -494,7 +515,7 @@ __global__ __launch_bounds__(BS, 4) void k_forcef(RadialParams rp, ForceFlatTab 
                                                  const double* __restrict__ xyz,
                                                  const int32_t* __restrict__ nbr_env,
                                                  const int32_t* __restrict__ ffq,
-                                                 const double2* __restrict__ Gbuf, int64_t estride,
+                                                 const double2* __restrict__ Gbuf, int64_t estride, GParts gp,
                                                  double* __restrict__ dE) {
     extern __shared__ double2 Gst[];  // [q][MAXE]
     // blocks XCD-contiguous: neighbouring blocks, which stage G rows of the
@@ -512,7 +533,8 @@ __global__ __launch_bounds__(BS, 4) void k_forcef(RadialParams rp, ForceFlatTab 
         if (r0 > 0) __syncthreads();  // the previous round's reads are done
         for (int i = threadIdx.x; i < ft.nq * nre; i += BS) {
             const int qq = i / nre, ee = i - qq * nre;
-            Gst[qq * MAXE + ee] = Gbuf[(int64_t)ffq[qq] * estride + e0 + r0 + ee];
+            const int64_t env = e0 + r0 + ee;
+            Gst[qq * MAXE + ee] = gp.sum(Gbuf + (int64_t)ffq[qq] * estride + env, env);
         }
         __syncthreads();
         if (!WIDE) {
@@ -544,8 +566,13 @@ static void launch_force(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32
                          const Workspace& ws, double* dE) {
     constexpr int NC = PROP == 0 ? 1 : 3;
     constexpr int NP = (L + 1) * (L + 2) / 2;
+    const GParts gp{ws.gparts, ws.genv_hi, (int64_t)ctx->npool * estride};
     if (PROP == 0 && ctx->flat_force) {
-        if (ctx->nfold > 0)
+        // G rows: the pair kernel's (summed over its parts while staging), or
+        // slots, split ones folded into their first
+        const int32_t* gq = ws.gparts > 0 ? ctx->ffk.p : ctx->ffq.p;
+        const GParts gf{std::max(1, ws.gparts), ws.gparts > 0 ? ws.genv_hi : nenv, gp.stride};
+        if (ws.gparts == 0 && ctx->nfold > 0)
             hipLaunchKernelGGL(k_gfold, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, ctx->nfold,
                                ctx->gfold.p, ws.Gbuf, estride);
         // radial functions held in registers: 12 when they suffice (fewer
@@ -562,9 +589,9 @@ static void launch_force(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32
     do {                                                                                                        \
         const dim3 grid((unsigned)((nnbr + BS_ - 1) / BS_));                                                    \
         hipLaunchKernelGGL((k_forcef<L, NRM_, MAXE_, false, BS_>), grid, dim3(BS_), glds, st,                   \
-                           radial_params(ctx), ctx->fflat, nnbr, xyz, ne_, ctx->ffq.p, ws.Gbuf, estride, dE);   \
+                           radial_params(ctx), ctx->fflat, nnbr, xyz, ne_, gq, ws.Gbuf, estride, gf, dE);       \
         hipLaunchKernelGGL((k_forcef<L, NRM_, MAXE_, true, BS_>), grid, dim3(BS_), glds, st,                    \
-                           radial_params(ctx), ctx->fflat, nnbr, xyz, ne_, ctx->ffq.p, ws.Gbuf, estride, dE);   \
+                           radial_params(ctx), ctx->fflat, nnbr, xyz, ne_, gq, ws.Gbuf, estride, gf, dE);       \
     } while (0)
         if (ctx->nr <= 12 && wide)
             ACE_FORCEF(12, FF_MAXE_WIDE, 256);
@@ -603,7 +630,7 @@ static void launch_force(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32
         hipLaunchKernelGGL((k_force<L, PROP, NRM_>), dim3((unsigned)nenv), dim3(64), table, st, radial_params(ctx), \
                            ft, nenv, off, xyz, nnbr, ctx->nspecies > 0 ? species : nullptr, nsp, ctx->pool.p,     \
                            ctx->npool, ctx->gslot_ptr.p, ctx->gslot_list.p, gcls, ctx->cls_u.p, ws.Gbuf, estride, \
-                           dE);                                                                                   \
+                           gp, dE);                                                                                   \
     } while (0)
         // radial functions held in registers: 12 when they suffice, else 16
         if (ctx->nr <= 12)
@@ -617,7 +644,7 @@ static void launch_force(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32
     set_func_lds((const void*)k_force_lds<L, PROP>, lds);
     hipLaunchKernelGGL((k_force_lds<L, PROP>), dim3((unsigned)nenv), dim3(64), lds, st, radial_params(ctx),
                        nenv, off, xyz, nnbr, ctx->nspecies > 0 ? species : nullptr, ctx->kidx.p,
-                       ctx->npool, ctx->gslot_ptr.p, ctx->gslot_list.p, gcls, ctx->cls_u.p, ws.Gbuf, estride, dE);
+                       ctx->npool, ctx->gslot_ptr.p, ctx->gslot_list.p, gcls, ctx->cls_u.p, ws.Gbuf, estride, gp, dE);
 }
 
 }  // namespace

@@ -1,7 +1,8 @@
 // libacehip.so — MI355X (gfx950) basis-evaluation path of the Atomic Cluster
 // Expansion with ACE.jl v0.12.46 semantics.  FP64 throughout.
 //
-// Pipeline of an energy (+ forces) call:
+// Pipeline of an energy (+ forces) call (k_pairs, ace_pairs.hip, takes the place of
+// the product DAG for Invariant bases up to order 4):
 //   k_pool   (ace_pool.hip): one wave per environment (two, one per
 //              half-wave, for bases with at most 32 pooled values), lanes =
 //              neighbours.  Radial basis and m >= 0 spherical harmonics per
@@ -762,8 +763,37 @@ __global__ void k_esum(int64_t nenv, int parts, int64_t env_hi, const double* __
 // The scratch of ace_energy_forces_noalloc: a fixed device array, one copy
 // per device, held for the life of the process.  Host code reaches it only
 // through the address hipGetSymbolAddress returns (ace_ctx::scratch).
+// A batch may take ACE_SCRATCH_BYTES with one G share per slot; the pair
+// kernel's shares beyond that have ACE_SHARE_BYTES behind them, five shares of
+// any batch within the limit (A+ and one share together stay below it).
 constexpr size_t ACE_SCRATCH_BYTES = (size_t)64 << 20;
-static __device__ __align__(256) unsigned char scratch[ACE_SCRATCH_BYTES];
+constexpr size_t ACE_SHARE_BYTES = (size_t)160 << 20;
+static __device__ __align__(256) unsigned char scratch[ACE_SCRATCH_BYTES + ACE_SHARE_BYTES];
+
+// Scratch of the allocation-free entry point: A+, the G slots, the energy
+// shares, the neighbour map.
+struct ScratchNeed {
+    size_t A, G, E, N;
+    size_t all() const { return A + G + E + N; }
+};
+static size_t scratch_up(size_t b) { return (b + 255) & ~(size_t)255; }
+static ScratchNeed scratch_need(const ace_ctx* ctx, int64_t nenv, int64_t nnbr) {
+    const int64_t estride = ((nenv + 63) / 64) * 64;
+    ScratchNeed n;
+    n.A = scratch_up((size_t)ctx->npool * estride * sizeof(double2));
+    n.G = scratch_up((size_t)std::max(1, ctx->ngslots) * gslot_width(ctx) * estride * sizeof(double2));
+    n.E = ctx->seg_et > 0 || ctx->rec_et > 0
+              ? scratch_up((size_t)MAX_PARTS * (ctx->classed ? 6 : 1) * estride * sizeof(double))
+              : 0;
+    n.N = ctx->flat_force ? scratch_up((size_t)nnbr * sizeof(int32_t)) : 0;
+    return n;
+}
+// Bytes of n pair-kernel shares of G and the energies.
+static size_t share_bytes(const ace_ctx* ctx, int64_t nenv, int n) {
+    const int64_t estride = ((nenv + 63) / 64) * 64;
+    return scratch_up((size_t)n * ctx->npool * estride * sizeof(double2)) +
+           scratch_up((size_t)n * estride * sizeof(double));
+}
 
 // ---------------------------------------------------------------------------
 // host side
@@ -810,6 +840,7 @@ static int upload_coeffs(ace_ctx* ctx, const double* c) {
             ctx->seg_ptr.upload(sg.seg_ptr.data(), sg.seg_ptr.size()))
             return -1;
     }
+    if (ctx->pairs_ok && pairs_set_coeffs(ctx, cf.leaf)) return -1;
     if (ctx->task_const.upload(cf.task.data(), cf.task.size())) return -1;
     double ev[3] = {cf.e0[0], cf.e0[2], cf.e0[4]};
     if (ctx->nfeat > 0) {
@@ -1008,6 +1039,12 @@ extern "C" int ace_ctx_create(const ace_pack* pk, int device, const double* c, i
             if ((int)qslot.size() > FF_QMAX) ctx->flat_force = false;
             ctx->fflat.nq = (int16_t)std::min<size_t>(qslot.size(), FF_QMAX);
             if (ctx->flat_force && ctx->ffq.upload(qslot.data(), qslot.size())) return fail("upload");
+            // the same entries as pooled functions
+            std::vector<int32_t> kslot((size_t)std::max(1, pk->ngslots), 0), qk;
+            for (int k = 0; k < pk->npool; ++k)
+                if (pk->gslot_ptr[k + 1] > pk->gslot_ptr[k]) kslot[pk->gslot_list[pk->gslot_ptr[k]]] = k;
+            for (int32_t s : qslot) qk.push_back(kslot[s]);
+            if (ctx->flat_force && ctx->ffk.upload(qk.data(), qk.size())) return fail("upload");
             ctx->nfold = (int)fold.size() / 2;
             if (ctx->flat_force && ctx->nfold > 0 && ctx->gfold.upload(fold.data(), fold.size()))
                 return fail("upload");
@@ -1060,6 +1097,7 @@ extern "C" int ace_ctx_create(const ace_pack* pk, int device, const double* c, i
             ctx->fgrad_coef.upload(pk->fgrad_coef, ng))
             return fail("upload");
     }
+    if (pairs_create(ctx, std::vector<int32_t>(pk->pool, pk->pool + 4 * (size_t)pk->npool))) return fail("pair programs");
     if (upload_coeffs(ctx, c)) return fail("set_params");
     for (auto& e : ctx->ev)
         if (hipEventCreate(&e) != hipSuccess) return fail("event");
@@ -1114,14 +1152,13 @@ extern "C" int ace_set_params(ace_ctx* ctx, const double* c, int64_t nB) {
 }
 
 // Tail tiles for the automatic parts choice.  The grid runs in rounds of ncu
-// workgroups of equal length (1/P of a tile's work).  Giving the last n tiles
-// P + 1 parts fills the partial last round with shorter workgroups, each
-// 1/(P+1) of the work plus 8 % (re-staging and thinner task lists: measured
-// 0.200 ms per workgroup with 4 parts against 0.246 ms with 3 at 100k
+// workgroups of equal length d.  Giving the last n tiles P + 1 parts fills the
+// partial last round with shorter workgroups of length dh (segment kernel:
+// 1/(P + 1) of the tile's work plus 8 % for re-staging and thinner task lists,
+// measured 0.200 ms per workgroup with 4 parts against 0.246 ms with 3 at 100k
 // environments).  The makespan of a greedy dispatch of such workgroups onto
 // ncu units is flat over a range of n; take the middle of that range.
-static int64_t choose_tail(int64_t ntile, int P, int ncu) {
-    const double d = 1.0 / P, dh = 1.08 / (P + 1);
+static int64_t choose_tail(int64_t ntile, int P, int ncu, double d, double dh) {
     std::vector<double> h((size_t)ncu);
     auto makespan = [&](int64_t nhi) {
         // the P-part workgroups: full rounds, then r units busy one more
@@ -1146,6 +1183,91 @@ static int64_t choose_tail(int64_t ntile, int P, int ncu) {
     for (int64_t n = 0; n <= nmax; ++n)
         if (ms[(size_t)n] <= best * (1.0 + 1e-9)) ties.push_back(n);
     return ties[ties.size() / 2];
+}
+
+// The segment kernel's parts per tile when the caller leaves the choice: the
+// grid runs in rounds of ncu workgroups, and the last round may be nearly
+// empty; splitting each tile's tasks over P workgroups shortens the rounds.
+// Pick P in 1..4 minimising rounds(P) / P, with 2 % per extra part for
+// re-staging the A+ tile.  A split is only considered while every virtual wave
+// keeps at least 3 tasks (fewer leave the part workgroups unbalanced or idle).
+static int segment_parts(const ace_ctx* ctx, int64_t ntile, int ntask, int W) {
+    int pmax = 1, P = 1;
+    while (pmax < MAX_PARTS && ntask >= 3 * (pmax + 1) * W) ++pmax;
+    double best = 1e300;
+    for (int q = 1; q <= pmax; ++q) {
+        const double rounds = (double)((ntile * q + ctx->ncu - 1) / ctx->ncu);
+        const double cost = rounds / q * (1.0 + 0.02 * (q - 1));
+        if (cost < best - 1e-12) {
+            best = cost;
+            P = q;
+        }
+    }
+    return P;
+}
+
+// The pair kernel takes the call: its programs exist, no other kernel was asked
+// for (ace_set_kernel), and the programs are long enough.  Order 4: always
+// (with forces at 100,000 / 8,000 / 64 environments: degree 12 1.52 / 0.143 /
+// 0.029 ms against the segment kernel's 2.89 / 0.287 / 0.126, degree 8 0.299 /
+// 0.024 / 0.016 against 0.387 / 0.057 / 0.054).  Order 3: its rounds are few
+// and their barriers show once every CU has more than one tile (degree 10,
+// 100,000 environments 0.382 against 0.298 ms, 1,000 0.019 against 0.024), for
+// energies alone, without barriers, never (0.097 against 0.107).  Below order 3
+// the segment kernel (energies of one environment 8 against 11 us).
+static bool use_pairs(const ace_ctx* ctx, int64_t nenv, bool forces) {
+    if (!ctx->pairs_ok || ctx->force_interp || ctx->rec_dispatch) return false;
+    return ctx->maxorder == 4 || !forces || (nenv + 31) / 32 <= ctx->ncu;
+}
+
+// Workgroups per 32-environment tile of the pair kernel, and tail tiles.
+//   Up to one workgroup per CU: as many parts as the CUs take (256 order-4
+//   environments: 8 parts 0.026 ms, 2 parts 0.062, 1 part 0.110).
+//   More tiles than CUs: energies alone by the rounds' length; with forces
+//   two parts or more, whose tail tiles fill the last round at any tile
+//   count (100,000 environments: 2 parts with 64 tail tiles 1.48 ms, without
+//   1.51, 1 part 1.47 to 1.51, 3 parts 1.56; each part's G share is written
+//   and summed apart).
+// Batches that fit the allocation-free entry point take a split whose shares
+// fit it too, so that both entry points give the same bits.
+static int pair_shape(ace_ctx* ctx, int64_t nenv, bool forces, int& P, int64_t& nhi) {
+    const acehost::PairProgram& pp = ctx->pairs[forces ? 0 : 1].host;
+    const int64_t ntile = (nenv + 31) / 32;
+    // a workgroup's clocks: its rounds, and loading A+ and storing G (measured
+    // with empty rounds: 0.094 ms for 13 workgroups per CU)
+    auto clocks = [&](int q) { return pp.part_cost[(size_t)q] + (forces ? 17000.0 : 8000.0); };
+    P = ctx->parts;
+    if (P == 0) {
+        double best = 1e300;
+        const bool small = forces && scratch_need(ctx, nenv, 0).all() <= ACE_SCRATCH_BYTES;
+        for (int q = forces && ntile > ctx->ncu ? 2 : 1; q <= acehost::PAIR_MAXP; ++q) {
+            if (small && share_bytes(ctx, nenv, q + 1) > ACE_SHARE_BYTES) break;
+            const double c = (double)((ntile * q + ctx->ncu - 1) / ctx->ncu) * clocks(q);
+            if (c < best) {
+                best = c;
+                P = q;
+            }
+        }
+    }
+    nhi = 0;
+    if (ctx->tail > 0) {
+        // the caller's tail tiles, where the segment kernel would take them
+        const WaveCfg* wc = ctx->wcfg[ctx->cur_w];
+        const int64_t nt = (nenv + ctx->seg_et - 1) / ctx->seg_et;
+        if (ctx->parts == 0) P = segment_parts(ctx, nt, forces ? wc->ptr_all[wc->W] : wc->ptr_e[wc->W], wc->W);
+        if (P < 2 || P >= MAX_PARTS)
+            return set_err("ace_set_tail_parts: tail tiles need 2 or 3 parts per tile (ace_set_parts)");
+        nhi = std::min<int64_t>(ctx->tail, ntile);
+    } else if (ctx->tail < 0 && ctx->parts == 0 && P >= 2 && ntile * P > ctx->ncu) {
+        const auto key = std::make_pair(ntile, P + (forces ? 64 : 128));
+        auto it = ctx->tail_cache.find(key);
+        if (it == ctx->tail_cache.end()) {
+            if (ctx->tail_cache.size() >= 64) ctx->tail_cache.clear();
+            it = ctx->tail_cache.emplace(key, choose_tail(ntile, P, ctx->ncu, clocks(P), clocks(P + 1))).first;
+        }
+        nhi = it->second;
+    }
+    return 0;
 }
 
 extern "C" int ace_set_tail_parts(ace_ctx* ctx, int ntail) {
@@ -1339,7 +1461,7 @@ static void launch_dagr(int ET, dim3 grid, dim3 block, size_t lds, hipStream_t s
 // holds A+ [npool][estride], G [ngslots * NC][estride] (forces), MAX_PARTS
 // energy shares [estride] and, for the flat force kernel, nnbr map entries.
 static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* off, const double* xyz,
-                     int64_t nnbr, const int8_t* species, double* E_out, double* dE, const Workspace& ws) {
+                     int64_t nnbr, const int8_t* species, double* E_out, double* dE, Workspace ws) {
     const int64_t estride = ((nenv + 63) / 64) * 64;
     const bool forces = dE != nullptr;
     WaveCfg* wc = ctx->wcfg[ctx->cur_w];
@@ -1369,32 +1491,26 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
     if (ctx->rec_dispatch && ctx->rec_et == 0 && !ctx->force_interp)
         return set_err("ace_set_kernel mode 2: per-record dispatch needs records (correlation order <= 4, npool <= 320)");
     ctx->last_tail = 0;
-    if (use_records) {
+    if (use_pairs(ctx, nenv, forces)) {
+        int P = 0;
+        int64_t nhi = 0;
+        if (pair_shape(ctx, nenv, forces, P, nhi)) return -1;
+        if (launch_pairs(ctx, st, nenv, estride, forces, P, nhi, ws, P == 1 ? E_out : ws.Epart)) return -1;
+        if (P > 1)
+            hipLaunchKernelGGL(k_esum<false>, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, P,
+                               ((nenv + 31) / 32 - nhi) * 32, ws.Epart, estride, ctx->e0v.p, ctx->cls_u.p, E_out);
+        ws.gparts = P;
+        ws.genv_hi = ((nenv + 31) / 32 - nhi) * 32;
+        ctx->last_parts = P;
+        ctx->last_tail = nhi;
+        ctx->last_kernel = 0;
+    } else if (use_records) {
         const int ET = rec_et;
         const int NE = ctx->classed ? 6 : 1;
         const int64_t ntile = (nenv + ET - 1) / ET;
         const size_t lds = std::max((size_t)ctx->npool * ET * sizeof(double2), (size_t)wc->W * NE * ET * sizeof(double));
-        // Parts per tile: the grid runs in rounds of ncu workgroups, and the last
-        // round may be nearly empty; splitting each tile's tasks over P
-        // workgroups shortens the rounds.  Pick P in 1..4 minimising
-        // rounds(P) / P, with 2 % per extra part for re-staging the A+ tile.
-        // A split is only considered while every virtual wave keeps at least 3
-        // tasks (fewer leave the part workgroups unbalanced or idle).
-        int P = ctx->parts;
         const int ntask_mode = forces ? wc->ptr_all[wc->W] : wc->ptr_e[wc->W];
-        int pmax = 1;
-        while (pmax < MAX_PARTS && ntask_mode >= 3 * (pmax + 1) * wc->W) ++pmax;
-        if (P == 0) {
-            double best = 1e300;
-            for (int q = 1; q <= pmax; ++q) {
-                const double rounds = (double)((ntile * q + ctx->ncu - 1) / ctx->ncu);
-                const double cost = rounds / q * (1.0 + 0.02 * (q - 1));
-                if (cost < best - 1e-12) {
-                    best = cost;
-                    P = q;
-                }
-            }
-        }
+        const int P = ctx->parts > 0 ? ctx->parts : segment_parts(ctx, ntile, ntask_mode, wc->W);
         ctx->last_parts = P;
         ctx->last_kernel = ET == 64 ? 0 : 1;  // 1: narrower tiles
         // tail tiles with P + 1 parts (P >= 2, so every tile sums shares in k_esum)
@@ -1408,7 +1524,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
             auto it = ctx->tail_cache.find(key);
             if (it == ctx->tail_cache.end()) {
                 if (ctx->tail_cache.size() >= 64) ctx->tail_cache.clear();
-                it = ctx->tail_cache.emplace(key, choose_tail(ntile, P, ctx->ncu)).first;
+                it = ctx->tail_cache.emplace(key, choose_tail(ntile, P, ctx->ncu, 1.0 / P, 1.08 / (P + 1))).first;
             }
             nhi = it->second;
         }
@@ -1469,9 +1585,16 @@ static int run_path(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double
     const int64_t estride = ((nenv + 63) / 64) * 64;
     const bool forces = dE != nullptr;
     if (ctx->Aplus.ensure((size_t)ctx->npool * estride)) return -1;
-    if (forces && ctx->Gbuf.ensure((size_t)std::max(1, ctx->ngslots) * gslot_width(ctx) * estride)) return -1;
-    if ((ctx->seg_et > 0 || ctx->rec_et > 0) && ctx->Epart.ensure((size_t)MAX_PARTS * (ctx->classed ? 6 : 1) * estride))
-        return -1;
+    size_t gslots = (size_t)std::max(1, ctx->ngslots) * gslot_width(ctx), eslots = (size_t)MAX_PARTS * (ctx->classed ? 6 : 1);
+    if (use_pairs(ctx, nenv, forces)) {
+        int P = 0;
+        int64_t nhi = 0;
+        if (pair_shape(ctx, nenv, forces, P, nhi)) return -1;
+        gslots = std::max(gslots, (size_t)(P + (nhi > 0)) * ctx->npool);
+        eslots = std::max(eslots, (size_t)(P + (nhi > 0)));
+    }
+    if (forces && ctx->Gbuf.ensure(gslots * estride)) return -1;
+    if ((ctx->seg_et > 0 || ctx->rec_et > 0) && ctx->Epart.ensure(eslots * estride)) return -1;
     if (forces && ctx->flat_force && nnbr > 0 && ctx->nbr_env.ensure(nnbr)) return -1;
     return eval_path(ctx, (hipStream_t)stream, nenv, off, xyz, nnbr, species, E_out, dE, ctx_buffers(ctx));
 }
@@ -1488,24 +1611,26 @@ extern "C" int ace_energy_forces_noalloc(ace_ctx* ctx, int64_t nenv, const int32
     if (!ctx->scratch) return set_err("ace_energy_forces_noalloc: no scratch array on this device");
     HIP_TRY(hipSetDevice(ctx->device));
     // carve the fixed array: A+, G, the energy shares, the neighbour map
-    const int64_t estride = ((nenv + 63) / 64) * 64;
-    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t bA = up((size_t)ctx->npool * estride * sizeof(double2));
-    const size_t bG = up((size_t)std::max(1, ctx->ngslots) * gslot_width(ctx) * estride * sizeof(double2));
-    const size_t bE = ctx->seg_et > 0 || ctx->rec_et > 0
-                          ? up((size_t)MAX_PARTS * (ctx->classed ? 6 : 1) * estride * sizeof(double))
-                          : 0;
-    const size_t bN = ctx->flat_force ? up((size_t)nnbr * sizeof(int32_t)) : 0;
-    const size_t need = bA + bG + bE + bN;
-    if (need > ACE_SCRATCH_BYTES)
-        return set_err("ace_energy_forces_noalloc: the batch needs " + std::to_string(need) + " bytes of scratch, " +
+    const ScratchNeed need = scratch_need(ctx, nenv, nnbr);
+    if (need.all() > ACE_SCRATCH_BYTES)
+        return set_err("ace_energy_forces_noalloc: the batch needs " + std::to_string(need.all()) + " bytes of scratch, " +
                        "more than the fixed " + std::to_string(ACE_SCRATCH_BYTES) + "; split it into smaller batches");
     Workspace ws;
     ws.Aplus = reinterpret_cast<double2*>(ctx->scratch);
-    ws.Gbuf = reinterpret_cast<double2*>(ctx->scratch + bA);
-    ws.Epart = bE ? reinterpret_cast<double*>(ctx->scratch + bA + bG) : nullptr;
-    ws.nbr_env = bN ? reinterpret_cast<int32_t*>(ctx->scratch + bA + bG + bE) : nullptr;
-    ws.nbr_cap = bN ? (size_t)nnbr : 0;
+    ws.Gbuf = reinterpret_cast<double2*>(ctx->scratch + need.A);
+    ws.Epart = need.E ? reinterpret_cast<double*>(ctx->scratch + need.A + need.G) : nullptr;
+    ws.nbr_env = need.N ? reinterpret_cast<int32_t*>(ctx->scratch + need.A + need.G + need.E) : nullptr;
+    if (use_pairs(ctx, nenv, true)) {
+        int P = 0;
+        int64_t nhi = 0;
+        if (pair_shape(ctx, nenv, true, P, nhi)) return -1;
+        const int n = P + (nhi > 0);
+        if (share_bytes(ctx, nenv, n) > ACE_SHARE_BYTES) return set_err("ace_energy_forces_noalloc: shares too large");
+        const size_t g = scratch_up((size_t)n * ctx->npool * (((nenv + 63) / 64) * 64) * sizeof(double2));
+        ws.Gbuf = reinterpret_cast<double2*>(ctx->scratch + ACE_SCRATCH_BYTES);
+        ws.Epart = reinterpret_cast<double*>(ctx->scratch + ACE_SCRATCH_BYTES + g);
+    }
+    ws.nbr_cap = need.N ? (size_t)nnbr : 0;
     return eval_path(ctx, (hipStream_t)stream, nenv, off, xyz, nnbr, species, E_out, dE_dr, ws);
 }
 

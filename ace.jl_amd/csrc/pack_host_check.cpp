@@ -1,11 +1,15 @@
 // CPU test shim over pack_host.hpp and compile_host.hpp: the host-side pack
 // logic and the program compiler of libacehip.so built without HIP (tests
 // build it with the address sanitizer, and plain for the larger bases).
+#include <complex>
 #include <cstring>
+#include <map>
+#include <set>
 
 #include "compile_host.hpp"
 #include "nbrlist_host.hpp"
 #include "pack_host.hpp"
+#include "pairs_host.hpp"
 
 extern "C" int acehost_validate(const ace_pack* pk, char* msg, int len) {
     std::string e = acehost::validate_pack(pk);
@@ -36,6 +40,72 @@ extern "C" int acehost_lookup(const ace_pack* pk, short* kidx, int* a4) {
     std::memcpy(kidx, kx.data(), kx.size() * sizeof(int16_t));
     std::vector<int32_t> a = acehost::aspec_rows(pk);
     std::memcpy(a4, a.data(), a.size() * sizeof(int32_t));
+    return 0;
+}
+
+// A pair program run on the CPU as k_pairs runs it, on pooled values A[npool]
+// (re, im) and parameters c: the energy, and with forces G[npool].  Returns 0,
+// 1 when the basis has no pair form, -1 on a rejected table or two panels of
+// one turn with a common target.
+extern "C" int acehost_pairs(const ace_pack* pk, const double* c, int forces, int parts, const double* A, double* E,
+                             double* G) {
+    if (!acehost::validate_pack(pk).empty()) return -1;
+    const acehost::PackCopy pc = acehost::copy_pack(pk);
+    const int np = pk->npool, rb = forces ? 1024 : 512;
+    acehost::PairForm pf;
+    acehost::PairProgram pp;
+    if (!acehost::pair_form(pc, std::vector<int32_t>(pk->pool, pk->pool + 4 * (size_t)np), pf).empty()) return 1;
+    if (!acehost::pair_program(pf, forces != 0, rb, np, 96, pp).empty()) return -1;
+    const acehost::Coeffs cf = acehost::coefficients(pc, c);
+    acehost::pair_coefs(pp, cf.leaf);
+    typedef std::complex<double> C;
+    auto val = [&](uint32_t w) {
+        const int k = (int)(w & ~1u) / rb;
+        const C a = k == np ? C(1.0) : C(A[2 * k], A[2 * k + 1]);
+        return w & 1u ? std::conj(a) : a;
+    };
+    std::vector<C> g((size_t)np + 1, 0.0);
+    double e = 0.0;
+    for (int part = 0; part < parts; ++part) {
+        const int32_t* sq = pp.seq[parts].data() + pp.seq_ptr[parts][(size_t)part];
+        const int nround = *sq++;
+        for (int r = 0; r < nround; ++r, sq += acehost::PAIR_SEQ) {
+            std::map<int, std::set<int>> hit;
+            for (int w = 0; w < acehost::PAIR_WAVES; ++w) {
+                if (sq[1 + w] < 0) continue;
+                const uint32_t* hd = pp.words.data() + sq[1 + w];
+                const double* co = pp.coef.data() + hd[2];
+                const uint32_t* q = hd + acehost::PAIR_HDR;
+                C h[acehost::PAIR_ROWS] = {};
+                const int n[3] = {(int)(hd[0] & 1023u), (int)(hd[0] >> 10 & 1023u), (int)(hd[0] >> 20)};
+                for (int kind = 0; kind < 3; ++kind)
+                    for (int i = 0, nq = 4 >> kind; i < n[kind]; ++i, q += acehost::pair_rec_words(nq))
+                        for (int j = 0; j < nq; ++j)
+                            for (C& hr : h) hr += *co++ * val(q[0]) * val(q[1 + j]);
+                std::set<int> mine;
+                for (int s = 0; s < acehost::PAIR_ROWS; ++s) {
+                    const uint32_t wa = hd[4 + 2 * s], wd = hd[5 + 2 * s];
+                    const int ka = (int)wa / rb, kd = (int)(wd & ~1u) / rb;
+                    const C gp = std::conj(h[s]), t2 = gp * val(wa);
+                    e += (gp * val(wa) * val(wd)).real();
+                    g[(size_t)ka] += gp * val(wd);
+                    g[(size_t)kd] += wd & 1u ? std::conj(t2) : t2;
+                    if (ka < np) mine.insert(ka);
+                    if (kd < np) mine.insert(kd);
+                }
+                if (!forces) continue;
+                const int turn = (int)(hd[1] >> 8);
+                if (turn >= sq[0]) return -1;
+                for (int k : mine)
+                    if (!hit[turn].insert(k).second) return -1;
+            }
+        }
+    }
+    *E = cf.e0[0] + (forces ? 0.5 : 1.0) * e;
+    for (int k = 0; forces && k < np; ++k) {
+        G[2 * k] = g[(size_t)k].real();
+        G[2 * k + 1] = g[(size_t)k].imag();
+    }
     return 0;
 }
 

@@ -81,6 +81,8 @@ def executed_flops(pack, forces=True, kernel=0):
     4 per leaf, 6 per new prefix product, 8 per run."""
     import numpy as np
     cplx = bool(getattr(pack, "classed", 0))
+    if pair_kernel(pack, kernel):
+        return None
     if kernel not in (0, 1):
         w = pack.work_counts(forces)
         per_leaf = 8.0 if cplx else 4.0
@@ -90,6 +92,13 @@ def executed_flops(pack, forces=True, kernel=0):
     per_leaf = 8.0 if cplx else 4.0
     rec = per_leaf * nl - per_leaf / 2 + 6.0 * np.maximum(d - 1, 0) + np.where(d > 0, 8.0, 2.0)
     return float(lanes * np.sum(rec))
+
+
+def pair_kernel(pack, kernel):
+    """Whether the pair kernel took the benchmark's calls (Invariant,
+    correlation order 4, at most 159 pooled values): its programs are the
+    library's own, so their operations are not counted here."""
+    return kernel == 0 and pack.prop == 0 and pack.maxorder == 4 and len(pack.pool) <= 159
 
 
 def _segment_records(pack, forces):
@@ -116,15 +125,17 @@ def lds_read_bytes(pack, forces=True, kernel=0):
     tiles (ET < 64) each environment costs 64 / ET lanes.  None for the other
     kernels."""
     import numpy as np
-    if kernel not in (0, 1):
+    if kernel not in (0, 1) or pair_kernel(pack, kernel):
         return None
     d, nl, et = _segment_records(pack, forces)
     lanes = 64.0 / et if kernel == 1 else 1.0
     return float(16.0 * lanes * np.sum(d + nl))
 
 
-def dag_kernel_name(code):
+def dag_kernel_name(pack, code):
     """The product-DAG kernel of ace_last_dag_shape's code."""
+    if pair_kernel(pack, code):
+        return "k_pairs (quadratic form in products of two pooled values, 32-environment tiles)"
     if code == 0:
         return "k_dags (kind-sorted record segments, 64-environment tiles)"
     if code == 1:
@@ -386,7 +397,7 @@ def main():
     lds_env = lds_read_bytes(pk, True, dag_kernel)
     dag_avg = float(np.mean(dag_ms))
     achieved = f_alg * b.nenv / (dag_avg * 1e-3) / 1e12
-    achieved_exe = f_exe * b.nenv / (dag_avg * 1e-3) / 1e12
+    achieved_exe = None if f_exe is None else f_exe * b.nenv / (dag_avg * 1e-3) / 1e12
     out = {
         "metric": METRIC,
         "value": round(value, 1),
@@ -420,11 +431,11 @@ def main():
                      "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
                      "traffic": DAG_TRAFFIC_BYTES.get(b.nenv) if headline else None,
                      "traffic_source": TRAFFIC_SOURCE if headline and b.nenv in DAG_TRAFFIC_BYTES else None,
-                     "kernel": dag_kernel_name(dag_kernel),
+                     "kernel": dag_kernel_name(pk, dag_kernel),
                      "kernel_ms": round(dag_avg, 4), "dag_parts": dag_parts, "dag_tail_tiles": dag_tail,
                      "flops_per_env_algorithmic": f_alg, "flops_per_env_executed": f_exe,
-                     "executed_tflops": round(achieved_exe, 3),
-                     "executed_frac": round(achieved_exe / FP64_PEAK_TFLOPS, 4),
+                     "executed_tflops": None if f_exe is None else round(achieved_exe, 3),
+                     "executed_frac": None if f_exe is None else round(achieved_exe / FP64_PEAK_TFLOPS, 4),
                      # the segment kernel's binding resource: 16-byte LDS reads
                      "lds_read_bytes_per_env": lds_env,
                      "lds_read_TBps": None if lds_env is None else round(lds_env * b.nenv / (dag_avg * 1e-3) / 1e12, 2),

@@ -232,13 +232,16 @@ int ace_set_tail_parts(ace_ctx* ctx, int ntail);
 
 /* The product-DAG launch of the last evaluation call: workgroups per tile,
  * the number of tail tiles that ran one more part, and the kernel (0: the
- * record kernel on 64-environment tiles, 1: on 32-environment tiles; 64, 32
+ * pair kernel on 32-environment tiles or the segment kernel on
+ * 64-environment tiles, 1: the segment kernel on narrower tiles; 64, 32
  * or 16: the run interpreter with that many environments per tile).
  * Instrumentation; no counterpart in the reference. */
 int ace_last_dag_shape(ace_ctx* ctx, int* parts, int64_t* tail_tiles, int* kernel);
 
-/* Product-DAG kernel choice: 0 (default) the record-segment kernel where the
- * basis allows it (Invariant or class-split EuclideanVector programs,
+/* Product-DAG kernel choice: 0 (default) the pair kernel for Invariant bases of
+ * correlation order 4 with at most 159 pooled values (order 3: energies, and
+ * batches of one tile per compute unit), else the
+ * record-segment kernel where the basis allows it (Invariant or class-split EuclideanVector programs,
  * correlation order <= 4, at most 320 pooled values), else the run
  * interpreter; 1 the run interpreter always; 2 the per-record dispatch kernel
  * over the same records where they exist.  A tuning and testing knob of this
