@@ -185,69 +185,52 @@ __global__ void k_AAdir(int64_t nenv, int nA, int nAA, int maxord, const int32_t
 
 // Factor f of the staged tile, conjugated when f carries ACE_CONJ (the sign
 // bit of the imaginary part flipped without a branch).
+__device__ __forceinline__ double2 conj_if(double2 v, uint32_t sign) {
+    return make_double2(v.x, __hiloint2double(__double2hiint(v.y) ^ (int)sign, __double2loint(v.y)));
+}
+
 template <int ENVS>
 __device__ __forceinline__ double2 bt_factor(const double2* As, int f, int e) {
-    const double2 v = As[(f & 0x7fff) * ENVS + e];
-    return make_double2(v.x, __hiloint2double(__double2hiint(v.y) ^ ((f & ACE_CONJ) << 16), __double2loint(v.y)));
+    return conj_if(As[(f & 0x7fff) * ENVS + e], (uint32_t)(f & ACE_CONJ) << 16);
 }
 
 // The records [za, zb) of one row whose AA columns have order O: each
-// recomputes its product (or dual-number derivative, DIR) left to right
-// from the staged tiles, straight-line code, four records per iteration so
-// that their scalar loads and LDS reads overlap (two for the dual numbers of
-// DIR: registers).
-template <int O, int PROP, bool DIR, int ENVS>
+// recomputes its product left to right from the staged tile, straight-line
+// code, four records per iteration so that their scalar loads and LDS reads
+// overlap.
+template <int O, int ENVS>
 __device__ __forceinline__ void bt_order(int za, int zb, const BtRec* __restrict__ recs,
-                                         const double* __restrict__ vals, const double2* As, const double2* Ws,
-                                         int e, double* s) {
-#pragma unroll(DIR ? 2 : 4)
+                                         const double* __restrict__ vals, const double2* As, int e, double* s) {
+#pragma unroll(4)
     for (int z = za; z < zb; ++z) {
         const BtRec r = recs[z];
-        double2 p = make_double2(1.0, 0.0), dp = make_double2(0.0, 0.0);
+        double2 p = make_double2(1.0, 0.0);
 #pragma unroll
-        for (int q = 0; q < O; ++q) {
-            const double2 a = bt_factor<ENVS>(As, r.f[q], e);
-            if (DIR) {
-                const double2 da = bt_factor<ENVS>(Ws, r.f[q], e);
-                const double2 x = cmul(dp, a), y = cmul(p, da);
-                dp = make_double2(x.x + y.x, x.y + y.y);
-            }
-            p = cmul(p, a);
-        }
-        const double2 v = DIR ? dp : p;
-        if (PROP == 0) {
-            s[0] += r.coef * v.x;
-        } else {
-            const double sg = r.coef;
+        for (int q = 0; q < O; ++q) p = cmul(p, bt_factor<ENVS>(As, r.f[q], e));
+        const double sg = r.sgn;
 #pragma unroll
-            for (int q = 0; q < 3; ++q) s[q] += sg * (vals[6 * r.z + 2 * q] * v.x - vals[6 * r.z + 2 * q + 1] * v.y);
-        }
+        for (int q = 0; q < 3; ++q) s[q] += sg * (vals[6 * r.z + 2 * q] * p.x - vals[6 * r.z + 2 * q + 1] * p.y);
     }
 }
 
-// k_Bt: basis values B = A2B . AA (DIR = false; pibasis.jl:265-275,
-// symmbasis.jl:248-264) or their directional derivative A2B . dAA along
-// per-neighbour weights (DIR = true; evaluator.jl:225-240) for a tile of
-// ENVS environments, without materialising AA.  The pooled A+ tile (and
-// dA+w for DIR) is staged in LDS as in k_dagr; every A2B nonzero (one BtRec,
-// read with scalar loads) recomputes its AA product from it.  A row's
-// nonzeros are ordered by the order of their AA column (rowo: where each
+// k_Bt: EuclideanVector basis values B = A2B . AA (pibasis.jl:265-275,
+// symmbasis.jl:248-264) for a tile of ENVS environments, without
+// materialising AA.  The pooled A+ tile is staged in LDS; every A2B nonzero
+// (one BtRec, read with scalar loads) recomputes its AA product from it.  A
+// row's nonzeros are ordered by the order of their AA column (rowo: where each
 // order starts), one straight-line loop per order.  A workgroup is (tile,
 // chunk of rows); each wave takes rpw consecutive rows (with ENVS = 32 the two
 // half-waves take alternate rows).  Workgroups of one tile are consecutive on
 // one XCD so the staged tile is read from that XCD's L2.
 constexpr int BT_NW = 16;  // waves per k_Bt workgroup
 
-template <int PROP, bool DIR, int ENVS>
+template <int ENVS>
 __global__ __launch_bounds__(64 * BT_NW) void k_Bt(int64_t nenv, int npool, int nB, int nchunk, int rpw,
                                             const int32_t* __restrict__ rowo, const BtRec* __restrict__ recs,
                                             const double* __restrict__ vals, const double2* __restrict__ Aplus,
-                                            const double2* __restrict__ Wplus, int64_t estride,
-                                            double* __restrict__ out) {
-    constexpr int NC = PROP == 0 ? 1 : 3;
+                                            int64_t estride, double* __restrict__ out) {
     extern __shared__ double2 tilebuf[];
     double2* As = tilebuf;
-    double2* Ws = tilebuf + (size_t)npool * ENVS;
     const int64_t ntile = (nenv + ENVS - 1) / ENVS;
     const int64_t lin = xcd_env(blockIdx.x, ntile * nchunk);
     const int64_t t = lin / nchunk;
@@ -256,13 +239,9 @@ __global__ __launch_bounds__(64 * BT_NW) void k_Bt(int64_t nenv, int npool, int 
     for (int i = threadIdx.x; i < npool * ENVS; i += 64 * BT_NW) {
         const int k = i / ENVS;
         const int64_t env = e0 + (i % ENVS);
-        double2 v = make_double2(0.0, 0.0), w = make_double2(0.0, 0.0);
-        if (env < nenv) {
-            v = Aplus[(int64_t)k * estride + env];
-            if (DIR) w = Wplus[(int64_t)k * estride + env];
-        }
+        double2 v = make_double2(0.0, 0.0);
+        if (env < nenv) v = Aplus[(int64_t)k * estride + env];
         As[i] = v;
-        if (DIR) Ws[i] = w;
     }
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -273,20 +252,168 @@ __global__ __launch_bounds__(64 * BT_NW) void k_Bt(int64_t nenv, int npool, int 
     const int b0 = (chunk * BT_NW + wave) * rpw;
     const int b1 = min(b0 + rpw, nB);
     for (int b = b0 + half; b < b1; b += (ENVS == 32 ? 2 : 1)) {
-        double s[NC];
-#pragma unroll
-        for (int q = 0; q < NC; ++q) s[q] = 0.0;
+        double s[3] = {0.0, 0.0, 0.0};
         const int32_t* ro = rowo + (int64_t)b * BT_ROWO;
-        bt_order<0, PROP, DIR, ENVS>(ro[0], ro[1], recs, vals, As, Ws, e, s);
-        bt_order<1, PROP, DIR, ENVS>(ro[1], ro[2], recs, vals, As, Ws, e, s);
-        bt_order<2, PROP, DIR, ENVS>(ro[2], ro[3], recs, vals, As, Ws, e, s);
-        bt_order<3, PROP, DIR, ENVS>(ro[3], ro[4], recs, vals, As, Ws, e, s);
-        bt_order<4, PROP, DIR, ENVS>(ro[4], ro[5], recs, vals, As, Ws, e, s);
+        bt_order<0, ENVS>(ro[0], ro[1], recs, vals, As, e, s);
+        bt_order<1, ENVS>(ro[1], ro[2], recs, vals, As, e, s);
+        bt_order<2, ENVS>(ro[2], ro[3], recs, vals, As, e, s);
+        bt_order<3, ENVS>(ro[3], ro[4], recs, vals, As, e, s);
+        bt_order<4, ENVS>(ro[4], ro[5], recs, vals, As, e, s);
         if (env < nenv) {
 #pragma unroll
-            for (int q = 0; q < NC; ++q) out[(env * nB + b) * NC + q] = s[q];
+            for (int q = 0; q < 3; ++q) out[(env * nB + b) * 3 + q] = s[q];
         }
     }
+}
+
+// n pairs of records of order O from r on (lanes 0-31 the first of a pair,
+// lanes 32-63 the second).  `next` is the record read ahead: the stream runs on
+// over the segments of a wave, so a record is in flight while one is used.
+template <int O, bool DIR>
+__device__ __forceinline__ void bv_run(int n, const uint4*& r, uint4& next, const char* tile, uint32_t e16, double& s) {
+    constexpr int SH = DIR ? 10 : 9;  // a pooled value's row: 32 x A+, and 32 x dA+w
+    for (int i = 0; i < n; ++i) {
+        const uint4 q = next;
+        r += 2;
+        next = *r;
+        const double c = __hiloint2double((int)q.w, (int)q.z);
+        if (O == 0) {
+            if (!DIR) s += c;
+            continue;
+        }
+        double2 a[4], d[4];
+#pragma unroll
+        for (int t = 0; t < O; ++t) {
+            const uint32_t w = t < 2 ? q.x : q.y;
+            const char* at = tile + ((((t & 1 ? w >> 16 : w) & 0x1ffu) << SH) | e16);
+            const uint32_t sign = (t & 1 ? w : w << 16) & 0x80000000u;
+            a[t] = *reinterpret_cast<const double2*>(at);
+            if (DIR) d[t] = *reinterpret_cast<const double2*>(at + 512);
+            if (t > 0) {
+                a[t] = conj_if(a[t], sign);
+                if (DIR) d[t] = conj_if(d[t], sign);
+            }
+        }
+        // products and their derivatives of the first two and the other factors
+        double2 p = a[0], dp = d[0], u, du;
+        if (O == 2) {
+            u = a[1];
+            if (DIR) du = d[1];
+        } else if (O >= 3) {
+            if (DIR) {
+                const double2 x = cmul(d[0], a[1]), y = cmul(a[0], d[1]);
+                dp = make_double2(x.x + y.x, x.y + y.y);
+            }
+            p = cmul(a[0], a[1]);
+            u = a[2];
+            if (DIR) du = d[2];
+            if (O == 4) {
+                if (DIR) {
+                    const double2 x = cmul(d[2], a[3]), y = cmul(a[2], d[3]);
+                    du = make_double2(x.x + y.x, x.y + y.y);
+                }
+                u = cmul(a[2], a[3]);
+            }
+        }
+        if (O == 1)
+            s += c * (DIR ? dp.x : p.x);
+        else if (DIR)
+            s += c * ((dp.x * u.x - dp.y * u.y) + (p.x * du.x - p.y * du.y));
+        else
+            s += c * (p.x * u.x - p.y * u.y);
+    }
+}
+
+// k_Bv: Invariant basis values B = A2B . AA (DIR = false; pibasis.jl:265-275,
+// symmbasis.jl:248-264) or their directional derivative A2B . dAA along
+// per-neighbour weights (DIR = true; evaluator.jl:225-240), records and their
+// order as basis_host.hpp lays them out.  Tiles of 32 environments staged in
+// LDS (A+, with DIR dA+w beside it); lane = environment, the half-waves take
+// alternate records.  Bound by the LDS reads (16 B per factor and environment,
+// twice that with DIR), with the vector unit close behind, provided that the
+// records arrive in time: they are vector loads, one record ahead.  Scalar
+// loads, each waited for before its product's LDS reads, left a wave 0.75 us
+// per record.  Rows are shared out by cost over the waves of nchunk
+// workgroups per tile (bv_chunks), so that a batch of a few tiles still fills the chip.
+// Measured with 3,235 functions of 139 pooled values, pooling included: 2,003
+// environments 438 -> 112 us for values and 903 -> 210 us for derivatives, 108
+// environments 317 -> 45 us, 20,000 environments 2.77 -> 0.88 ms and 6.17 ->
+// 1.61 ms (one scalar-loaded record per A2B nonzero, 12 workgroups per tile of
+// 64); with 97 functions of order 3, where pooling dominates, 20,000
+// environments 66 -> 63 and 185 -> 151 us.
+// Two rows are finished at a time: one swap of half-waves and one add sum
+// both, and lanes 0-31 store the first, lanes 32-63 the second.
+template <bool DIR>
+__global__ __launch_bounds__(64 * acehost::BV_WAVES) void k_Bv(int64_t nenv, int npool, int nB, int nchunk,
+                                                               const int2* __restrict__ seg,
+                                                               const int2* __restrict__ unit,
+                                                               const uint4* __restrict__ recs,
+                                                               const double2* __restrict__ Aplus,
+                                                               const double2* __restrict__ Wplus, int64_t estride,
+                                                               double* __restrict__ out) {
+    extern __shared__ double2 tilebuf[];
+    const int64_t ntile = (nenv + 31) / 32;
+    const int64_t lin = xcd_env(blockIdx.x, ntile * nchunk);
+    const int64_t e0 = lin / nchunk * 32;
+    const int chunk = (int)(lin % nchunk);
+    for (int i = threadIdx.x; i < npool * 32; i += 64 * acehost::BV_WAVES) {
+        const int k = i / 32;
+        const int64_t env = e0 + i % 32;
+        double2 v = make_double2(0.0, 0.0), w = make_double2(0.0, 0.0);
+        if (env < nenv) {
+            v = Aplus[(int64_t)k * estride + env];
+            if (DIR) w = Wplus[(int64_t)k * estride + env];
+        }
+        double2* to = tilebuf + (DIR ? k * 64 : k * 32) + i % 32;
+        to[0] = v;
+        if (DIR) to[32] = w;
+    }
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, half = lane >> 5;
+    const int64_t env = e0 + (lane & 31);
+    const char* tile = reinterpret_cast<const char*>(tilebuf);
+    const uint32_t e16 = (uint32_t)(lane & 31) * 16;
+    constexpr int UW = acehost::BV_UNITS / acehost::BV_WAVES;  // shares of a wave if one workgroup does a tile
+    const int u = (chunk * acehost::BV_WAVES + wave) * (UW / nchunk);
+    const int2 from = unit[u];
+    const int s1 = unit[u + UW / nchunk].x;
+    const uint4* r = recs + 2 * (int64_t)from.y + half;
+    uint4 next = *r;
+    int2 head = make_int2(0, 0);
+    double s = 0.0, first = 0.0;
+    int bfirst = -1;
+    auto finish = [&](double x, double y, int bx, int by, bool both) {
+        const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false, false);
+        const double v = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+        if (env < nenv && (both || half == 0)) out[env * nB + (half ? by : bx)] = v;
+    };
+    for (int g = from.x; g < s1; ++g) {
+        const int i = (g - from.x) & 63;
+        if (i == 0) head = seg[min(g + lane, s1 - 1)];
+        const int row = __builtin_amdgcn_readlane(head.x, i), nw = __builtin_amdgcn_readlane(head.y, i);
+        const int n = nw & 0xfffffff;
+        switch (nw >> 28) {
+            case 4: bv_run<4, DIR>(n, r, next, tile, e16, s); break;
+            case 3: bv_run<3, DIR>(n, r, next, tile, e16, s); break;
+            case 2: bv_run<2, DIR>(n, r, next, tile, e16, s); break;
+            case 1: bv_run<1, DIR>(n, r, next, tile, e16, s); break;
+            default: bv_run<0, DIR>(n, r, next, tile, e16, s);
+        }
+        if (row < 0) {
+            const int b = row & 0x7fffffff;
+            if (bfirst < 0) {
+                first = s;
+                bfirst = b;
+            } else {
+                finish(first, s, bfirst, b, true);
+                bfirst = -1;
+            }
+            s = 0.0;
+        }
+    }
+    if (bfirst >= 0) finish(first, 0.0, bfirst, bfirst, false);
 }
 
 // dAA[j][iAA][3] = sum_a (prod_{t != a} A_t) dphi[j][v_a]  (pibasis.jl:402-432)
@@ -576,46 +703,52 @@ extern "C" int ace_basis_AA(ace_ctx* ctx, int64_t nenv, const int32_t* off, cons
     return 0;
 }
 
-// Fused basis values (k_Bt): the tile it runs on (environments; 0 when the
-// pooled tile does not fit LDS), and the launch.  Basis values take 64
-// environments when their A+ tile fits, else 32 (npool <= 320); the
-// directional derivative stages A+ and dA+w, 32 environments.
-static int bt_envs(const ace_ctx* ctx, bool dir) {
-    if (ctx->maxorder > 4) return 0;  // BtRec holds four factors
-    const size_t row = (size_t)ctx->npool * sizeof(double2) * (dir ? 2 : 1);
-    if (!dir && row * 64 <= 160 * 1024) return 64;
-    return row * 32 <= 160 * 1024 ? 32 : 0;
+// Whether the fused kernels (k_Bv, k_Bt) take this basis: four factors per
+// record, and the staged tile of 32 environments fits LDS (A+ alone up to 320
+// pooled values, A+ and dA+w up to 160).
+static bool bt_fits(const ace_ctx* ctx, bool dir) {
+    return ctx->maxorder <= 4 && (size_t)ctx->npool * 32 * sizeof(double2) * (dir ? 2 : 1) <= 160 * 1024;
 }
 
-template <int PROP, bool DIR, int ENVS>
+template <int ENVS>
 static int launch_bt_shape(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, double* out) {
-    const size_t lds = (size_t)ctx->npool * ENVS * sizeof(double2) * (DIR ? 2 : 1);
+    const size_t lds = (size_t)ctx->npool * ENVS * sizeof(double2);
     constexpr int NW = BT_NW;
     const int rpw = std::max(1, (ctx->nB + NW * 12 - 1) / (NW * 12));
     const int nchunk = (ctx->nB + NW * rpw - 1) / (NW * rpw);
     const int64_t nblk = (nenv + ENVS - 1) / ENVS * nchunk;
     if (nblk >= ((int64_t)1 << 31)) return set_err("batch too large for one launch");
-    set_func_lds((const void*)k_Bt<PROP, DIR, ENVS>, lds);
-    hipLaunchKernelGGL((k_Bt<PROP, DIR, ENVS>), dim3((unsigned)nblk), dim3(64 * NW), lds, st, nenv, ctx->npool,
-                       ctx->nB, nchunk, rpw, ctx->bt_rowo.p, ctx->bt_rec.p, ctx->vals.p, ctx->Aplus.p, ctx->Wplus.p,
-                       estride, out);
+    set_func_lds((const void*)k_Bt<ENVS>, lds);
+    hipLaunchKernelGGL(k_Bt<ENVS>, dim3((unsigned)nblk), dim3(64 * NW), lds, st, nenv, ctx->npool, ctx->nB, nchunk,
+                       rpw, ctx->bt_rowo.p, ctx->bt_rec.p, ctx->vals.p, ctx->Aplus.p, estride, out);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+template <bool DIR>
+static int launch_bv(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, double* out) {
+    if (ctx->nB == 0) return 0;
+    const int64_t tiles = (nenv + 31) / 32;
+    const size_t lds = (size_t)ctx->npool * 32 * sizeof(double2) * (DIR ? 2 : 1);
+    const int resident = 2 * lds <= 160 * 1024 ? 2 : 1;  // 16 waves each
+    const int nchunk = acehost::bv_chunks(ctx->bv_iter, ctx->bv_cost * (DIR ? 1.8 : 1.0), tiles, ctx->ncu, resident, (double)lds);
+    if (tiles * nchunk >= ((int64_t)1 << 31)) return set_err("batch too large for one launch");
+    set_func_lds((const void*)k_Bv<DIR>, lds);
+    hipLaunchKernelGGL(k_Bv<DIR>, dim3((unsigned)(tiles * nchunk)), dim3(64 * acehost::BV_WAVES), lds, st, nenv,
+                       ctx->npool, ctx->nB, nchunk, reinterpret_cast<const int2*>(ctx->bv_seg.p),
+                       reinterpret_cast<const int2*>(ctx->bv_unit.p), reinterpret_cast<const uint4*>(ctx->bv_rec.p),
+                       ctx->Aplus.p, DIR ? ctx->Wplus.p : nullptr, estride, out);
     HIP_TRY(hipGetLastError());
     return 0;
 }
 
 template <bool DIR>
 static int launch_bt(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, double* out) {
-    const int envs = bt_envs(ctx, DIR);
-    if (envs == 0) return set_err("pooled tile does not fit LDS");
-    if (DIR) {
-        if (ctx->prop != ACE_PROP_INVARIANT) return set_err("directional basis derivative: Invariant bases only");
-        return launch_bt_shape<0, true, 32>(ctx, st, nenv, estride, out);
-    }
-    if (ctx->prop == ACE_PROP_INVARIANT)
-        return envs == 64 ? launch_bt_shape<0, false, 64>(ctx, st, nenv, estride, out)
-                          : launch_bt_shape<0, false, 32>(ctx, st, nenv, estride, out);
-    return envs == 64 ? launch_bt_shape<1, false, 64>(ctx, st, nenv, estride, out)
-                      : launch_bt_shape<1, false, 32>(ctx, st, nenv, estride, out);
+    if (!bt_fits(ctx, DIR)) return set_err("pooled tile does not fit LDS");
+    if (ctx->prop == ACE_PROP_INVARIANT) return launch_bv<DIR>(ctx, st, nenv, estride, out);
+    if (DIR) return set_err("directional basis derivative: Invariant bases only");
+    return (size_t)ctx->npool * 64 * sizeof(double2) <= 160 * 1024 ? launch_bt_shape<64>(ctx, st, nenv, estride, out)
+                                                                   : launch_bt_shape<32>(ctx, st, nenv, estride, out);
 }
 
 extern "C" int ace_basis_B(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* xyz,
@@ -627,7 +760,7 @@ extern "C" int ace_basis_B(ace_ctx* ctx, int64_t nenv, const int32_t* off, const
     hipStream_t st = (hipStream_t)stream;
     {
         const int64_t estride = ((nenv + 63) / 64) * 64;
-        if (bt_envs(ctx, false) > 0) {
+        if (bt_fits(ctx, false)) {
             if (ctx->Aplus.ensure((size_t)ctx->npool * estride)) return -1;
             if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false)) return -1;
             return launch_bt<false>(ctx, st, nenv, estride, B_out);
@@ -765,7 +898,7 @@ extern "C" int ace_adjoint_EVAL_D(ace_ctx* ctx, int64_t nenv, const int32_t* off
     if (!dB_out || (nnbr > 0 && !w)) return set_err("ace_adjoint_EVAL_D: null argument");
     hipStream_t st = (hipStream_t)stream;
     const int64_t estride = ((nenv + 63) / 64) * 64;
-    if (bt_envs(ctx, true) > 0) {
+    if (bt_fits(ctx, true)) {
         if (ctx->Aplus.ensure((size_t)ctx->npool * estride) || ctx->Wplus.ensure((size_t)ctx->npool * estride))
             return -1;
         if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false) ||

@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "../../include/acehip.h"
+#include "basis_host.hpp"
 #include "host_util.hpp"
 #include "pack_host.hpp"
 #include "pairs_host.hpp"
@@ -209,15 +210,14 @@ __device__ __forceinline__ double flip_sign_if(double c, uint32_t f) {
     return __hiloint2double(__double2hiint(c) ^ (int)((f & 0x8000u) << 16), __double2loint(c));
 }
 
-// One A2B nonzero of the fused basis-value kernel, pre-decoded on the host:
-// the AA column's order and pooled factor ids (k | ACE_CONJ), and the A2B
-// value times the sign of the m < 0 factors (Invariant; EuclideanVector
-// rows read their 3 complex values from the CSR array).
+// One A2B nonzero of the EuclideanVector basis-value kernel, pre-decoded on
+// the host: the AA column's order, pooled factor ids (k | ACE_CONJ) and the
+// sign of the m < 0 factors (the three complex values stay in the CSR array).
 struct BtRec {
     int32_t o;
     int32_t f[4];
     int32_t z;  // CSR index of the nonzero
-    double coef;
+    double sgn;
 };
 static_assert(sizeof(BtRec) == 32, "BtRec is 8 dwords");
 // per basis row of the fused kernel: where its records of order 0, 1, ..., 4
@@ -313,6 +313,10 @@ struct ace_ctx {
     DevBuf<double> aspec_sgn, vals;
     DevBuf<BtRec> bt_rec;
     DevBuf<int32_t> bt_rowo;  // [nB][BT_ROWO] record ranges per order
+    // Invariant basis values (k_Bv): acehost::BvProgram
+    DevBuf<acehost::BvRec> bv_rec;
+    DevBuf<int32_t> bv_seg, bv_unit;
+    double bv_iter = 0, bv_cost = 0;
     DevBuf<int32_t> ffq;  // G slots of the flat force kernel's staged (l, m, n) entries
     DevBuf<int32_t> ffk;  // their pooled functions (the pair kernel's G rows)
     DevBuf<int16_t> kidx;

@@ -951,44 +951,52 @@ extern "C" int ace_ctx_create(const ace_pack* pk, int device, const double* c, i
             return fail("upload");
     }
     {
-        // one record per A2B nonzero for the fused basis-value kernel: the AA
-        // column's pooled factor ids and order, and (Invariant) the A2B value
-        // times the product of the m < 0 factor signs (EuclideanVector: the sign)
-        std::vector<BtRec> rec(std::max(1, pk->a2b_nnz));
-        for (int z = 0; z < pk->a2b_nnz; ++z) {
-            const int col = pk->a2b_cols[z];
-            BtRec& r = rec[z];
-            r.o = pk->orders[col];
-            r.z = z;
-            double sg = 1.0;
-            for (int q = 0; q < 4; ++q) {
-                r.f[q] = 0;
-                if (q < r.o) {
-                    const int iA = pk->iAA2iA[(size_t)col * pk->maxorder + q];
-                    r.f[q] = pk->aspec_fid[iA];
-                    sg *= pk->aspec_sgn[iA];
+        // basis values without AA (k_Bv, k_Bt); larger orders do not use them
+        if (acehost::bv_usable(pk)) {
+            const acehost::BvProgram bv = acehost::bv_program(pk);
+            if (ctx->bv_rec.upload(bv.rec.data(), bv.rec.size()) ||
+                ctx->bv_seg.upload(bv.seg.data(), bv.seg.size()) ||
+                ctx->bv_unit.upload(bv.unit.data(), bv.unit.size()))
+                return fail("upload");
+            ctx->bv_iter = bv.iter;
+            ctx->bv_cost = bv.cost;
+        } else if (pk->prop != ACE_PROP_INVARIANT) {
+            // one record per A2B nonzero: the AA column's pooled factor ids
+            // and order, and the product of the m < 0 factor signs
+            std::vector<BtRec> rec(std::max(1, pk->a2b_nnz));
+            for (int z = 0; z < pk->a2b_nnz; ++z) {
+                const int col = pk->a2b_cols[z];
+                BtRec& r = rec[z];
+                r.o = pk->orders[col];
+                r.z = z;
+                r.sgn = 1.0;
+                for (int q = 0; q < 4; ++q) {
+                    r.f[q] = 0;
+                    if (q < r.o) {
+                        const int iA = pk->iAA2iA[(size_t)col * pk->maxorder + q];
+                        r.f[q] = pk->aspec_fid[iA];
+                        r.sgn *= pk->aspec_sgn[iA];
+                    }
                 }
             }
-            r.coef = pk->prop == ACE_PROP_INVARIANT ? pk->a2b_vals[z] * sg : sg;
-        }
-        // every row's nonzeros ordered by the order of their AA column, and
-        // where each order's records start, so that the kernel runs one
-        // straight-line loop per order (orders 0 to 4; larger bases do not
-        // use the fused kernel)
-        std::vector<int32_t> rowo((size_t)std::max(1, pk->nB) * BT_ROWO, 0);
-        for (int b = 0; b < pk->nB; ++b) {
-            const int z0 = pk->a2b_rowptr[b], z1 = pk->a2b_rowptr[b + 1];
-            std::stable_sort(rec.begin() + z0, rec.begin() + z1, [](const BtRec& x, const BtRec& y) { return x.o < y.o; });
-            int32_t* ro = rowo.data() + (size_t)b * BT_ROWO;
-            ro[0] = z0;
-            for (int o = 0; o + 1 < BT_ROWO; ++o) {
-                int n = 0;
-                for (int z = z0; z < z1; ++z) n += rec[z].o == o;
-                ro[o + 1] = ro[o] + n;
+            // every row's nonzeros ordered by the order of their AA column, and
+            // where each order's records start, so that the kernel runs one
+            // straight-line loop per order (orders 0 to 4)
+            std::vector<int32_t> rowo((size_t)std::max(1, pk->nB) * BT_ROWO, 0);
+            for (int b = 0; b < pk->nB; ++b) {
+                const int z0 = pk->a2b_rowptr[b], z1 = pk->a2b_rowptr[b + 1];
+                std::stable_sort(rec.begin() + z0, rec.begin() + z1, [](const BtRec& x, const BtRec& y) { return x.o < y.o; });
+                int32_t* ro = rowo.data() + (size_t)b * BT_ROWO;
+                ro[0] = z0;
+                for (int o = 0; o + 1 < BT_ROWO; ++o) {
+                    int n = 0;
+                    for (int z = z0; z < z1; ++z) n += rec[z].o == o;
+                    ro[o + 1] = ro[o] + n;
+                }
             }
+            if (ctx->bt_rec.upload(rec.data(), rec.size()) || ctx->bt_rowo.upload(rowo.data(), rowo.size()))
+                return fail("upload");
         }
-        if (ctx->bt_rec.upload(rec.data(), rec.size()) || ctx->bt_rowo.upload(rowo.data(), rowo.size()))
-            return fail("upload");
         std::vector<int32_t> a4 = acehost::aspec_rows(pk);
         if (ctx->aspec4.upload(a4.data(), a4.size())) return fail("upload");
         std::vector<int16_t> kx = acehost::pool_lookup(pk);

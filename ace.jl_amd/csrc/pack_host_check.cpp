@@ -6,6 +6,7 @@
 #include <map>
 #include <set>
 
+#include "basis_host.hpp"
 #include "compile_host.hpp"
 #include "nbrlist_host.hpp"
 #include "pack_host.hpp"
@@ -184,4 +185,52 @@ extern "C" int64_t acehost_compiled_array(void* p, const char* name, void* out) 
     ACE_ARR(wave_etask_list)
 #undef ACE_ARR
     return -1;
+}
+
+// The basis-value records run on the CPU as k_Bv runs them on pooled values
+// A[npool] and directions W[npool] (re, im): B[nB] and its derivative D[nB],
+// with nchunk workgroups a tile.  Returns 0, 1 when the basis has no such
+// records, -1 when a row is not written exactly once or a unit's records are
+// not where it begins.
+extern "C" int acehost_bv(const ace_pack* pk, int nchunk, const double* A, const double* W, double* B, double* D) {
+    if (!acehost::validate_pack(pk).empty()) return -1;
+    if (!acehost::bv_usable(pk)) return 1;
+    const acehost::BvProgram p = acehost::bv_program(pk);
+    typedef std::complex<double> C;
+    auto val = [](const double* x, uint16_t f) {
+        const C a(x[2 * (f & 0x1ff)], x[2 * (f & 0x1ff) + 1]);
+        return f & 0x8000 ? std::conj(a) : a;
+    };
+    std::vector<int> seen((size_t)pk->nB, 0);
+    const int uw = acehost::BV_UNITS / acehost::BV_WAVES / nchunk;
+    for (int w = 0; w < nchunk * acehost::BV_WAVES; ++w) {
+        const int32_t* u = p.unit.data() + 2 * (size_t)w * uw;
+        int pair = u[1];
+        double b = 0.0, d = 0.0;
+        for (int g = u[0]; g < u[2 * uw]; ++g) {
+            const int row = p.seg[2 * (size_t)g], n = p.seg[2 * (size_t)g + 1] & 0xfffffff, o = p.seg[2 * (size_t)g + 1] >> 28;
+            for (int i = 0; i < 2 * n; ++i) {
+                const acehost::BvRec& r = p.rec[2 * (size_t)pair + i];
+                if (o > 0 && (r.f[0] & 0x8000)) return -1;
+                C x = 1.0, dx = 0.0;
+                for (int q = 0; q < o; ++q) {
+                    dx = dx * val(A, r.f[q]) + x * val(W, r.f[q]);
+                    x *= val(A, r.f[q]);
+                }
+                b += r.c * x.real();
+                d += r.c * dx.real();
+            }
+            pair += n;
+            if (row < 0) {
+                seen[(size_t)(row & 0x7fffffff)] += 1;
+                B[row & 0x7fffffff] = b;
+                D[row & 0x7fffffff] = d;
+                b = d = 0.0;
+            }
+        }
+        if (pair != u[2 * uw + 1] || 2 * (size_t)pair + 2 > p.rec.size()) return -1;
+    }
+    for (int n : seen)
+        if (n != 1) return -1;
+    return 0;
 }

@@ -1,0 +1,35 @@
+"""Fused basis values and their directional derivative on the GPU against the
+oracle at the edges of the kernel's range: tiles of 32 environments (one, a
+full one, one more, several), orders 1 to 4, one and two species, pooled
+values up to the limit of two staged tiles (160) and past it.  Tolerances are
+those of the other parity tests (1e-12 for values, 1e-10 for derivatives)."""
+import numpy as np
+import pytest
+import torch
+
+import ace_oracle as O
+from acehip import synth
+from acehip.evaluator import EnvBatch, HIPEvaluator
+from helpers import basis_for, random_batch, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("args,species,nenv", [((1, 4, 2), 0, 1), ((2, 6, 3), 0, 33), ((3, 6, 4), 0, 32),
+                                               ((4, 8, 4), 0, 97), ((3, 6, 3), 2, 31), ((2, 13, 6), 0, 40),
+                                               ((2, 16, 7), 0, 5), ((4, 10, 5), 0, 700)])
+def test_basis_values(cuda, args, species, nenv):
+    print(f"[gpu] basis values {args} species {species} nenv {nenv}", flush=True)
+    basis, T = basis_for(*args, species=species)
+    off, R, sp = random_batch(nenv, 9, nspecies=species)
+    ev = HIPEvaluator(basis, synth.coefficients(len(basis), 3), device=0)
+    b = EnvBatch(off, R.T.copy(), sp, device="cuda:0")
+    w = np.random.default_rng(4).normal(size=R.shape)
+    B = ev.basis_B(b).cpu().numpy()
+    D = ev.adjoint_EVAL_D(b, torch.as_tensor(w.T.copy())).cpu().numpy()
+    assert rel_err(B, O.eval_B(T, O.eval_AA(T, O.eval_A(T, off, R, sp)))) < 1e-12
+    # the oracle's derivative one environment at a time: the first and the last ones
+    es = sorted(set(range(min(nenv, 40))) | set(range(max(0, nenv - 9), nenv)))
+    ref = [O.adjoint_EVAL_D(T, None, off[e:e + 2] - off[e], R[off[e]:off[e + 1]], w[off[e]:off[e + 1]],
+                            None if sp is None else sp[off[e]:off[e + 1]]) for e in es]
+    assert rel_err(D[es], np.stack(ref).reshape(len(es), -1)) < 1e-10
