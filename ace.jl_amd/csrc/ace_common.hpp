@@ -253,7 +253,8 @@ constexpr int PAIR_MAX_POOL = 159;
 constexpr int PAIR_CAP = 96;
 struct PairDev {
     acehost::PairProgram host;
-    DevBuf<uint32_t> words;
+    DevBuf<uint32_t> words, virt, back;
+    DevBuf<int32_t> back_ptr;
     DevBuf<double> coef;
     DevBuf<int32_t> seq[acehost::PAIR_MAXP + 2];
 };

@@ -1,5 +1,5 @@
 // libacehip.so, pair kernel: site energies and the adjoint G of Invariant
-// bases of correlation order 3 and 4 (evaluator.jl:121-185 restated on A+) as a
+// bases of correlation order 3 to 7 (evaluator.jl:121-185 restated on A+) as a
 // quadratic form in the products of two pooled values; the programs are
 // compiled by pairs_host.hpp, whose head states the form.
 #include "ace_common.hpp"
@@ -12,7 +12,11 @@ struct PairArgs {
     const int32_t* seq;  // the parts of the first ntile_lo tiles: their rounds
     const int32_t* seq_hi;  // and those of the tail tiles, parts + 1 workgroups each
     int32_t seq_ptr[acehost::PAIR_MAXP + 1], seq_ptr_hi[acehost::PAIR_MAXP + 1];
-    int npool;
+    // products that are values of their own, and what they pass on
+    const uint32_t* virt;
+    const uint32_t* back;
+    const int32_t* back_ptr;
+    int npool, nvirt;
     int parts;
     int64_t ntile_lo;
 };
@@ -134,6 +138,9 @@ struct PairSums {
 // A+ and storing G.  Energies alone need no turns: 0.51 ms (0.79 ms).  Columns
 // per panel and rows per panel: 8 rows keep 64 % of the coefficients nonzero;
 // 16 rows 47 %, more multiply-adds on zeros than products saved.
+// Order 5, degree 10, Lmax 4 (84 pooled values and 36 products of their own):
+// 0.394 ms for 30,000 environments; with each monomial's five factors
+// multiplied out in the segment kernel, 0.973 ms.
 template <bool FORCES>
 __global__ __launch_bounds__(1024) void k_pairs(PairArgs a, int64_t nenv, const double* __restrict__ Aplus,
                                                 int64_t estride, double* __restrict__ E_out,
@@ -163,6 +170,22 @@ __global__ __launch_bounds__(1024) void k_pairs(PairArgs a, int64_t nenv, const 
     const char* const a16 = lds + 16 * (lane >> 1);
     const char* const oth = lds + 8 * (lane ^ 1);
     const uint32_t mim = (uint32_t)lane << 31;  // sign bit in imaginary lanes
+    // own part of (x.x + i x.y) X, X the value at o or its conjugate (cj: sign
+    // bit set): re x.x X.re - x.y X.im, im x.x X.im + x.y X.re
+    auto times = [&](double2 x, uint32_t o, uint32_t cj) {
+        return fma(xor_hi(x.y, mim ^ 0x80000000u ^ (cj & ~mim)), *reinterpret_cast<const double*>(oth + o),
+                   xor_hi(x.x, cj & mim) * *reinterpret_cast<const double*>(own + o));
+    };
+    if (a.nvirt > 0) {
+        PairWord* const vw = (PairWord*)(uintptr_t)a.virt;
+        for (int i = wave; i < a.nvirt; i += NW) {
+            const uint32_t oa = vw[2 * i], od = vw[2 * i + 1];
+            char* const to = own + (a.npool + 1 + i) * RB;
+            *reinterpret_cast<double*>(to) = times(*reinterpret_cast<const double2*>(a16 + oa), od & ~1u, od << 31);
+            if (FORCES) *reinterpret_cast<double*>(to + 512) = 0.0;
+        }
+        __syncthreads();
+    }
     double e = 0.0;
     // one panel: h_p of its rows, then h_p X_d and h_p X_a per row (forces), and
     // its energy
@@ -263,10 +286,23 @@ __global__ __launch_bounds__(1024) void k_pairs(PairArgs a, int64_t nenv, const 
         for (int q = 0; q < acehost::PAIR_SLOTS; ++q) po[q] = pn[q];
     }
     __syncthreads();
-    if (FORCES && valid)
-        for (int k = wave; k < a.npool; k += NW)
-            __builtin_nontemporal_store(*reinterpret_cast<const double*>(own + k * RB + 512),
-                                        Gbuf + 2 * (((int64_t)part * a.npool + k) * estride + env0) + lane);
+    if (FORCES) {
+        PairInt* const bp = (PairInt*)(uintptr_t)a.back_ptr;
+        PairWord* const bw = (PairWord*)(uintptr_t)a.back;
+        for (int k = wave; k < a.npool; k += NW) {
+            double g = *reinterpret_cast<const double*>(own + k * RB + 512);
+            if (a.nvirt > 0)
+                for (int i = bp[k]; i < bp[k + 1]; ++i) {
+                    const uint32_t o = bw[2 * i + 1];
+                    const double2 gu = *reinterpret_cast<const double2*>(a16 + bw[2 * i] + 512);
+                    const double t = times(gu, o & ~3u, (o & acehost::PAIR_BACK_IN) << 31);
+                    g += xor_hi(t, (o & acehost::PAIR_BACK_OUT ? 0x80000000u : 0u) & mim);
+                }
+            if (valid)
+                __builtin_nontemporal_store(g, Gbuf + 2 * (((int64_t)part * a.npool + k) * estride + env0) + lane);
+        }
+        if (a.nvirt > 0) __syncthreads();  // the A+ rows are read above and reused below
+    }
     // energy: the waves' sums over the A+ rows, which nothing reads any more
     if (FORCES) e = xor_hi(e, mim);
     e += dpp<DPP_SWAP>(e);
@@ -286,24 +322,28 @@ __global__ __launch_bounds__(1024) void k_pairs(PairArgs a, int64_t nenv, const 
 
 }  // namespace
 
-// LDS bytes of a workgroup: the pooled values and the constant, at least one
-// row per wave for the energy sums.
-static size_t pair_lds(int npool, bool forces) {
-    return (size_t)std::max(npool + 1, acehost::PAIR_WAVES) * (forces ? 1024 : 512);
+// LDS bytes of a workgroup: the pooled values, the constant and the products
+// of their own, at least one row per wave for the energy sums.
+static size_t pair_lds(int npool, int nvirt, bool forces) {
+    return (size_t)std::max(npool + 1 + nvirt, acehost::PAIR_WAVES) * (forces ? 1024 : 512);
 }
 
 int pairs_create(ace_ctx* ctx, const std::vector<int32_t>& pool) {
     ctx->pairs_ok = false;
-    if (ctx->prop != ACE_PROP_INVARIANT || ctx->maxorder < 3 || ctx->maxorder > 4 || ctx->npool > PAIR_MAX_POOL ||
+    if (ctx->prop != ACE_PROP_INVARIANT || ctx->maxorder < 3 || ctx->npool > PAIR_MAX_POOL ||
         ctx->ngslots < ctx->npool)
         return 0;
     acehost::PairForm pf;
-    if (!acehost::pair_form(ctx->host, pool, pf).empty() || pf.entries.empty()) return 0;  // other kernels take it
+    if (!acehost::pair_form(ctx->host, pool, PAIR_MAX_POOL, pf).empty() || pf.entries.empty()) return 0;  // other kernels take it
     for (int m = 0; m < 2; ++m) {
         PairDev& d = ctx->pairs[m];
         const std::string err = acehost::pair_program(pf, m == 0, m == 0 ? 1024 : 512, ctx->npool, PAIR_CAP, d.host);
         if (!err.empty()) return set_err(err);
-        if (d.words.upload(d.host.words.data(), d.host.words.size())) return -1;
+        if (d.words.upload(d.host.words.data(), d.host.words.size()) ||
+            d.virt.upload(d.host.virt.data(), d.host.virt.size()) ||
+            d.back.upload(d.host.back.data(), d.host.back.size()) ||
+            d.back_ptr.upload(d.host.back_ptr.data(), d.host.back_ptr.size()))
+            return -1;
         for (int P = 1; P <= acehost::PAIR_MAXP + 1; ++P)
             if (d.seq[P].upload(d.host.seq[P].data(), d.host.seq[P].size())) return -1;
     }
@@ -331,10 +371,14 @@ int launch_pairs(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, bo
     a.seq_hi = d.seq[P + 1].p;
     for (int q = 0; q < P; ++q) a.seq_ptr[q] = d.host.seq_ptr[P][(size_t)q];
     for (int q = 0; q < P + 1; ++q) a.seq_ptr_hi[q] = d.host.seq_ptr[P + 1][(size_t)q];
+    a.virt = d.virt.p;
+    a.back = d.back.p;
+    a.back_ptr = d.back_ptr.p;
     a.npool = ctx->npool;
+    a.nvirt = (int)d.host.virt.size() / 2;
     a.parts = P;
     a.ntile_lo = ntile - nhi;
-    const size_t lds = pair_lds(ctx->npool, forces);
+    const size_t lds = pair_lds(ctx->npool, a.nvirt, forces);
     auto go = [&](auto kern) {
         if (set_func_lds((const void*)kern, lds)) return -1;
         hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(64 * acehost::PAIR_WAVES), lds, st, a, nenv,

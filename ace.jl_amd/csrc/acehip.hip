@@ -1218,14 +1218,18 @@ static int segment_parts(const ace_ctx* ctx, int64_t ntile, int ntask, int W) {
 // for (ace_set_kernel), and the programs are long enough.  Order 4: always
 // (with forces at 100,000 / 8,000 / 64 environments: degree 12 1.52 / 0.143 /
 // 0.029 ms against the segment kernel's 2.89 / 0.287 / 0.126, degree 8 0.299 /
-// 0.024 / 0.016 against 0.387 / 0.057 / 0.054).  Order 3: its rounds are few
+// 0.024 / 0.016 against 0.387 / 0.057 / 0.054).  Orders 5 to 7: always (order
+// 5, degree 10 at 60,000 / 8,000 / 64: 0.746 / 0.104 / 0.026 ms against 1.807 /
+// 0.272 / 0.176, energies alone 0.252 / 0.045 / 0.022 against 0.412 / 0.105 /
+// 0.099; order 6, degree 7 0.226 / 0.030 / 0.018 against 0.390 / 0.095 / 0.088;
+// order 5, degree 6, the closest, 0.133 against 0.142 at 60,000).  Order 3: its rounds are few
 // and their barriers show once every CU has more than one tile (degree 10,
 // 100,000 environments 0.382 against 0.298 ms, 1,000 0.019 against 0.024), for
 // energies alone, without barriers, never (0.097 against 0.107).  Below order 3
 // the segment kernel (energies of one environment 8 against 11 us).
 static bool use_pairs(const ace_ctx* ctx, int64_t nenv, bool forces) {
     if (!ctx->pairs_ok || ctx->force_interp || ctx->rec_dispatch) return false;
-    return ctx->maxorder == 4 || !forces || (nenv + 31) / 32 <= ctx->ncu;
+    return ctx->maxorder >= 4 || !forces || (nenv + 31) / 32 <= ctx->ncu;
 }
 
 // Workgroups per 32-environment tile of the pair kernel, and tail tiles.

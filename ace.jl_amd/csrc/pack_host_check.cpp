@@ -55,17 +55,21 @@ extern "C" int acehost_pairs(const ace_pack* pk, const double* c, int forces, in
     const int np = pk->npool, rb = forces ? 1024 : 512;
     acehost::PairForm pf;
     acehost::PairProgram pp;
-    if (!acehost::pair_form(pc, std::vector<int32_t>(pk->pool, pk->pool + 4 * (size_t)np), pf).empty()) return 1;
+    if (!acehost::pair_form(pc, std::vector<int32_t>(pk->pool, pk->pool + 4 * (size_t)np), 159, pf).empty()) return 1;
     if (!acehost::pair_program(pf, forces != 0, rb, np, 96, pp).empty()) return -1;
     const acehost::Coeffs cf = acehost::coefficients(pc, c);
     acehost::pair_coefs(pp, cf.leaf);
     typedef std::complex<double> C;
+    const int nrow = np + 1 + (int)pf.virt.size();
+    std::vector<C> row;
     auto val = [&](uint32_t w) {
-        const int k = (int)(w & ~1u) / rb;
-        const C a = k == np ? C(1.0) : C(A[2 * k], A[2 * k + 1]);
+        const C a = row[(w & ~1u) / rb];
         return w & 1u ? std::conj(a) : a;
     };
-    std::vector<C> g((size_t)np + 1, 0.0);
+    for (int k = 0; k < np; ++k) row.push_back(C(A[2 * k], A[2 * k + 1]));
+    row.push_back(1.0);
+    for (size_t i = 0; i < pf.virt.size(); ++i) row.push_back(val(pp.virt[2 * i]) * val(pp.virt[2 * i + 1]));
+    std::vector<C> g((size_t)nrow, 0.0);
     double e = 0.0;
     for (int part = 0; part < parts; ++part) {
         const int32_t* sq = pp.seq[parts].data() + pp.seq_ptr[parts][(size_t)part];
@@ -91,8 +95,8 @@ extern "C" int acehost_pairs(const ace_pack* pk, const double* c, int forces, in
                     e += (gp * val(wa) * val(wd)).real();
                     g[(size_t)ka] += gp * val(wd);
                     g[(size_t)kd] += wd & 1u ? std::conj(t2) : t2;
-                    if (ka < np) mine.insert(ka);
-                    if (kd < np) mine.insert(kd);
+                    if (ka != np) mine.insert(ka);
+                    if (kd != np) mine.insert(kd);
                 }
                 if (!forces) continue;
                 const int turn = (int)(hd[1] >> 8);
@@ -103,6 +107,12 @@ extern "C" int acehost_pairs(const ace_pack* pk, const double* c, int forces, in
         }
     }
     *E = cf.e0[0] + (forces ? 0.5 : 1.0) * e;
+    for (int k = 0; k < np; ++k)
+        for (int i = pp.back_ptr[(size_t)k]; i < pp.back_ptr[(size_t)k + 1]; ++i) {
+            const uint32_t o = pp.back[2 * (size_t)i + 1];
+            const C x = row[(o & ~3u) / rb], t = g[pp.back[2 * (size_t)i] / rb] * (o & acehost::PAIR_BACK_IN ? std::conj(x) : x);
+            g[(size_t)k] += o & acehost::PAIR_BACK_OUT ? std::conj(t) : t;
+        }
     for (int k = 0; forces && k < np; ++k) {
         G[2 * k] = g[(size_t)k].real();
         G[2 * k + 1] = g[(size_t)k].imag();

@@ -1,6 +1,13 @@
 // Host-side (CPU) compiler of the pair programs: the site energy of an
-// Invariant basis of correlation order <= 4 as a quadratic form in the
-// products of two pooled values, for the kernel k_pairs (ace_pairs.hip).
+// Invariant basis as a quadratic form in the products of two pooled values,
+// for the kernel k_pairs (ace_pairs.hip).
+//
+// Monomials of more than four factors (correlation order 5 to 7) are first
+// brought to four: products of two pooled values that occur in many of them
+// become values of their own, rows behind the pooled ones (greedily, the product
+// that shortens most monomials next; order 5 of degree 10: 36 rows for 7,128
+// monomials of five factors).  G of such a row u = X_s X_t is passed on in the
+// end: G[s] += G_u X_t, G[t] += G_u X_s.
 //
 // Every monomial of the energy polynomial E = c0 + Re sum c prod X_f (X_f =
 // A+[k] or its conjugate; the reference's sum over AA functions,
@@ -48,6 +55,8 @@ constexpr int pair_rec_words(int nq) { return 1 + nq; }
 // two addresses, two products and 8 multiply-adds.
 constexpr int pair_rec_cost(int nq) { return 6 + 12 * nq; }
 
+constexpr uint32_t PAIR_BACK_IN = 1, PAIR_BACK_OUT = 2;
+
 // One mode's program.  Panel words: [records of 4 | of 2 << 10 | of 1 << 20
 // columns, rows | turn << 8, first coefficient, cost of the records], then per
 // row the LDS offsets of its two factors (bit 0 of the second: the second
@@ -67,6 +76,12 @@ struct PairProgram {
         float scale;
     };
     std::vector<Term> terms;
+    // products of their own: [row] LDS offsets of the two factors (bit 0 of the
+    // second: conjugated); and per pooled value k those it is a factor of:
+    // back_ptr[npool + 1], then [offset of the product's row, offset of the
+    // other factor | PAIR_BACK_IN: conjugated | PAIR_BACK_OUT: the sum is]
+    std::vector<uint32_t> virt, back;
+    std::vector<int32_t> back_ptr;
     // the rounds of each of P workgroups: at seq_ptr[P][part] their count, then
     // the rounds (PAIR_SEQ words each), one unused round behind the last
     std::vector<int32_t> seq_ptr[PAIR_MAXP + 2], seq[PAIR_MAXP + 2];
@@ -77,7 +92,7 @@ struct PairProgram {
 // The monomials of the energy polynomial: factors (device ids) and leaf index.
 struct PairMono {
     int n;
-    uint16_t f[4];
+    uint16_t f[7];
     int32_t leaf;
 };
 
@@ -85,56 +100,38 @@ struct PairMono {
 // matrix per class (m, parity of l).
 struct PairForm {
     struct Half {
-        uint16_t a, d;  // x = A[a] * (conj ? conj(A[d]) : A[d]); ONE = npool
+        uint16_t a, d;  // x = A[a] * (conj ? conj(A[d]) : A[d]); ONE = npool, rows of virt behind it
         bool conj;
     };
     struct Entry {
         int32_t p, q, leaf;
     };
+    std::vector<Half> virt;    // products that are values of their own
     std::vector<Half> halves;
     std::vector<int> cls;      // class of every half
     std::vector<Entry> entries;
     int ncls = 0;
 };
 
-inline std::string pair_form(const PackCopy& pc, const std::vector<int32_t>& pool, PairForm& out) {
+// max_rows: pooled values and products of their own that the kernel has room for.
+inline std::string pair_form(const PackCopy& pc, const std::vector<int32_t>& pool, int max_rows, PairForm& out) {
     const int npool = (int)pool.size() / 4, ONE = npool;
-    auto m_of = [&](uint32_t f) {
-        const int k = (int)(f & 0x7fff);
-        if (k == ONE) return 0;
-        const int m = pool[4 * (size_t)k + 3];
-        return (f & 0x8000) ? -m : m;
-    };
-    auto deg = [&](uint32_t f) {
-        const int k = (int)(f & 0x7fff);
-        return k == ONE ? 0 : pool[4 * (size_t)k + 1] - 1 + pool[4 * (size_t)k + 2];
-    };
-    auto par = [&](uint32_t f) {
-        const int k = (int)(f & 0x7fff);
-        return k == ONE ? 0 : pool[4 * (size_t)k + 2] & 1;
-    };
-    auto cj = [&](uint32_t f) { return m_of(f) == 0 ? f & 0x7fffu : f ^ 0x8000u; };
-    std::vector<PairMono> monos;
-    for (int t = 0; t < pc.ntasks; ++t) {
-        if (pc.tasks[5 * (size_t)t + 2] >= 0) continue;  // gradient tasks
-        if (pc.task_term_ptr[t + 1] != pc.task_term_ptr[t]) return "energy task with constant terms";
-        for (int r = pc.tasks[5 * (size_t)t]; r < pc.tasks[5 * (size_t)t + 1]; ++r) {
-            const int32_t* run = pc.runs.data() + (size_t)ACE_RUN_W * r;
-            if (run[0] > 3) return "correlation order above 4";
-            for (int i = 0; i < run[2]; ++i) {
-                PairMono m;
-                m.n = run[0] + 1;
-                for (int q = 0; q < run[0]; ++q) m.f[q] = (uint16_t)run[4 + q];
-                m.f[run[0]] = (uint16_t)pc.leaf_fid[(size_t)run[3] + i];
-                for (int q = m.n; q < 4; ++q) m.f[q] = (uint16_t)ONE;
-                m.leaf = run[3] + i;
-                monos.push_back(m);
-            }
-        }
+    out = PairForm();
+    // |m|, degree and parity of l of every row
+    std::vector<int> rm, rdeg, rpar;
+    for (int k = 0; k < npool; ++k) {
+        rm.push_back(pool[4 * (size_t)k + 3]);
+        rdeg.push_back(pool[4 * (size_t)k + 1] - 1 + pool[4 * (size_t)k + 2]);
+        rpar.push_back(pool[4 * (size_t)k + 2] & 1);
     }
-    // halves up to conjugation, m >= 0, the conjugated factor (if any) second
-    std::unordered_map<uint32_t, int32_t> ids;
-    std::map<std::pair<int, int>, int> classes;
+    rm.push_back(0);
+    rdeg.push_back(0);
+    rpar.push_back(0);
+    auto m_of = [&](uint32_t f) { return (f & 0x8000) ? -rm[f & 0x7fff] : rm[f & 0x7fff]; };
+    auto deg = [&](uint32_t f) { return rdeg[f & 0x7fff]; };
+    auto par = [&](uint32_t f) { return rpar[f & 0x7fff]; };
+    auto cj = [&](uint32_t f) { return m_of(f) == 0 ? f & 0x7fffu : f ^ 0x8000u; };
+    // a product up to conjugation, m >= 0, the conjugated factor (if any) second
     auto half_key = [&](uint32_t f, uint32_t g) -> uint32_t {
         if (m_of(f) + m_of(g) < 0) {
             f = cj(f);
@@ -144,9 +141,73 @@ inline std::string pair_form(const PackCopy& pc, const std::vector<int32_t>& poo
         if ((fc && !gc) || (fc == gc && f > g)) std::swap(f, g);
         return f << 16 | g;
     };
+    // one real coefficient serves both parts: not for m = 0 products of complex factors
+    auto usable = [&](uint32_t f, uint32_t g) { return m_of(f) + m_of(g) != 0 || (m_of(f) == 0 && m_of(g) == 0); };
+    std::vector<PairMono> monos;
+    for (int t = 0; t < pc.ntasks; ++t) {
+        if (pc.tasks[5 * (size_t)t + 2] >= 0) continue;  // gradient tasks
+        if (pc.task_term_ptr[t + 1] != pc.task_term_ptr[t]) return "energy task with constant terms";
+        for (int r = pc.tasks[5 * (size_t)t]; r < pc.tasks[5 * (size_t)t + 1]; ++r) {
+            const int32_t* run = pc.runs.data() + (size_t)ACE_RUN_W * r;
+            if (run[0] > 6) return "correlation order above 7";  // the last two of 8 factors may be X and its conjugate
+            for (int i = 0; i < run[2]; ++i) {
+                PairMono m;
+                m.n = run[0] + 1;
+                for (int q = 0; q < run[0]; ++q) m.f[q] = (uint16_t)run[4 + q];
+                m.f[run[0]] = (uint16_t)pc.leaf_fid[(size_t)run[3] + i];
+                m.leaf = run[3] + i;
+                monos.push_back(m);
+            }
+        }
+    }
+    // products of their own until no monomial has more than four factors
+    for (;;) {
+        std::unordered_map<uint32_t, int> count;
+        for (const PairMono& m : monos) {
+            if (m.n <= 4) continue;
+            uint32_t seen[21];
+            int ns = 0;
+            for (int i = 0; i < m.n; ++i)
+                for (int j = i + 1; j < m.n; ++j) {
+                    if ((m.f[i] & 0x7fff) > ONE || (m.f[j] & 0x7fff) > ONE || !usable(m.f[i], m.f[j])) continue;
+                    const uint32_t k = half_key(m.f[i], m.f[j]);
+                    if (std::find(seen, seen + ns, k) == seen + ns) seen[ns++] = k;
+                }
+            if (ns == 0) return "monomial without a product to replace";
+            for (int i = 0; i < ns; ++i) ++count[seen[i]];
+        }
+        if (count.empty()) break;
+        if (npool + (int)out.virt.size() >= max_rows) return "too many products";
+        uint32_t key = 0;
+        int most = 0;
+        for (const auto& kv : count)
+            if (kv.second > most || (kv.second == most && kv.first < key)) {
+                key = kv.first;
+                most = kv.second;
+            }
+        const uint32_t f = key >> 16, g = key & 0xffffu, u = (uint32_t)rm.size();
+        out.virt.push_back({(uint16_t)(f & 0x7fff), (uint16_t)(g & 0x7fff), (g & 0x8000) != 0});
+        rm.push_back(m_of(f) + m_of(g));
+        rdeg.push_back(deg(f) + deg(g));
+        rpar.push_back((par(f) + par(g)) & 1);
+        for (PairMono& m : monos)
+            for (int i = 0; i < m.n && m.n > 4; ++i)
+                for (int j = i + 1; j < m.n && m.n > 4; ++j) {
+                    const uint32_t a = m.f[i], b = m.f[j];
+                    if ((int)(a & 0x7fff) > ONE || (int)(b & 0x7fff) > ONE || !usable(a, b) || half_key(a, b) != key) continue;
+                    m.f[i] = (uint16_t)(m_of(a) + m_of(b) < 0 ? u | 0x8000u : u);
+                    m.f[j] = m.f[m.n - 1];
+                    --m.n;
+                    j = i;  // the rest against the new factor: it is passed over
+                }
+    }
+    for (PairMono& m : monos)
+        for (int q = m.n; q < 4; ++q) m.f[q] = (uint16_t)ONE;
+    std::unordered_map<uint32_t, int32_t> ids;
+    std::map<std::pair<int, int>, int> classes;
     auto half = [&](uint32_t f, uint32_t g) -> int32_t {
         const int M = std::abs(m_of(f) + m_of(g));
-        if (M == 0 && (m_of(f) != 0 || m_of(g) != 0)) return -1;  // not a real product
+        if (!usable(f, g)) return -1;
         const uint32_t key = half_key(f, g);
         f = key >> 16;
         g = key & 0xffffu;
@@ -160,7 +221,6 @@ inline std::string pair_form(const PackCopy& pc, const std::vector<int32_t>& poo
         ids.emplace(key, id);
         return id;
     };
-    out = PairForm();
     for (const PairMono& m : monos) {
         // the three splits of four factors; shorter monomials are padded with
         // the constant and keep one factor per half where they can
@@ -203,6 +263,25 @@ inline std::string pair_form(const PackCopy& pc, const std::vector<int32_t>& poo
 inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, int npool, int cap, PairProgram& out) {
     out = PairProgram();
     const int nh = (int)pf.halves.size();
+    {
+        std::vector<std::vector<uint32_t>> back((size_t)npool);
+        for (size_t i = 0; i < pf.virt.size(); ++i) {
+            const PairForm::Half& v = pf.virt[i];
+            const uint32_t u = ((uint32_t)npool + 1 + (uint32_t)i) * row_bytes, oa = (uint32_t)v.a * row_bytes,
+                           od = (uint32_t)v.d * row_bytes;
+            out.virt.push_back(oa);
+            out.virt.push_back(od | (v.conj ? 1u : 0u));
+            back[v.a].push_back(u);
+            back[v.a].push_back(od | (v.conj ? PAIR_BACK_IN : 0u));
+            back[v.d].push_back(u);
+            back[v.d].push_back(oa | (v.conj ? PAIR_BACK_OUT : 0u));
+        }
+        out.back_ptr.push_back(0);
+        for (const auto& b : back) {
+            out.back.insert(out.back.end(), b.begin(), b.end());
+            out.back_ptr.push_back((int32_t)out.back.size() / 2);
+        }
+    }
     struct Cell {
         int32_t q;
         std::vector<std::pair<int32_t, float>> terms;
@@ -393,7 +472,7 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
                 if (disjoint(panels[i], hit[k]) && (t < 0 || load[k] < load[(size_t)t])) t = (int)k;
             if ((int)hit.size() < most && (t < 0 || load[(size_t)t] >= NP / TURNS)) {
                 t = (int)hit.size();
-                hit.emplace_back((size_t)npool, (char)0);
+                hit.emplace_back((size_t)npool + 1 + pf.virt.size(), (char)0);
                 load.push_back(0);
             }
             if (t < 0) return;

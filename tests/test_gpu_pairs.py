@@ -1,7 +1,8 @@
 """The pair kernel on the GPU against the oracle at the edges of its range:
 tiles of 32 environments (one, a full one, one more), few and many pooled
 values up to its limit of 159 and past it (another kernel), one and two
-species, an order-3 batch past one tile per compute unit (another kernel), and every split of a tile over workgroups, whose G shares the force
+species, an order-3 batch past one tile per compute unit (another kernel),
+orders 5 to 7, and every split of a tile over workgroups, whose G shares the force
 kernels add up.  Tolerances are those of the other parity tests (1e-12 for
 energies, 1e-10 for gradients, of the largest value); splits only change the
 order of a few sums, 1e-13."""
@@ -19,7 +20,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("args,species,nenv", [((3, 4, 2), 0, 33), ((4, 5, 3), 0, 1), ((3, 6, 4), 0, 32),
                                                ((3, 13, 5), 0, 9), ((2, 13, 6), 0, 40), ((3, 6, 3), 2, 31),
-                                               ((4, 8, 4), 0, 70), ((3, 6, 4), 0, 8193)])
+                                               ((4, 8, 4), 0, 70), ((3, 6, 4), 0, 8193),
+                                               # products of their own behind the pooled values
+                                               ((5, 6, 3), 0, 33), ((5, 5, 3), 2, 40), ((7, 5, 2), 0, 65)])
 def test_pair_kernel(cuda, args, species, nenv):
     print(f"[gpu] pair kernel {args} species {species} nenv {nenv}", flush=True)
     basis, T = basis_for(*args, species=species)

@@ -44,7 +44,9 @@ def direct(pk, ct, A):
 
 
 @pytest.mark.parametrize("args,kw", [((1, 4, 2), {}), ((2, 5, 3), {}), ((3, 6, 4), {}), ((4, 8, 4), {}),
-                                     ((4, 12, 6), {}), ((2, 13, 5), {}), ((3, 6, 3), {"species": 2})])
+                                     ((4, 12, 6), {}), ((2, 13, 5), {}), ((3, 6, 3), {"species": 2}),
+                                     # monomials brought to four factors first
+                                     ((5, 6, 3), {}), ((5, 5, 3), {"species": 2}), ((6, 6, 3), {}), ((7, 5, 2), {})])
 def test_pair_program(shim, args, kw):
     basis, T = basis_for(*args, **kw)
     pk = Pack(T)
@@ -69,12 +71,3 @@ def test_pair_program(shim, args, kw):
                 d = G[:, 0] + 1j * G[:, 1] - G0
                 # the real (m = 0) pooled values fix the real part only
                 assert np.max(np.abs(np.where(pk.pool[:, 3] > 0, d, d.real))) < 1e-12 * scale
-
-
-def test_order_5_has_no_pair_form(shim):
-    basis, T = basis_for(5, 6, 3)
-    s, keep = _lib.make_pack(Pack(T))
-    z = np.zeros(4096)
-    dp = z.ctypes.data_as(C.POINTER(C.c_double))
-    c = synth.coefficients(len(basis), 5)
-    assert shim.acehost_pairs(C.byref(s), c.ctypes.data_as(C.POINTER(C.c_double)), 1, 1, dp, dp, dp) == 1
