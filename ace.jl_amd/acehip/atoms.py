@@ -150,9 +150,12 @@ class NeighbourList:
         if F is None:
             F = torch.empty((3, self.natoms), dtype=torch.float64, device=self.dev)
         W = torch.empty((3, 3), dtype=torch.float64, device=self.dev) if virial else None
+        self._forces(dE_dr, F, W, stream)
+        return (F, W) if virial else F
+
+    def _forces(self, dE_dr, F, W, stream=None):
         _lib.check(self.lib.ace_nbrlist_forces(self.h, self.natoms, _vp(self.offsets), _vp(self.rev), self.nnbr,
                                                _vp(self.xyz), _vp(dE_dr), _vp(F), _vp(W), self._stream(stream)))
-        return (F, W) if virial else F
 
     def forces_multi(self, g, stream=None):
         """Forces of many fields at once: g (nnbr, nvec, 3) -> F (natoms, nvec, 3)."""
@@ -212,10 +215,14 @@ class ACECalculator:
         """(E total, F (N, 3)[, W (3, 3)]) as NumPy."""
         nl = self._list(at)
         E, dE = self.model.energy_forces(nl.batch())
-        out = nl.forces(dE, virial=virial)
-        F, W = out if virial else (out, None)
-        res = (float(E.sum().item()), F.t().cpu().numpy())
-        return res + (W.cpu().numpy(),) if virial else res
+        # one buffer, so that one copy brings everything to the host
+        n = nl.natoms
+        buf = torch.empty(10 + 3 * n, dtype=torch.float64, device=nl.dev)
+        torch.sum(E, 0, out=buf[0])
+        nl._forces(dE, buf[10:], buf[1:10] if virial else None)
+        host = buf.cpu().numpy()
+        res = (float(host[0]), host[10:].reshape(3, n).T)
+        return res + (host[1:10].reshape(3, 3),) if virial else res
 
     def forces(self, at: Atoms):
         return self.energy_forces(at)[1]

@@ -661,7 +661,6 @@ extern "C" int ace_basis_A(ace_ctx* ctx, int64_t nenv, const int32_t* off, const
                            const int8_t* species, double* A_out, void* stream) {
     int64_t nnbr = 0;
     if (check_common(ctx, nenv, off, xyz, species, &nnbr, stream)) return -1;
-    if (validate_inputs(ctx, nenv, off, nnbr, species, (hipStream_t)stream)) return -1;
     if (nenv == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     if (basis_A_internal(ctx, nenv, off, xyz, species, nnbr, st)) return -1;
@@ -688,7 +687,6 @@ extern "C" int ace_basis_AA(ace_ctx* ctx, int64_t nenv, const int32_t* off, cons
                             const int8_t* species, double* AA_out, void* stream) {
     int64_t nnbr = 0;
     if (check_common(ctx, nenv, off, xyz, species, &nnbr, stream)) return -1;
-    if (validate_inputs(ctx, nenv, off, nnbr, species, (hipStream_t)stream)) return -1;
     if (nenv == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     if (basis_A_internal(ctx, nenv, off, xyz, species, nnbr, st)) return -1;
@@ -755,7 +753,6 @@ extern "C" int ace_basis_B(ace_ctx* ctx, int64_t nenv, const int32_t* off, const
                            const int8_t* species, double* B_out, void* stream) {
     int64_t nnbr = 0;
     if (check_common(ctx, nenv, off, xyz, species, &nnbr, stream)) return -1;
-    if (validate_inputs(ctx, nenv, off, nnbr, species, (hipStream_t)stream)) return -1;
     if (nenv == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     {
@@ -859,7 +856,6 @@ extern "C" int ace_basis_dB(ace_ctx* ctx, int64_t nenv, const int32_t* off, cons
                             const int8_t* species, double* dB_out, void* stream) {
     int64_t nnbr = 0;
     if (check_common(ctx, nenv, off, xyz, species, &nnbr, stream)) return -1;
-    if (validate_inputs(ctx, nenv, off, nnbr, species, (hipStream_t)stream)) return -1;
     if (nenv == 0 || nnbr == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     const int rc = basis_dB_weights(ctx, st, nenv, off, xyz, species, nnbr, dB_out);
@@ -893,7 +889,6 @@ extern "C" int ace_adjoint_EVAL_D(ace_ctx* ctx, int64_t nenv, const int32_t* off
     int64_t nnbr = 0;
     if (check_common(ctx, nenv, off, xyz, species, &nnbr, stream)) return -1;
     if (ctx->prop != ACE_PROP_INVARIANT) return set_err("ace_adjoint_EVAL_D: Invariant bases only");
-    if (validate_inputs(ctx, nenv, off, nnbr, species, (hipStream_t)stream)) return -1;
     if (nenv == 0) return 0;
     if (!dB_out || (nnbr > 0 && !w)) return set_err("ace_adjoint_EVAL_D: null argument");
     hipStream_t st = (hipStream_t)stream;

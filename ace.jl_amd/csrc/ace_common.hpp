@@ -365,9 +365,12 @@ struct ace_ctx {
     DevBuf<int32_t> io_off;
     DevBuf<double> io_xyz, io_w, io_out1, io_out2;
     DevBuf<int8_t> io_sp;
-    // pinned host words for the stream-ordered reads of env_offsets[0] and
-    // env_offsets[nenv] (hipHostMalloc)
+    // pinned host words that the argument checks' kernels write (k_check:
+    // env_offsets[0] and [nenv], what is wrong), their device address, and the
+    // neighbours whose species may be read
     int32_t* h_words = nullptr;
+    int32_t* d_words = nullptr;
+    DevBuf<int32_t> usable;
     // timing
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool timing_valid = false;
@@ -453,13 +456,11 @@ inline RadialParams radial_params(const ace_ctx* ctx) {
 // ---- launchers shared between units (all stream-ordered; 0 or -1 with the
 // error recorded)
 
-// acehip.hip: argument checks of every evaluation call.  check_common
-// returns the neighbour count env_offsets[nenv] (read in stream order);
-// validate_inputs checks offsets and species on the host.
+// acehip.hip: argument checks of every evaluation call: the neighbour count
+// env_offsets[nenv] (read in stream order), and with validation on the order of
+// the offsets and the range of the species.
 int check_common(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* xyz, const int8_t* species,
                  int64_t* nnbr_out, void* stream);
-int validate_inputs(ace_ctx* ctx, int64_t nenv, const int32_t* off, int64_t nnbr, const int8_t* species,
-                    hipStream_t st);
 // acehip.hip: the product DAG over the environments listed in env_list
 // (device count env_count): energies, and the adjoint G with forces.
 int launch_dag_listed(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, bool forces, double* E_out,

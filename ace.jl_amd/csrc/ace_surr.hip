@@ -162,7 +162,6 @@ extern "C" int ace_surr_features(ace_ctx* ctx, int64_t nenv, const int32_t* off,
     int64_t nnbr = 0;
     if (check_common(ctx, nenv, off, xyz, species, &nnbr, stream)) return -1;
     if (ctx->prop != ACE_PROP_INVARIANT || ctx->nfeat < 1) return set_err("surrogate features need an Invariant basis");
-    if (validate_inputs(ctx, nenv, off, nnbr, species, (hipStream_t)stream)) return -1;
     if (nenv == 0) return 0;
     if (!xmean || !xinvstd || !E2) return set_err("ace_surr_features: null argument");
     hipStream_t st = (hipStream_t)stream;
