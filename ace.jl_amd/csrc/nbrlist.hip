@@ -420,67 +420,61 @@ __global__ __launch_bounds__(256) void k_nbr_update(int natoms, NbrArgs a, const
     }
 }
 
-// F_k = sum_{m in N(k)} (g_m - g_rev(m)) for FA_ATOMS atoms per block.  The
-// block's entries [off[a0], off[a0 + FA_ATOMS]) are read coalesced by all
-// threads, FA_CH at a time, as d_m = g_m - g_rev(m) into LDS; then one thread
-// per atom sums its own entries in order.  Virial partials -g_m r_m^T are
-// summed per thread over its strided entries and reduced in a fixed order.
-constexpr int FA_ATOMS = 64;
-constexpr int FA_CH = 1024;
+// F_k = sum_{m in N(k)} (g_m - g_rev(m)): 16 lanes per atom take its entries in
+// turn, four at a time so that their gathers are in flight together, and are
+// summed by a fixed tree.  A workgroup takes `per` groups of 16 atoms, the
+// workgroups of one XCD neighbouring ones.  Virial partials -g_m r_m^T stay in
+// registers to the end and are reduced over the workgroup in a fixed order.
+// Bound by the gathers of g at rev(m), 24 bytes to lines of their own: 55,296 atoms
+// of 54 neighbours, 92 -> 54 us, 256 atoms 36 -> 8 us, against 64 atoms per
+// workgroup staged in LDS, one thread of which then added up each atom.
+constexpr int FA_ATOMS = 16;
+constexpr int FA_BLOCKS = 2048;  // workgroups at most
 
-__global__ __launch_bounds__(256) void k_nbr_forces(int natoms, const int32_t* __restrict__ off,
+__global__ __launch_bounds__(256) void k_nbr_forces(int natoms, int per, const int32_t* __restrict__ off,
                                                     const int32_t* __restrict__ rev, int64_t nnbr,
                                                     const double* __restrict__ g, const double* __restrict__ xyz,
                                                     double* __restrict__ F, double* __restrict__ vpart) {
-    static_assert(9 * 256 <= 3 * FA_CH, "the virial reduction reuses the staging array");
-    __shared__ double dl[3][FA_CH];
-    double (*red)[256] = reinterpret_cast<double (*)[256]>(&dl[0][0]);
-    const int a0 = blockIdx.x * FA_ATOMS;
-    const int a1 = min(a0 + FA_ATOMS, natoms);
-    const int tid = threadIdx.x;
-    const int m0 = off[a0], m1 = off[a1];
-    // this thread's atom (tid < FA_ATOMS) and its entry range
-    const int k = a0 + tid;
-    const bool own = tid < FA_ATOMS && k < a1;
-    const int mk0 = own ? off[k] : 0, mk1 = own ? off[k + 1] : 0;
-    double fx = 0, fy = 0, fz = 0;
+    __shared__ double red[9][256];
+    const int tid = threadIdx.x, sub = tid & 15;
+    const int64_t n = natoms;
+    const int64_t g0 = (int64_t)xcd_share(blockIdx.x, gridDim.x) * per;
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int c0 = m0; c0 < m1; c0 += FA_CH) {
-        const int c1 = min(c0 + FA_CH, m1);
-        for (int m = c0 + tid; m < c1; m += 256) {
-            const int r = rev[m];
-            const double gx = g[m], gy = g[nnbr + m], gz = g[2 * nnbr + m];
-            dl[0][m - c0] = gx - g[r];
-            dl[1][m - c0] = gy - g[nnbr + r];
-            dl[2][m - c0] = gz - g[2 * nnbr + r];
-            if (vpart) {
-                const double rx = xyz[m], ry = xyz[nnbr + m], rz = xyz[2 * nnbr + m];
-                v[0] -= gx * rx;
-                v[1] -= gx * ry;
-                v[2] -= gx * rz;
-                v[3] -= gy * rx;
-                v[4] -= gy * ry;
-                v[5] -= gy * rz;
-                v[6] -= gz * rx;
-                v[7] -= gz * ry;
-                v[8] -= gz * rz;
-            }
+    for (int64_t q = g0; q < g0 + per; ++q) {
+        const int64_t k = q * FA_ATOMS + (tid >> 4);
+        const int m0 = k < n ? off[k] : 0, m1 = k < n ? off[k + 1] : 0;
+        double f[3] = {0, 0, 0};
+        for (int mb = m0 + sub; mb < m1; mb += 64) {
+            int r[4];
+            double gm[4][3], gr[4][3], x[4][3];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) r[h] = mb + 16 * h < m1 ? rev[mb + 16 * h] : -1;
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    gm[h][d] = gr[h][d] = x[h][d] = 0.0;
+                    if (r[h] >= 0) {
+                        gm[h][d] = g[d * nnbr + mb + 16 * h];
+                        gr[h][d] = g[d * nnbr + r[h]];
+                        if (vpart) x[h][d] = xyz[d * nnbr + mb + 16 * h];
+                    }
+                }
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    f[d] += gm[h][d] - gr[h][d];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) v[3 * d + c] -= gm[h][d] * x[h][c];
+                }
         }
-        __syncthreads();
-        if (own) {
-            const int s0 = max(mk0, c0), s1 = min(mk1, c1);
-            for (int m = s0; m < s1; ++m) {
-                fx += dl[0][m - c0];
-                fy += dl[1][m - c0];
-                fz += dl[2][m - c0];
-            }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+#pragma unroll
+            for (int h = 8; h > 0; h >>= 1) f[d] += __shfl_xor(f[d], h);
         }
-        __syncthreads();
-    }
-    if (own) {
-        F[k] = fx;
-        F[natoms + k] = fy;
-        F[2 * natoms + k] = fz;
+        if (k < n && sub < 3) F[sub * n + k] = sub == 0 ? f[0] : sub == 1 ? f[1] : f[2];
     }
     if (!vpart) return;  // uniform over the block
     for (int c = 0; c < 9; ++c) red[c][tid] = v[c];
@@ -878,9 +872,11 @@ extern "C" int ace_nbrlist_forces(ace_nbrlist* nl, int64_t natoms, const int32_t
         HIP_TRY(hipGetLastError());
         return 0;
     }
-    const int nblk = (n + FA_ATOMS - 1) / FA_ATOMS;
+    const int64_t ngrp = ((int64_t)n + FA_ATOMS - 1) / FA_ATOMS;
+    const int per = (int)((ngrp + FA_BLOCKS - 1) / FA_BLOCKS);
+    const int nblk = (int)((ngrp + per - 1) / per);
     if (virial && nl->vpart.ensure((size_t)nblk * 9)) return -1;
-    hipLaunchKernelGGL(k_nbr_forces, dim3((unsigned)nblk), dim3(256), 0, st, n, env_offsets, rev, nnbr, dE_dr, xyz, F,
+    hipLaunchKernelGGL(k_nbr_forces, dim3((unsigned)nblk), dim3(256), 0, st, n, per, env_offsets, rev, nnbr, dE_dr, xyz, F,
                        virial ? nl->vpart.p : nullptr);
     HIP_TRY(hipGetLastError());
     if (virial) {
