@@ -27,6 +27,7 @@
 #include "host_util.hpp"
 #include "pack_host.hpp"
 #include "pairs_host.hpp"
+#include "slots_host.hpp"
 
 #define ACE_LMAX 10
 #define ACE_NPMAX ((ACE_LMAX + 1) * (ACE_LMAX + 2) / 2)
@@ -259,6 +260,14 @@ struct PairDev {
     DevBuf<int32_t> seq[acehost::PAIR_MAXP + 2];
 };
 
+// A slot program on the device: forces, or energies alone.
+struct SlotDev {
+    acehost::SlotProgram host;
+    DevBuf<uint32_t> hdr, codes;
+    DevBuf<double> coef;
+    DevBuf<int32_t> list_ptr[acehost::SLOT_MAXP + 1], list[acehost::SLOT_MAXP + 1];
+};
+
 struct ForceFlatTab {
     int8_t nrl[ACE_LMAX + 1];  // n bound per l
     int16_t nq;  // number of (l, m, n) entries (their G slots in staging order: ace_ctx::ffq)
@@ -283,6 +292,10 @@ struct ace_ctx {
     int seg_et = 0;
     bool force_interp = false;
     // pair kernel programs (energy + forces, energy only) of bases it takes
+    // slot kernel (class-split bases): programs, and the force kernel's slot table
+    bool slots_ok = false;
+    SlotDev slots[2];
+    DevBuf<int32_t> slot_ptr, slot_list, slot_cls;
     bool pairs_ok = false;
     PairDev pairs[2];
     // rec_dispatch: the record kernel that switches per record (ace_set_kernel
@@ -403,6 +416,7 @@ struct Workspace {
     // [part][npool][estride], P of them (P + 1 for environments from genv_hi on)
     int gparts = 0;
     int64_t genv_hi = 0;
+    bool slots = false;  // the slots of the slot kernel's program
 };
 
 // The context's own buffers (as sized by their last ensure).
@@ -472,6 +486,14 @@ int pairs_create(ace_ctx* ctx, const std::vector<int32_t>& pool);
 int pairs_set_coeffs(ace_ctx* ctx, const std::vector<double>& leaf);
 int launch_pairs(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, bool forces, int P, int64_t nhi,
                  const Workspace& ws, double* E_out);
+// ace_slots.hip: the slot programs at context creation (sets slots_ok), their
+// coefficients, workgroups per tile of 32 environments, and the launch: class
+// values [part][class][re, im][estride] into ws.Epart, with forces G.
+int slots_create(ace_ctx* ctx, const ace_pack* pk);
+int slots_set_coeffs(ace_ctx* ctx, const acehost::Coeffs& cf);
+acehost::SlotShape slot_shape(const ace_ctx* ctx, int64_t nenv, bool forces);
+int launch_slots(ace_ctx* ctx, hipStream_t st, int64_t nenv, int64_t estride, bool forces, const acehost::SlotShape& sh,
+                 const Workspace& ws);
 // ace_pool.hip: A+[k][env] into ws.Aplus (stride estride); with nbr_map
 // also the neighbour -> environment map ws.nbr_env (flat force kernel).
 int launch_pool_any(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* off, const double* xyz,

@@ -49,23 +49,38 @@ __device__ __forceinline__ void gather_g(const int32_t* __restrict__ gslot_ptr,
         g[0] = gp.sum(Gbuf + (int64_t)k * estride + env, env);
         return;
     }
-    for (int s = gslot_ptr[k]; s < gslot_ptr[k + 1]; ++s) {
-        const int slot = gslot_list[s];
-        if (NC > 1 && gcls) {
+    const int s1 = gslot_ptr[k + 1];
+    if (NC > 1 && gcls) {
+        // per class first: two additions per slot, and the slots' reads do not
+        // wait for the class vectors
+        double2 q[3] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
+#pragma unroll 4
+        for (int s = gslot_ptr[k]; s < s1; ++s) {
+            const int slot = gslot_list[s], c = gcls[slot];
             const double2 v = Gbuf[(int64_t)slot * estride + env];
-            const double2* u = cls_u + 3 * gcls[slot];
 #pragma unroll
-            for (int p = 0; p < NC; ++p) {
-                g[p].x += u[p].x * v.x - u[p].y * v.y;
-                g[p].y += u[p].x * v.y + u[p].y * v.x;
+            for (int i = 0; i < 3; ++i) {
+                q[i].x += c == i ? v.x : 0.0;
+                q[i].y += c == i ? v.y : 0.0;
             }
-        } else {
+        }
 #pragma unroll
-            for (int p = 0; p < NC; ++p) {
-                const double2 v = Gbuf[((int64_t)slot * NC + p) * estride + env];
-                g[p].x += v.x;
-                g[p].y += v.y;
+        for (int p = 0; p < NC; ++p)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const double2 u = cls_u[3 * i + p];
+                g[p].x += u.x * q[i].x - u.y * q[i].y;
+                g[p].y += u.x * q[i].y + u.y * q[i].x;
             }
+        return;
+    }
+    for (int s = gslot_ptr[k]; s < s1; ++s) {
+        const int slot = gslot_list[s];
+#pragma unroll
+        for (int p = 0; p < NC; ++p) {
+            const double2 v = Gbuf[((int64_t)slot * NC + p) * estride + env];
+            g[p].x += v.x;
+            g[p].y += v.y;
         }
     }
 }
@@ -229,8 +244,10 @@ struct ForceTab {
     int32_t spstride;                                    // entries per species: NC sum_l (l + 1) nrl[l]
 };
 
+constexpr int FORCE_EPB = 4;
+
 template <int L, int PROP, int NRM>
-__global__ __launch_bounds__(64) void k_force(RadialParams rp, ForceTab ft, int64_t nenv,
+__global__ __launch_bounds__(256) void k_force(RadialParams rp, ForceTab ft, int64_t nenv,
                                                const int32_t* __restrict__ off,
                                                const double* __restrict__ xyz, int64_t nnbr,
                                                const int8_t* __restrict__ species, int nsp,
@@ -243,23 +260,28 @@ __global__ __launch_bounds__(64) void k_force(RadialParams rp, ForceTab ft, int6
                                                double* __restrict__ dE) {
     constexpr int NP = (L + 1) * (L + 2) / 2;
     constexpr int NC = PROP == 0 ? 1 : 3;
-    extern __shared__ double2 Gd[];  // [nsp][spstride]
-    const int lane = threadIdx.x;
-    const int64_t env = xcd_env(blockIdx.x, nenv);
+    // a wave per environment, FORCE_EPB environments (or one) per workgroup: the
+    // tables are filled together, neighbouring environments by neighbouring
+    // threads, since G is stored [slot][environment]
+    extern __shared__ double2 Gall[];  // [environment][nsp][spstride]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, epb = blockDim.x >> 6;
+    const int64_t env0 = xcd_env(blockIdx.x, gridDim.x) * epb, env = env0 + wave;
     const int nr = rp.nr;
-    if (env >= nenv) return;
     const int ntab = nsp * ft.spstride;
-    for (int q = lane; q < ntab; q += 64) Gd[q] = make_double2(0.0, 0.0);
+    for (int q = threadIdx.x; q < epb * ntab; q += blockDim.x) Gall[q] = make_double2(0.0, 0.0);
     __syncthreads();
-    for (int k = lane; k < npool; k += 64) {
+    const int es = threadIdx.x % epb;
+    for (int k = threadIdx.x / epb; k < npool && env0 + es < nenv; k += 64) {
         const int mu = max(0, pool[4 * k]), n = pool[4 * k + 1] - 1, l = pool[4 * k + 2], m = pool[4 * k + 3];
         const int d = mu * ft.spstride + ft.off[idxp(l, m)] + n * NC;
         double2 g[NC];
-        gather_g<NC>(gslot_ptr, gslot_list, gcls, cls_u, Gbuf, estride, env, k, gp, g);
+        gather_g<NC>(gslot_ptr, gslot_list, gcls, cls_u, Gbuf, estride, env0 + es, k, gp, g);
 #pragma unroll
-        for (int p = 0; p < NC; ++p) Gd[d + p] = g[p];
+        for (int p = 0; p < NC; ++p) Gall[es * ntab + d + p] = g[p];
     }
     __syncthreads();
+    if (env >= nenv) return;
+    const double2* const Gd = Gall + wave * ntab;
     const int j0 = off[env], j1 = off[env + 1];
     for (int j = j0 + lane; j < j1; j += 64) {
         const double x = xyz[j], y = xyz[nnbr + j], z = xyz[2 * nnbr + j];
@@ -609,7 +631,9 @@ static void launch_force(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32
         return;
     }
     const int nsp = std::max(1, ctx->nspecies);
-    const int32_t* gcls = ctx->classed ? ctx->gslot_cls.p : nullptr;
+    const int32_t* gcls = ws.slots ? ctx->slot_cls.p : ctx->classed ? ctx->gslot_cls.p : nullptr;
+    const int32_t *gptr = ws.slots ? ctx->slot_ptr.p : ctx->gslot_ptr.p,
+                  *glist = ws.slots ? ctx->slot_list.p : ctx->gslot_list.p;
     // the per-environment table: each (l, m >= 0) holds the n < nrl[l]
     ForceTab ft;
     std::memset(&ft, 0, sizeof(ft));
@@ -624,12 +648,15 @@ static void launch_force(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32
     ft.spstride = ent;
     const size_t table = (size_t)nsp * ent * sizeof(double2);
     if (ctx->nr <= FORCE_NRMAX && table <= 64 * 1024) {
+        // several environments per workgroup where each CU has some workgroups even so
+        const int epb = table * FORCE_EPB <= 64 * 1024 && nenv >= (int64_t)8 * FORCE_EPB * ctx->ncu ? FORCE_EPB : 1;
 #define ACE_FORCE(NRM_)                                                                                          \
     do {                                                                                                          \
-        set_func_lds((const void*)k_force<L, PROP, NRM_>, table);                                                 \
-        hipLaunchKernelGGL((k_force<L, PROP, NRM_>), dim3((unsigned)nenv), dim3(64), table, st, radial_params(ctx), \
+        set_func_lds((const void*)k_force<L, PROP, NRM_>, epb * table);                                           \
+        hipLaunchKernelGGL((k_force<L, PROP, NRM_>), dim3((unsigned)((nenv + epb - 1) / epb)), dim3(64 * epb),      \
+                           epb * table, st, radial_params(ctx),                                                     \
                            ft, nenv, off, xyz, nnbr, ctx->nspecies > 0 ? species : nullptr, nsp, ctx->pool.p,     \
-                           ctx->npool, ctx->gslot_ptr.p, ctx->gslot_list.p, gcls, ctx->cls_u.p, ws.Gbuf, estride, \
+                           ctx->npool, gptr, glist, gcls, ctx->cls_u.p, ws.Gbuf, estride, \
                            gp, dE);                                                                                   \
     } while (0)
         // radial functions held in registers: 12 when they suffice, else 16
@@ -644,7 +671,7 @@ static void launch_force(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32
     set_func_lds((const void*)k_force_lds<L, PROP>, lds);
     hipLaunchKernelGGL((k_force_lds<L, PROP>), dim3((unsigned)nenv), dim3(64), lds, st, radial_params(ctx),
                        nenv, off, xyz, nnbr, ctx->nspecies > 0 ? species : nullptr, ctx->kidx.p,
-                       ctx->npool, ctx->gslot_ptr.p, ctx->gslot_list.p, gcls, ctx->cls_u.p, ws.Gbuf, estride, gp, dE);
+                       ctx->npool, gptr, glist, gcls, ctx->cls_u.p, ws.Gbuf, estride, gp, dE);
 }
 
 }  // namespace

@@ -728,15 +728,15 @@ __global__ __launch_bounds__(1024) void k_dags(DagRecArgs a, const uint32_t* __r
 }
 
 // E = e0 + sum of the parts' energy shares (fixed order: deterministic).
-// Environments from env_hi on belong to tiles with parts + 1 shares.  CPLX:
+// Environments from env_hi on belong to tiles with parts_hi shares.  CPLX:
 // the shares are the class values Q_c, E_p = e0_p + Re sum_c u[c][p] Q_c.
 template <bool CPLX>
-__global__ void k_esum(int64_t nenv, int parts, int64_t env_hi, const double* __restrict__ Ep, int64_t estride,
+__global__ void k_esum(int64_t nenv, int parts, int parts_hi, int64_t env_hi, const double* __restrict__ Ep, int64_t estride,
                        const double* __restrict__ e0p, const double2* __restrict__ cls_u, double* __restrict__ E_out) {
     constexpr int NE = CPLX ? 6 : 1;
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= nenv) return;
-    const int np = e >= env_hi ? parts + 1 : parts;
+    const int np = e >= env_hi ? parts_hi : parts;
     double Q[NE];
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
@@ -841,6 +841,7 @@ static int upload_coeffs(ace_ctx* ctx, const double* c) {
             return -1;
     }
     if (ctx->pairs_ok && pairs_set_coeffs(ctx, cf.leaf)) return -1;
+    if (ctx->slots_ok && slots_set_coeffs(ctx, cf)) return -1;
     if (ctx->task_const.upload(cf.task.data(), cf.task.size())) return -1;
     double ev[3] = {cf.e0[0], cf.e0[2], cf.e0[4]};
     if (ctx->nfeat > 0) {
@@ -1106,6 +1107,7 @@ extern "C" int ace_ctx_create(const ace_pack* pk, int device, const double* c, i
             return fail("upload");
     }
     if (pairs_create(ctx, std::vector<int32_t>(pk->pool, pk->pool + 4 * (size_t)pk->npool))) return fail("pair programs");
+    if (slots_create(ctx, pk)) return fail("slot programs");
     if (upload_coeffs(ctx, c)) return fail("set_params");
     for (auto& e : ctx->ev)
         if (hipEventCreate(&e) != hipSuccess) return fail("event");
@@ -1230,6 +1232,33 @@ static int segment_parts(const ace_ctx* ctx, int64_t ntile, int ntask, int W) {
 static bool use_pairs(const ace_ctx* ctx, int64_t nenv, bool forces) {
     if (!ctx->pairs_ok || ctx->force_interp || ctx->rec_dispatch) return false;
     return ctx->maxorder >= 4 || !forces || (nenv + 31) / 32 <= ctx->ncu;
+}
+
+// Bytes of the slot kernel's G and class values.
+static size_t slot_bytes(const ace_ctx* ctx, int64_t nenv, int P) {
+    const int64_t estride = ((nenv + 63) / 64) * 64;
+    return scratch_up((size_t)ctx->slots[0].host.nslots * estride * sizeof(double2)) +
+           scratch_up((size_t)P * 6 * estride * sizeof(double));
+}
+
+// The slot kernel takes the call: its programs exist and no other kernel or
+// split was asked for.  With forces from order 3 on (degree 10, 110 pooled values,
+// at 40,000 / 8,192 / 64 environments: 0.294 / 0.072 / 0.029 ms against the
+// segment kernel's 0.377 / 0.096 / 0.048, degree 6 0.063 / 0.022 / 0.015 against
+// 0.079 / 0.025 / 0.020; order 2: 0.018 against 0.016 at 8,192).  Energies alone
+// where the segment kernel's tile is narrow (220 pooled values 0.496 / 0.112 /
+// 0.033 against 0.743 / 0.207 / 0.183), else up to one tile per compute unit
+// and for programs that are worth the second launch (110 pooled values
+// 0.148 / 0.037 / 0.021 against 0.126 / 0.042 / 0.043; degree 6 0.036 / 0.015 /
+// 0.014 against 0.031 / 0.013 / 0.013).
+// Batches that fit the allocation-free entry point only where its shares do
+// too, so that both entry points give the same bits.
+static bool use_slots(const ace_ctx* ctx, int64_t nenv, bool forces) {
+    if (!ctx->slots_ok || ctx->force_interp || ctx->rec_dispatch || ctx->parts > 0 || ctx->tail > 0) return false;
+    if (ctx->maxorder < 3) return false;
+    if (!forces && ctx->npool < 160 && ((nenv + 31) / 32 > ctx->ncu || ctx->slots[1].host.load[1] < 30000.0)) return false;
+    return !forces || scratch_need(ctx, nenv, 0).all() > ACE_SCRATCH_BYTES ||
+           slot_bytes(ctx, nenv, acehost::SLOT_MAXP) <= ACE_SHARE_BYTES;
 }
 
 // Workgroups per 32-environment tile of the pair kernel, and tail tiles.
@@ -1530,13 +1559,22 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
         if (pair_shape(ctx, nenv, forces, P, nhi)) return -1;
         if (launch_pairs(ctx, st, nenv, estride, forces, P, nhi, ws, P == 1 ? E_out : ws.Epart)) return -1;
         if (P > 1)
-            hipLaunchKernelGGL(k_esum<false>, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, P,
+            hipLaunchKernelGGL(k_esum<false>, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, P, P + 1,
                                ((nenv + 31) / 32 - nhi) * 32, ws.Epart, estride, ctx->e0v.p, ctx->cls_u.p, E_out);
         ws.gparts = P;
         ws.genv_hi = ((nenv + 31) / 32 - nhi) * 32;
         ctx->last_parts = P;
         ctx->last_tail = nhi;
         ctx->last_kernel = 0;
+    } else if (use_slots(ctx, nenv, forces)) {
+        const acehost::SlotShape sh = slot_shape(ctx, nenv, forces);
+        if (launch_slots(ctx, st, nenv, estride, forces, sh, ws)) return -1;
+        hipLaunchKernelGGL(k_esum<true>, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, sh.P, sh.P_hi,
+                           ((nenv + 31) / 32 - sh.nhi) * 32, ws.Epart, estride, ctx->e0v.p, ctx->cls_u.p, E_out);
+        ws.slots = true;
+        ctx->last_parts = sh.P;
+        ctx->last_tail = sh.nhi;
+        ctx->last_kernel = ctx->seg_et == 64 ? 0 : 1;  // as the segment kernel's tiles
     } else if (use_records) {
         const int ET = rec_et;
         const int NE = ctx->classed ? 6 : 1;
@@ -1590,10 +1628,10 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
         if (P > 1) {
             const dim3 g((unsigned)((nenv + 255) / 256)), b(256);
             if (ctx->classed)
-                hipLaunchKernelGGL(k_esum<true>, g, b, 0, st, nenv, P, (ntile - nhi) * ET, ws.Epart, estride,
+                hipLaunchKernelGGL(k_esum<true>, g, b, 0, st, nenv, P, P + 1, (ntile - nhi) * ET, ws.Epart, estride,
                                    ctx->e0v.p, ctx->cls_u.p, E_out);
             else
-                hipLaunchKernelGGL(k_esum<false>, g, b, 0, st, nenv, P, (ntile - nhi) * ET, ws.Epart, estride,
+                hipLaunchKernelGGL(k_esum<false>, g, b, 0, st, nenv, P, P + 1, (ntile - nhi) * ET, ws.Epart, estride,
                                    ctx->e0v.p, ctx->cls_u.p, E_out);
         }
     } else {
@@ -1624,6 +1662,9 @@ static int run_path(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double
         if (pair_shape(ctx, nenv, forces, P, nhi)) return -1;
         gslots = std::max(gslots, (size_t)(P + (nhi > 0)) * ctx->npool);
         eslots = std::max(eslots, (size_t)(P + (nhi > 0)));
+    } else if (use_slots(ctx, nenv, forces)) {
+        gslots = std::max(gslots, (size_t)ctx->slots[0].host.nslots);
+        eslots = std::max(eslots, (size_t)6 * slot_shape(ctx, nenv, forces).P_hi);
     }
     if (forces && ctx->Gbuf.ensure(gslots * estride)) return -1;
     if ((ctx->seg_et > 0 || ctx->rec_et > 0) && ctx->Epart.ensure(eslots * estride)) return -1;
@@ -1659,6 +1700,11 @@ extern "C" int ace_energy_forces_noalloc(ace_ctx* ctx, int64_t nenv, const int32
         const int n = P + (nhi > 0);
         if (share_bytes(ctx, nenv, n) > ACE_SHARE_BYTES) return set_err("ace_energy_forces_noalloc: shares too large");
         const size_t g = scratch_up((size_t)n * ctx->npool * (((nenv + 63) / 64) * 64) * sizeof(double2));
+        ws.Gbuf = reinterpret_cast<double2*>(ctx->scratch + ACE_SCRATCH_BYTES);
+        ws.Epart = reinterpret_cast<double*>(ctx->scratch + ACE_SCRATCH_BYTES + g);
+    } else if (use_slots(ctx, nenv, true)) {
+        const int64_t estride = ((nenv + 63) / 64) * 64;
+        const size_t g = scratch_up((size_t)ctx->slots[0].host.nslots * estride * sizeof(double2));
         ws.Gbuf = reinterpret_cast<double2*>(ctx->scratch + ACE_SCRATCH_BYTES);
         ws.Epart = reinterpret_cast<double*>(ctx->scratch + ACE_SCRATCH_BYTES + g);
     }

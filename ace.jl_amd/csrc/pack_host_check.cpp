@@ -11,6 +11,7 @@
 #include "nbrlist_host.hpp"
 #include "pack_host.hpp"
 #include "pairs_host.hpp"
+#include "slots_host.hpp"
 
 extern "C" int acehost_validate(const ace_pack* pk, char* msg, int len) {
     std::string e = acehost::validate_pack(pk);
@@ -242,5 +243,77 @@ extern "C" int acehost_bv(const ace_pack* pk, int nchunk, const double* A, const
     }
     for (int n : seen)
         if (n != 1) return -1;
+    return 0;
+}
+
+// A slot program run on the CPU as k_slots runs it, on pooled values A[npool]
+// (re, im) and parameters c, with P workgroups: the class values Q[3], and with
+// forces G[npool][3 classes].  Returns 0, 1 when the basis has no slot form,
+// -1 on a rejected table or when a piece is not run exactly once.
+extern "C" int acehost_slots(const ace_pack* pk, const double* c, int forces, int P, const double* A, double* Q, double* G) {
+    if (!acehost::validate_pack(pk).empty()) return -1;
+    if (!pk->classed) return 1;
+    const acehost::PackCopy pc = acehost::copy_pack(pk);
+    acehost::SlotProgram sp;
+    const std::vector<int32_t> ptr(pk->gslot_ptr, pk->gslot_ptr + pk->npool + 1);
+    if (!acehost::slot_program(pc, std::vector<int32_t>(pk->pool, pk->pool + 4 * (size_t)pk->npool), ptr,
+                               std::vector<int32_t>(pk->gslot_list, pk->gslot_list + ptr.back()),
+                               std::vector<int32_t>(pk->gslot_class, pk->gslot_class + pk->ngslots), forces != 0, sp)
+             .empty())
+        return 1;
+    acehost::slot_coefs(sp, acehost::coefficients(pc, c));
+    typedef std::complex<double> C;
+    constexpr int R = acehost::SLOT_ROWS;
+    auto val = [&](uint32_t w) {
+        const int k = (int)((w & 0x7fffffffu) / 256);
+        const C a = k == pk->npool ? C(1.0) : C(A[2 * k], A[2 * k + 1]);
+        return w >> 31 ? std::conj(a) : a;
+    };
+    std::vector<C> q(3, 0.0), g((size_t)pk->npool * 3, 0.0);
+    std::vector<int> seen((size_t)sp.pieces(), 0);
+    for (int w = 0; w < P * acehost::SLOT_WAVES; ++w)
+        for (int i = sp.list_ptr[P][(size_t)w]; i < sp.list_ptr[P][(size_t)w + 1]; ++i) {
+            const int piece = sp.list[P][(size_t)i];
+            ++seen[(size_t)piece];
+            const uint32_t* hd = sp.hdr.data() + (size_t)acehost::SLOT_HDR * piece;
+            C acc[R] = {}, wt[R] = {};
+            size_t col = 4 * (size_t)hd[0];
+            for (int o = 1; o <= 3; ++o) {
+                for (uint32_t n = 0; n < 4 * hd[o]; ++n, ++col) {
+                    const C y = val(sp.codes[2 * col]) * val(sp.codes[2 * col + 1]);
+                    for (int r = 0; r < R; ++r)
+                        acc[r] += C(sp.coef[2 * (R * col + r)], sp.coef[2 * (R * col + r) + 1]) * y;
+                }
+                for (int r = 0; r < R; ++r) wt[r] += acc[r] * (o == 1 ? 0.5 : o == 2 ? 1.0 / 6.0 : 1.0 / 3.0);
+            }
+            for (int r = 0; r < R; ++r) {
+                if (hd[4 + r] == ~0u) continue;
+                const uint32_t cls = hd[4 + 2 * R + r];
+                q[cls] += val(hd[4 + R + r]) * (forces ? wt[r] : acc[r]);
+                if (forces) g[(size_t)sp.slot_k[hd[4 + r]] * 3 + (size_t)sp.slot_cls[hd[4 + r]]] += acc[r];
+            }
+        }
+    for (int n : seen)
+        if (n != 1) return -1;
+    for (int i = 0; i < 3; ++i) {
+        Q[2 * i] = q[(size_t)i].real();
+        Q[2 * i + 1] = q[(size_t)i].imag();
+    }
+    for (size_t i = 0; forces && i < g.size(); ++i) {
+        G[2 * i] = g[i].real();
+        G[2 * i + 1] = g[i].imag();
+    }
+    return 0;
+}
+
+// The class vectors u[3][3] (re, im) of a class-split pack and the constant
+// term e0[3], for checks against the polynomials.
+extern "C" int acehost_class(const ace_pack* pk, const double* c, double* u, double* e0) {
+    if (!acehost::validate_pack(pk).empty() || !pk->classed) return -1;
+    const acehost::PackCopy pc = acehost::copy_pack(pk);
+    const acehost::Coeffs cf = acehost::coefficients(pc, c);
+    for (int i = 0; i < 3; ++i)
+        for (int q = 0; q < 6; ++q) u[6 * i + q] = pc.cv.u[i][q];
+    for (int q = 0; q < 3; ++q) e0[q] = cf.e0[2 * q];
     return 0;
 }
