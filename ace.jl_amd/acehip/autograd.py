@@ -36,9 +36,19 @@ from .evaluator import EnvBatch, HIPEvaluator
 
 
 def _env_of(offsets: torch.Tensor, nnbr: int) -> torch.Tensor:
-    counts = (offsets[1:] - offsets[:-1]).long()
-    return torch.repeat_interleave(torch.arange(counts.numel(), device=offsets.device), counts,
-                                   output_size=nnbr)
+    """The environment of every neighbour: the ends that lie at or before it."""
+    return torch.bucketize(torch.arange(nnbr, device=offsets.device), offsets[1:].long(), right=True)
+
+
+def _weighted(ev, gE, B):
+    """sum_env gE[env] B[env]: the library's kernel for plain tensors; where a
+    graph is being recorded through gE, or gE is a wrapped one (vmap), torch's."""
+    rows = getattr(ev, "weighted_rows", None)
+    F = torch._C._functorch
+    if (rows is None or (gE.requires_grad and torch.is_grad_enabled()) or F.is_functorch_wrapped_tensor(gE)
+            or F.is_legacy_batchedtensor(gE)):
+        return gE @ B
+    return rows(gE, B)
 
 
 class _Pullback(torch.autograd.Function):
@@ -71,33 +81,59 @@ class _Pullback(torch.autograd.Function):
             if ev.prop != 0:
                 raise NotImplementedError("mixed second derivatives are provided for Invariant bases only")
             adj = ev.adjoint_EVAL_D(b, w)
-            g_c = gE @ adj
+            g_c = _weighted(ev, gE, adj)
         return g_c, g_gE, None, None, None, None
 
 
-class _SiteEnergy(torch.autograd.Function):
-    """Site energies of a batch as a function of (c, xyz)
-    (linearmodel.jl:185-189)."""
+class _OfParams(torch.autograd.Function):
+    """Site energies as a function of c (linearmodel.jl:176-181)."""
 
     @staticmethod
-    def forward(ctx, c, xyz, ev, b):
-        E, dE = ev.energy_forces(b)
+    def forward(ctx, c, E, ev, b):
         ctx.ev, ctx.b = ev, b
-        ctx.save_for_backward(c, dE)
-        return E
+        ctx.save_for_backward(c)
+        return E.view_as(E)
 
     @staticmethod
     def backward(ctx, gE):
-        c, dE = ctx.saved_tensors
-        ev, b = ctx.ev, ctx.b
+        (c,) = ctx.saved_tensors
+        ev = ctx.ev
         gE = gE.contiguous()
-        g_c = g_xyz = None
-        if ctx.needs_input_grad[0]:
-            B = ev.basis_B(b)
-            g_c = gE @ B if ev.prop == 0 else torch.einsum("ep,ekp->k", gE, B)
-        if ctx.needs_input_grad[1]:
-            g_xyz = _Pullback.apply(c, gE, ev, b, dE, _env_of(b.offsets, b.nnbr))
-        return g_c, g_xyz, None, None
+        B = ev.basis_B(ctx.b)
+        return _weighted(ev, gE, B) if ev.prop == 0 else torch.einsum("ep,ekp->k", gE, B), None, None, None
+
+
+class _OfPositions(torch.autograd.Function):
+    """Site energies as a function of xyz.  The pullback is a function of c and
+    gE in turn; c reaches it as the tensor itself (held in ``c_graph``), not as an input, so
+    that a gradient in c does not run this node."""
+
+    @staticmethod
+    def forward(ctx, xyz, c, E, ev, b, dE, c_graph):
+        ctx.ev, ctx.b, ctx.c_graph = ev, b, c_graph
+        ctx.save_for_backward(c, dE)
+        return E.view_as(E)
+
+    @staticmethod
+    def backward(ctx, gE):
+        _, dE = ctx.saved_tensors
+        ev, b = ctx.ev, ctx.b
+        g = _Pullback.apply(ctx.c_graph[0], gE.contiguous(), ev, b, dE, _env_of(b.offsets, b.nnbr))
+        return g, None, None, None, None, None, None
+
+
+class _SiteEnergy(torch.autograd.Function):
+    """The site energies as a function of both (linearmodel.jl:185-189): a node
+    for each, side by side, so that a gradient in one does not evaluate what
+    only the other needs (the basis for c, the pullback for xyz)."""
+
+    @staticmethod
+    def forward(ctx, of_c, of_xyz):
+        return of_c.clone()  # not a view: callers may write to it
+
+    @staticmethod
+    def backward(ctx, gE):
+        return gE, gE
 
 
 def site_energies(ev: HIPEvaluator, c: torch.Tensor, offsets, xyz: torch.Tensor, species=None):
@@ -119,7 +155,9 @@ def site_energies(ev: HIPEvaluator, c: torch.Tensor, offsets, xyz: torch.Tensor,
         ev.set_params(c.detach().cpu().numpy())
         ev._autograd_c = c.detach().clone()
     b = EnvBatch(offsets, xyz.detach(), species, device=xyz.device)
-    return _SiteEnergy.apply(c, xyz, ev, b)
+    E, dE = ev.energy_forces(b)
+    return _SiteEnergy.apply(_OfParams.apply(c, E, ev, b),
+                             _OfPositions.apply(xyz, c.detach(), E, ev, b, dE, (c,)))
 
 
 class SiteEnergy(torch.nn.Module):

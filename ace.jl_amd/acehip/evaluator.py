@@ -235,6 +235,17 @@ class HIPEvaluator:
                                                _vp(w), _vp(out), self._stream(stream)))
         return out
 
+    def weighted_rows(self, w, B, stream=None):
+        """sum_r w[r] B[r] for w (nrow,) and B (nrow, ncol) on the device."""
+        w = w.to(device=B.device, dtype=torch.float64).contiguous()
+        B = B.contiguous()
+        if B.dim() != 2 or B.dtype != torch.float64 or tuple(w.shape) != (B.shape[0],):
+            raise ValueError("w must have one entry per row of the float64 matrix B")
+        out = torch.empty(B.shape[1], dtype=torch.float64, device=B.device)
+        _lib.check(self.lib.ace_weighted_rows(self.ctx, B.shape[0], B.shape[1], _vp(w), _vp(B), _vp(out),
+                                              self._stream(stream)))
+        return out
+
 
 # ---------------------------------------------------------------------------
 # ACE.jl-shaped functional API

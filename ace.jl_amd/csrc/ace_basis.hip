@@ -918,3 +918,57 @@ extern "C" int ace_adjoint_EVAL_D(ace_ctx* ctx, int64_t nenv, const int32_t* off
     HIP_TRY(hipGetLastError());
     return 0;
 }
+
+// out[c] = sum_r w[r] B[r][c]: rows in shares of `per`, a thread per column, then
+// the shares in order.  Bound by reading B once: 2,003 x 3,235, 52 MB, 10 us
+// and the shares 3 (as a matrix product of one row, from a library, 65).
+__global__ __launch_bounds__(256) void k_wrows(int64_t nrow, int64_t ncol, int per, const double* __restrict__ w,
+                                               const double* __restrict__ B, double* __restrict__ part) {
+    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t r0 = (int64_t)blockIdx.y * per, r1 = min(r0 + per, nrow);
+    if (c >= ncol) return;
+    double s = 0.0;
+#pragma unroll 8
+    for (int64_t r = r0; r < r1; ++r) s = fma(w[r], B[r * ncol + c], s);
+    part[(int64_t)blockIdx.y * ncol + c] = s;
+}
+
+__global__ __launch_bounds__(256) void k_wshares(int nshare, int64_t ncol, const double* __restrict__ part,
+                                                 double* __restrict__ out) {
+    __shared__ double red[4][64];
+    const int l = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int64_t c = (int64_t)blockIdx.x * 64 + l;
+    double s = 0.0;
+    if (c < ncol) {
+#pragma unroll 8
+        for (int i = q; i < nshare; i += 4) s += part[(int64_t)i * ncol + c];
+    }
+    red[q][l] = s;
+    __syncthreads();
+    if (q == 0 && c < ncol) out[c] = (red[0][l] + red[1][l]) + (red[2][l] + red[3][l]);
+}
+
+extern "C" int ace_weighted_rows(ace_ctx* ctx, int64_t nrow, int64_t ncol, const double* w, const double* B,
+                                 double* out, void* stream) {
+    if (!ctx) return set_err("null context");
+    if (nrow < 0 || ncol < 0) return set_err("ace_weighted_rows: negative size");
+    if (ncol == 0) return 0;
+    if (!out || (nrow > 0 && (!w || !B))) return set_err("ace_weighted_rows: null argument");
+    HIP_TRY(hipSetDevice(ctx->device));
+    const int64_t gx = (ncol + 255) / 256;
+    if (gx >= ((int64_t)1 << 31)) return set_err("ace_weighted_rows: too many columns");
+    // eight workgroups per compute unit, eight rows each at least
+    const int64_t want = std::max<int64_t>(1, std::min((int64_t)8 * ctx->ncu / gx, (nrow + 7) / 8));
+    const int64_t per = std::max<int64_t>(1, (nrow + want - 1) / want);
+    const int nshare = (int)((nrow + per - 1) / per);
+    if (per >= ((int64_t)1 << 31)) return set_err("ace_weighted_rows: too many rows");
+    if (ctx->wrows.ensure((size_t)std::max(1, nshare) * ncol)) return -1;
+    hipStream_t st = (hipStream_t)stream;
+    if (nshare > 0)
+        hipLaunchKernelGGL(k_wrows, dim3((unsigned)gx, (unsigned)nshare), dim3(256), 0, st, nrow, ncol, (int)per, w, B,
+                           ctx->wrows.p);
+    hipLaunchKernelGGL(k_wshares, dim3((unsigned)((ncol + 63) / 64)), dim3(256), 0, st, nshare, ncol,
+                       (const double*)ctx->wrows.p, out);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}

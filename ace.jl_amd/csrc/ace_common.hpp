@@ -328,6 +328,7 @@ struct ace_ctx {
     DevBuf<BtRec> bt_rec;
     DevBuf<int32_t> bt_rowo;  // [nB][BT_ROWO] record ranges per order
     // Invariant basis values (k_Bv): acehost::BvProgram
+    DevBuf<double> wrows;  // shares of ace_weighted_rows
     DevBuf<acehost::BvRec> bv_rec;
     DevBuf<int32_t> bv_seg, bv_unit;
     double bv_iter = 0, bv_cost = 0;

@@ -332,6 +332,11 @@ int ace_basis_dB(ace_ctx* ctx, int64_t nenv, const int32_t* env_offsets,
 int ace_adjoint_EVAL_D(ace_ctx* ctx, int64_t nenv, const int32_t* env_offsets, const double* xyz,
                        const int8_t* species, const double* w, double* dB_out, void* stream);
 
+/* out[ncol] = sum_r w[r] B[r][ncol] (device, row-major), e.g. the parameter
+ * gradient sum_env gE[env] B[env] from basis values (linearmodel.jl:176-181). */
+int ace_weighted_rows(ace_ctx* ctx, int64_t nrow, int64_t ncol, const double* w, const double* B, double* out,
+                      void* stream);
+
 /* Learned-surrogate support (no reference counterpart; for the surrogate
  * path of a LinearACEModel, see acemlp.h).
  *

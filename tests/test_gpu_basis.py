@@ -33,3 +33,32 @@ def test_basis_values(cuda, args, species, nenv):
     ref = [O.adjoint_EVAL_D(T, None, off[e:e + 2] - off[e], R[off[e]:off[e + 1]], w[off[e]:off[e + 1]],
                             None if sp is None else sp[off[e]:off[e + 1]]) for e in es]
     assert rel_err(D[es], np.stack(ref).reshape(len(es), -1)) < 1e-10
+
+
+@pytest.mark.parametrize("nrow,ncol", [(0, 3), (1, 1), (7, 255), (8, 257), (65, 64), (2003, 97), (50001, 2), (333, 3235)])
+def test_weighted_rows(cuda, nrow, ncol):
+    """Shares of rows and columns past a workgroup's 256; sums of at most 50,001
+    products of numbers of order one in FP64: 1e-12 of the largest possible sum."""
+    print(f"[gpu] weighted rows {nrow} x {ncol}", flush=True)
+    basis, _ = basis_for(1, 4, 2)
+    ev = HIPEvaluator(basis, synth.coefficients(len(basis), 3), device=0)
+    rng = np.random.default_rng(nrow)
+    w, B = rng.uniform(-1, 1, nrow), rng.uniform(-1, 1, (nrow, ncol))
+    got = ev.weighted_rows(torch.as_tensor(w).cuda(), torch.as_tensor(B).cuda()).cpu().numpy()
+    assert got.shape == (ncol,) and np.max(np.abs(got - w @ B)) <= 1e-12 * max(1, nrow)
+
+
+def test_batched_cotangents(cuda):
+    """A batch of cotangents (legacy vmap tensors, which have no storage) takes
+    torch's product, single ones the kernel: the same gradients."""
+    from acehip.autograd import site_energies
+    basis, _ = basis_for(2, 5, 3)
+    c = synth.coefficients(len(basis), 3)
+    ev = HIPEvaluator(basis, c, device=0)
+    off, R, _ = random_batch(5, 8)
+    ct = torch.as_tensor(c, device="cuda").requires_grad_(True)
+    E = site_energies(ev, ct, off, torch.as_tensor(R.T.copy(), device="cuda"))
+    eye = torch.eye(5, dtype=torch.float64, device="cuda")
+    (g,) = torch.autograd.grad(E, ct, eye, is_grads_batched=True, retain_graph=True)
+    one = torch.stack([torch.autograd.grad(E, ct, v, retain_graph=True)[0] for v in eye])
+    assert torch.allclose(g, one, rtol=1e-12, atol=1e-14)
