@@ -477,30 +477,43 @@ __global__ void k_dB(int64_t nnbr, int nB, int nAA, const int32_t* __restrict__ 
 // dB[j][b] = Re sum_k W+[b][k] dphi+[j][k], where W+ collects, for every A2B
 // entry z of row b and factor t of its AA column, the A2B value times the
 // product of the other factors (prefix and suffix products) times the
-// factor's sign, conjugated for conjugated (m < 0) factors, in the slot of
+// factors' signs, conjugated for conjugated (m < 0) factors, in the slot of
 // the factor's pooled function.  One workgroup per (environment, chunk of up
 // to 256 basis functions); thread = basis function.  W+ of the chunk lives in
-// LDS; the neighbours' pooled gradients dphi+ [npool][3] are staged DB_NJ at a
-// time (as many as DB_STAGE double2 hold), the next stage loaded into
-// registers while the current one is used.  The weights are built once per
+// LDS, [slot][lane] per wave; the neighbours' pooled gradients dphi+ [npool][3]
+// are staged DB_NJ at a time (as many as DB_STAGE double2 hold), the next stage
+// loaded into registers while the current one is used.  Bound by the LDS reads of
+// the gradients, three of 16 bytes per slot at each lane's own k (bank
+// conflicts): 108 environments of 42 neighbours, 3,235 functions 481 -> 436 us
+// with merged entries, functions ordered by loop length and stages that are
+// really in flight (97 functions, with all launches 142 -> 101 us).  The weights are built once per
 // workgroup, so a (environment, chunk) pair costs O(A2B entries x order) for
 // the weights and O(neighbours x slots) for the gradients, instead of the
 // dAA[neighbour][AA function] the materialising path writes.
 struct DbArgs {
-    const int32_t* chunk_b;   // [nchunk + 1]
+    const int4* wave;         // [nchunk][4]: first position, functions, first slot, first entry
+    const int32_t* fn;        // [position] basis function
+    const int2* cnt;          // [position] slots, entries
     const int32_t* chunk_s;   // [nchunk + 1]
-    const int32_t* b_slot;    // [nB + 1]
-    const int32_t* slot_k;    // [nslots]
-    const uint4* ztab;        // [nnz][MO / 4]: factor and slot codes per A2B entry
-    const int32_t* rowptr;
-    const double* vals;       // [nnz] or [nnz][6]
+    const int32_t* slot_k;
+    const uint4* ztab;        // [entry][MO / 4]: factor and slot codes
+    const double* vals;       // [entry] or [entry][6]
     int npool, nB;
 };
 
 constexpr int DB_NJ = DB_NJ_MAX;  // neighbours per stage (at most)
 constexpr int DB_STAGE = 2048;    // double2 per stage (8 per thread)
 
-template <int PROP, int MO>
+// A barrier for LDS data alone: __syncthreads also waits for the workgroup's
+// global loads and stores, here the next stage on its way in and the gradients
+// on theirs out, once per neighbour.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <int PROP, int MO, int NPF>
 __global__ __launch_bounds__(256) void k_dBw(DbArgs a, int64_t nenv, const int32_t* __restrict__ off,
                                              const double2* __restrict__ Aplus, int64_t estride,
                                              const double2* __restrict__ dphi, double* __restrict__ dB) {
@@ -509,8 +522,7 @@ __global__ __launch_bounds__(256) void k_dBw(DbArgs a, int64_t nenv, const int32
     const int64_t env = blockIdx.x;
     const int c = blockIdx.y;
     const int tid = threadIdx.x;
-    const int b0 = a.chunk_b[c], b1 = a.chunk_b[c + 1], s0 = a.chunk_s[c], s1 = a.chunk_s[c + 1];
-    const int ns = s1 - s0;
+    const int s0 = a.chunk_s[c], ns = a.chunk_s[c + 1] - s0;
     const int nq = 3 * a.npool;                           // double2 per neighbour
     const int njs = max(1, min(DB_NJ, DB_STAGE / nq));     // neighbours per stage
     double2* As = sm;                       // [npool]
@@ -524,87 +536,83 @@ __global__ __launch_bounds__(256) void k_dBw(DbArgs a, int64_t nenv, const int32
         for (int p = 0; p < NC; ++p) W[q * NC + p] = make_double2(0.0, 0.0);
     }
     __syncthreads();
-    const int b = b0 + tid;
-    const bool active = b < b1;
-    const int sb = active ? a.b_slot[b] - s0 : 0;
-    const int nsb = active ? a.b_slot[b + 1] - a.b_slot[b] : 0;
-    if (active) {
-        for (int z = a.rowptr[b]; z < a.rowptr[b + 1]; ++z) {
-            uint32_t code[MO];
+    const int4 wv = a.wave[4 * c + (tid >> 6)];
+    const int lane = tid & 63, lanes = wv.y;
+    const bool active = lane < lanes;
+    const int2 n = active ? a.cnt[wv.x + lane] : make_int2(0, 0);
+    const int b = active ? a.fn[wv.x + lane] : 0;
+    const int sb = wv.z + lane;  // slot q of this function: sb + q lanes
+    const int nsb = n.x;
+    for (int z = 0; z < n.y; ++z) {
+        const size_t e = (size_t)wv.w + (size_t)z * lanes + lane;
+        uint32_t code[MO];
 #pragma unroll
-            for (int h = 0; h < MO / 4; ++h) {
-                const uint4 w4 = a.ztab[(size_t)z * (MO / 4) + h];
-                code[4 * h] = w4.x;
-                code[4 * h + 1] = w4.y;
-                code[4 * h + 2] = w4.z;
-                code[4 * h + 3] = w4.w;
+        for (int h = 0; h < MO / 4; ++h) {
+            const uint4 w4 = a.ztab[e * (MO / 4) + h];
+            code[4 * h] = w4.x;
+            code[4 * h + 1] = w4.y;
+            code[4 * h + 2] = w4.z;
+            code[4 * h + 3] = w4.w;
+        }
+        double2 f[MO];
+#pragma unroll
+        for (int q = 0; q < MO; ++q) {
+            f[q] = make_double2(1.0, 0.0);
+            if (code[q] & (1u << 13)) {
+                f[q] = As[code[q] & 0x3ffu];
+                if (code[q] & 0x8000u) f[q].y = -f[q].y;
             }
-            if (!(code[0] & (1u << 13))) continue;  // order 0: no gradient
-            double2 f[MO];
-            double sg[MO];
+        }
+        double2 pre[MO];
+        pre[0] = make_double2(1.0, 0.0);
 #pragma unroll
-            for (int q = 0; q < MO; ++q) {
-                f[q] = make_double2(1.0, 0.0);
-                sg[q] = 1.0;
-                if (code[q] & (1u << 13)) {
-                    double2 v = As[code[q] & 0x3ffu];
-                    if (code[q] & 0x8000u) v.y = -v.y;
-                    sg[q] = (code[q] & 0x4000u) ? -1.0 : 1.0;
-                    f[q] = make_double2(sg[q] * v.x, sg[q] * v.y);
-                }
-            }
-            double2 pre[MO];
-            pre[0] = make_double2(1.0, 0.0);
+        for (int q = 1; q < MO; ++q) pre[q] = cmul(pre[q - 1], f[q - 1]);
+        double2 suf = make_double2(1.0, 0.0);
 #pragma unroll
-            for (int q = 1; q < MO; ++q) pre[q] = cmul(pre[q - 1], f[q - 1]);
-            double2 suf = make_double2(1.0, 0.0);
+        for (int t = MO - 1; t >= 0; --t) {
+            if (code[t] & (1u << 13)) {
+                const double2 P = cmul(pre[t], suf);
+                const uint32_t sc = code[t] >> 16;
+                const bool cj = (sc & 0x8000u) != 0;
+                double2* w = W + (size_t)(sb + (int)(sc & 0x7fffu) * lanes) * NC;
 #pragma unroll
-            for (int t = MO - 1; t >= 0; --t) {
-                if (code[t] & (1u << 13)) {
-                    const double2 P = cmul(pre[t], suf);
-                    const uint32_t sc = code[t] >> 16;
-                    const bool cj = (sc & 0x8000u) != 0;
-                    double2* w = W + (size_t)(sb + (int)(sc & 0x7fffu)) * NC;
-#pragma unroll
-                    for (int p = 0; p < NC; ++p) {
-                        double2 v;
-                        if (PROP == 0) {
-                            const double cv = a.vals[z] * sg[t];
-                            v = make_double2(cv * P.x, cv * P.y);
-                        } else {
-                            const double2 cv = make_double2(a.vals[6 * z + 2 * p] * sg[t], a.vals[6 * z + 2 * p + 1] * sg[t]);
-                            v = cmul(cv, P);
-                        }
-                        w[p].x += v.x;
-                        w[p].y += cj ? -v.y : v.y;
+                for (int p = 0; p < NC; ++p) {
+                    double2 v;
+                    if (PROP == 0) {
+                        const double cv = a.vals[e];
+                        v = make_double2(cv * P.x, cv * P.y);
+                    } else {
+                        const double2 cv = make_double2(a.vals[6 * e + 2 * p], a.vals[6 * e + 2 * p + 1]);
+                        v = cmul(cv, P);
                     }
-                    suf = cmul(suf, f[t]);
+                    w[p].x += v.x;
+                    w[p].y += cj ? -v.y : v.y;
                 }
+                suf = cmul(suf, f[t]);
             }
         }
     }
     __syncthreads();
     const int j0 = off[env], j1 = off[env + 1];
-    // stages of njs neighbours: their dphi+ rows are consecutive in memory
-    double2 pf[DB_STAGE / 256];
+    // stages of njs neighbours: their dphi+ rows are consecutive in memory, NPF
+    // values per thread (unconditional loads: a branch around each made the
+    // thread wait for it, and for the stores before it, at once)
+    double2 pf[NPF];
     auto fetch = [&](int jb) {
-        const int n = min(njs, j1 - jb) * nq;
+        const int last = min(njs, j1 - jb) * nq - 1;
         const double2* src = dphi + (int64_t)jb * nq;
 #pragma unroll
-        for (int r = 0; r < DB_STAGE / 256; ++r) {
-            const int q = tid + 256 * r;
-            if (q < n) pf[r] = src[q];
-        }
+        for (int r = 0; r < NPF; ++r) pf[r] = src[min(tid + 256 * r, last)];
     };
     if (j0 < j1) fetch(j0);
     for (int jb = j0; jb < j1; jb += njs) {
         const int nj = min(njs, j1 - jb);
 #pragma unroll
-        for (int r = 0; r < DB_STAGE / 256; ++r) {
+        for (int r = 0; r < NPF; ++r) {
             const int q = tid + 256 * r;
             if (q < nj * nq) dp[q] = pf[r];
         }
-        __syncthreads();
+        lds_barrier();
         if (jb + njs < j1) fetch(jb + njs);  // in flight while this stage is used
         if (active) {
             for (int jj = 0; jj < nj; ++jj) {
@@ -613,11 +621,11 @@ __global__ __launch_bounds__(256) void k_dBw(DbArgs a, int64_t nenv, const int32
 #pragma unroll
                 for (int p = 0; p < NC; ++p) acc[p][0] = acc[p][1] = acc[p][2] = 0.0;
                 for (int q = 0; q < nsb; ++q) {
-                    const int k = sk[sb + q];
+                    const int k = sk[sb + q * lanes];
                     const double2 x0 = d[3 * k], x1 = d[3 * k + 1], x2 = d[3 * k + 2];
 #pragma unroll
                     for (int p = 0; p < NC; ++p) {
-                        const double2 w = W[(size_t)(sb + q) * NC + p];
+                        const double2 w = W[(size_t)(sb + q * lanes) * NC + p];
                         acc[p][0] += w.x * x0.x - w.y * x0.y;
                         acc[p][1] += w.x * x1.x - w.y * x1.y;
                         acc[p][2] += w.x * x2.x - w.y * x2.y;
@@ -632,7 +640,7 @@ __global__ __launch_bounds__(256) void k_dBw(DbArgs a, int64_t nenv, const int32
                 }
             }
         }
-        __syncthreads();
+        lds_barrier();
     }
 }
 
@@ -807,13 +815,14 @@ static int basis_dB_weights(ace_ctx* ctx, hipStream_t st, int64_t nenv, const in
         // no empty uploads (a basis without A2B entries)
         if (t.slot_k.empty()) t.slot_k.push_back(0);
         if (t.ztab.size() < 4) t.ztab.resize(4, 0u);
-        if (ctx->db_chunk_b.upload(t.chunk_b.data(), t.chunk_b.size()) ||
+        if (t.vals.empty()) t.vals.push_back(0.0);
+        if (ctx->db_wave.upload(t.wave.data(), t.wave.size()) || ctx->db_fn.upload(t.fn.data(), t.fn.size()) ||
+            ctx->db_cnt.upload(t.cnt.data(), t.cnt.size()) ||
             ctx->db_chunk_s.upload(t.chunk_s.data(), t.chunk_s.size()) ||
-            ctx->db_b_slot.upload(t.b_slot.data(), t.b_slot.size()) ||
             ctx->db_slot_k.upload(t.slot_k.data(), t.slot_k.size()) ||
-            ctx->db_ztab.upload(t.ztab.data(), t.ztab.size()))
+            ctx->db_ztab.upload(t.ztab.data(), t.ztab.size()) || ctx->db_vals.upload(t.vals.data(), t.vals.size()))
             return -1;
-        ctx->db_nchunk = (int)t.chunk_b.size() - 1;
+        ctx->db_nchunk = t.nchunk();
         ctx->db_max_slots = t.max_chunk_slots;
         ctx->db_ready = true;
     }
@@ -827,13 +836,13 @@ static int basis_dB_weights(ace_ctx* ctx, hipStream_t st, int64_t nenv, const in
     DISPATCH_L(ctx->L, launch_dphi_pool, ctx, st, nnbr, xyz, species);
     HIP_TRY(hipGetLastError());
     DbArgs a;
-    a.chunk_b = ctx->db_chunk_b.p;
+    a.wave = reinterpret_cast<const int4*>(ctx->db_wave.p);
+    a.fn = ctx->db_fn.p;
+    a.cnt = reinterpret_cast<const int2*>(ctx->db_cnt.p);
     a.chunk_s = ctx->db_chunk_s.p;
-    a.b_slot = ctx->db_b_slot.p;
     a.slot_k = ctx->db_slot_k.p;
     a.ztab = reinterpret_cast<const uint4*>(ctx->db_ztab.p);
-    a.rowptr = ctx->rowptr.p;
-    a.vals = ctx->vals.p;
+    a.vals = ctx->db_vals.p;
     a.npool = ctx->npool;
     a.nB = ctx->nB;
     if (ctx->db_nchunk == 0) return 0;  // no basis functions
@@ -844,10 +853,23 @@ static int basis_dB_weights(ace_ctx* ctx, hipStream_t st, int64_t nenv, const in
         hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, a, nenv, off, ctx->Aplus.p, estride, ctx->dphi.p, dB_out);
     };
     const bool wide = ctx->db_host.zw == 8;
-    if (ctx->prop == ACE_PROP_INVARIANT)
-        wide ? go(k_dBw<0, 8>) : go(k_dBw<0, 4>);
+    // values per thread of a stage
+    const int nq = 3 * ctx->npool, npf = (std::max(1, std::min(DB_NJ, DB_STAGE / nq)) * nq + 255) / 256;
+    auto stage = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        if (ctx->prop == ACE_PROP_INVARIANT)
+            wide ? go(k_dBw<0, 8, N>) : go(k_dBw<0, 4, N>);
+        else
+            wide ? go(k_dBw<1, 8, N>) : go(k_dBw<1, 4, N>);
+    };
+    if (npf <= 1)
+        stage(std::integral_constant<int, 1>());
+    else if (npf <= 2)
+        stage(std::integral_constant<int, 2>());
+    else if (npf <= 4)
+        stage(std::integral_constant<int, 4>());
     else
-        wide ? go(k_dBw<1, 8>) : go(k_dBw<1, 4>);
+        stage(std::integral_constant<int, DB_STAGE / 256>());
     HIP_TRY(hipGetLastError());
     return 0;
 }

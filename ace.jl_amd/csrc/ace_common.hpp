@@ -171,11 +171,12 @@ __device__ __forceinline__ int64_t xcd_env(int64_t b, int64_t n) {
 
 constexpr int POOL_CH = 16;
 // LDS of the basis-gradient weight kernel (k_dBw), and neighbours staged per
-// barrier: measured at config 2, one neighbour per stage within 48 KB (three
-// workgroups per CU) beat 2 or 4 neighbours per stage (fewer functions per
-// chunk, fewer workgroups per CU) and a 32 KB budget
+// barrier: three workgroups per CU; with two neighbours per stage (a slot's
+// weight read once for both) 108 environments of 42 neighbours, 3,235 functions
+// took 562 us against 481, fewer functions per chunk and no fewer LDS reads of
+// the gradients
 constexpr int DB_NJ_MAX = 1;
-constexpr size_t DB_LDS_BUDGET = 48 * 1024;
+constexpr size_t DB_LDS_BUDGET = 53 * 1024;
 // k_dBw's LDS besides the weights: A+ [npool] and a stage of up to DB_NJ_MAX
 // neighbours' dphi+ [npool][3] within 2048 double2 (at least one neighbour)
 inline size_t db_fixed_lds(int npool) {
@@ -316,7 +317,8 @@ struct ace_ctx {
     acehost::DbTables db_host;
     bool db_usable = false, db_ready = false;
     int db_nchunk = 0, db_max_slots = 0;
-    DevBuf<int32_t> db_chunk_b, db_chunk_s, db_b_slot, db_slot_k;
+    DevBuf<int32_t> db_wave, db_fn, db_cnt, db_chunk_s, db_slot_k;
+    DevBuf<double> db_vals;
     DevBuf<uint32_t> db_ztab;
     DevBuf<double2> cls_u;        // [3 classes][3 components]
     DevBuf<int32_t> gslot_cls;    // [ngslots] class of every G slot

@@ -1066,7 +1066,7 @@ extern "C" int ace_ctx_create(const ace_pack* pk, int device, const double* c, i
         const size_t per_slot = (size_t)NC * sizeof(double2) + sizeof(int32_t);
         if (fixed + 64 * per_slot <= DB_LDS_BUDGET) {
             const int max_slots = (int)((DB_LDS_BUDGET - fixed) / per_slot);
-            ctx->db_host = acehost::db_tables(pk, 256, max_slots);
+            ctx->db_host = acehost::db_tables(pk, max_slots);
             ctx->db_usable = ctx->db_host.max_chunk_slots <= max_slots;
         }
     }

@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <map>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -602,60 +603,138 @@ inline void lpt_lists(const PackCopy& p, const std::vector<int>& tasks, int V, s
 // the product of the other factors times the A2B value goes to the slot of
 // pooled function k(iA_t) in b's slot list, conjugated when iA_t is a
 // conjugated (m < 0) function.
-//   b_slot[nB + 1]      CSR of slots per basis function
-//   slot_k[nslots]      pooled function of a slot
-//   ztab[nnz][zw]       per A2B entry, one word per factor t < zw (zw = 4
-//                       for correlation order <= 4, else 8): low half the
-//                       factor (pooled k in bits 0-9, bit 13 present, bit 14
-//                       negative sign, bit 15 conjugated), high half the slot
-//                       index within b's list (bits 0-14) | conjugated << 15
-//   chunk_b[nchunk + 1], chunk_s[nchunk + 1]: basis-function chunks of at
-//   most max_b functions and max_slots slots (one workgroup each)
+// Entries of one row with equal or mirrored monomials (every factor conjugated)
+// give the same gradient, so Invariant rows merge them; the factors' signs go
+// into the value.  A thread of the kernel has one basis function, a wave up to
+// 64: within 256 consecutive functions they are ordered by their slots and
+// entries, so that a wave's lanes have loops of about one length, and a wave's
+// tables are [slot or entry][lane].
+//   wave[chunk][4][4]   per wave: first position, functions, first slot in the
+//                       chunk, first entry
+//   fn[position], cnt[position][2]   basis function; its slots and entries
+//   chunk_s[nchunk + 1], slot_k      pooled function per slot, chunk after chunk
+//   ztab[entry][zw]     one word per factor t < zw (zw = 4 for correlation
+//                       order <= 4, else 8): low half the factor (pooled k in
+//                       bits 0-9, bit 13 present, bit 15 conjugated), high half
+//                       the function's slot (bits 0-14) | conjugated << 15
+//   vals[entry]         or [entry][6] (EuclideanVector)
+// A chunk has at most four waves and max_slots slots (one workgroup each).
 struct DbTables {
-    std::vector<int32_t> b_slot, slot_k, chunk_b, chunk_s;
+    std::vector<int32_t> wave, fn, cnt, chunk_s, slot_k;
     std::vector<uint32_t> ztab;
+    std::vector<double> vals;
     int zw = 4;
     int max_chunk_slots = 0;
+    int nchunk() const { return (int)chunk_s.size() - 1; }
 };
 
-inline DbTables db_tables(const ace_pack* pk, int max_b, int max_slots) {
+inline DbTables db_tables(const ace_pack* pk, int max_slots) {
     DbTables t;
-    const int mo = pk->maxorder;
+    const int mo = pk->maxorder, nc = pk->prop == ACE_PROP_INVARIANT ? 1 : 6;
     t.zw = mo <= 4 ? 4 : 8;
-    t.b_slot.assign((size_t)pk->nB + 1, 0);
-    t.ztab.assign((size_t)pk->a2b_nnz * t.zw, 0u);
-    std::vector<int> where((size_t)pk->npool, -1);
+    struct Entry {
+        std::vector<uint16_t> f;
+        double v[6];
+    };
+    std::vector<std::vector<Entry>> rows((size_t)pk->nB);
+    std::vector<std::vector<int32_t>> ks((size_t)pk->nB);
     for (int b = 0; b < pk->nB; ++b) {
-        const int s0 = (int)t.slot_k.size();
+        std::map<std::vector<uint16_t>, size_t> at;
         for (int z = pk->a2b_rowptr[b]; z < pk->a2b_rowptr[b + 1]; ++z) {
             const int col = pk->a2b_cols[z];
+            if (pk->orders[col] == 0) continue;  // no gradient
+            Entry e;
+            double sg = 1.0;
             for (int q = 0; q < pk->orders[col]; ++q) {
                 const int iA = pk->iAA2iA[(size_t)col * mo + q];
-                const int f = pk->aspec_fid[iA];
-                const int k = f & 0x7fff;
-                if (where[(size_t)k] < 0) {
-                    where[(size_t)k] = (int)t.slot_k.size() - s0;
-                    t.slot_k.push_back(k);
-                }
-                const uint32_t cj = (f & 0x8000) ? 1u : 0u;
-                const uint32_t fc = (uint32_t)k | (1u << 13) | (pk->aspec_sgn[iA] < 0 ? 1u << 14 : 0u) | (cj << 15);
-                const uint32_t sc = (uint32_t)where[(size_t)k] | (cj << 15);
-                t.ztab[(size_t)z * t.zw + q] = fc | (sc << 16);
+                e.f.push_back((uint16_t)pk->aspec_fid[iA]);
+                sg *= pk->aspec_sgn[iA];
+                const int32_t k = pk->aspec_fid[iA] & 0x7fff;
+                if (std::find(ks[(size_t)b].begin(), ks[(size_t)b].end(), k) == ks[(size_t)b].end())
+                    ks[(size_t)b].push_back(k);
             }
+            for (int q = 0; q < nc; ++q) e.v[q] = sg * pk->a2b_vals[(size_t)z * nc + q];
+            if (nc == 1) {
+                std::vector<uint16_t> x = e.f, y = e.f;
+                for (size_t q = 0; q < x.size(); ++q) {
+                    const bool real = pk->pool[4 * (x[q] & 0x7fff) + 3] == 0;
+                    x[q] = (uint16_t)(real ? x[q] & 0x7fff : x[q]);
+                    y[q] = (uint16_t)(real ? x[q] : x[q] ^ 0x8000);
+                }
+                std::sort(x.begin(), x.end());
+                std::sort(y.begin(), y.end());
+                const auto it = at.emplace(std::min(x, y), rows[(size_t)b].size());
+                if (!it.second) {
+                    rows[(size_t)b][it.first->second].v[0] += e.v[0];
+                    continue;
+                }
+            }
+            rows[(size_t)b].push_back(e);
         }
-        for (size_t i = (size_t)s0; i < t.slot_k.size(); ++i) where[(size_t)t.slot_k[i]] = -1;
-        t.b_slot[(size_t)b + 1] = (int32_t)t.slot_k.size();
     }
-    t.chunk_b.push_back(0);
+    for (int b = 0; b < pk->nB; ++b) t.fn.push_back(b);
+    for (int b = 0; b < pk->nB; b += 256)
+        std::stable_sort(t.fn.begin() + b, t.fn.begin() + std::min(b + 256, (int)pk->nB), [&](int x, int y) {
+            const size_t sx = ks[(size_t)x].size(), sy = ks[(size_t)y].size();
+            return sx != sy ? sx < sy : rows[(size_t)x].size() < rows[(size_t)y].size();
+        });
+    for (int b : t.fn) {
+        t.cnt.push_back((int32_t)ks[(size_t)b].size());
+        t.cnt.push_back((int32_t)rows[(size_t)b].size());
+    }
     t.chunk_s.push_back(0);
-    for (int b = 0; b < pk->nB;) {
-        int e = b;
-        while (e < pk->nB && e - b < max_b && t.b_slot[(size_t)e + 1] - t.b_slot[(size_t)b] <= max_slots) ++e;
-        if (e == b) e = b + 1;  // one function above the slot budget: a chunk of its own
-        t.max_chunk_slots = std::max(t.max_chunk_slots, t.b_slot[(size_t)e] - t.b_slot[(size_t)b]);
-        t.chunk_b.push_back(e);
-        t.chunk_s.push_back(t.b_slot[(size_t)e]);
-        b = e;
+    int pos = 0, used = 0;
+    int64_t entries = 0;
+    while (pos < pk->nB) {
+        // the next wave: 64 functions, or as many as the slots allow (one at least)
+        int lanes = std::min(64, pk->nB - pos), ns = 0, nz = 0;
+        for (;; lanes /= 2) {
+            ns = nz = 0;
+            for (int i = 0; i < lanes; ++i) {
+                ns = std::max(ns, t.cnt[2 * (size_t)(pos + i)]);
+                nz = std::max(nz, t.cnt[2 * (size_t)(pos + i) + 1]);
+            }
+            if (lanes == 1 || ns * lanes <= max_slots) break;
+        }
+        const bool fresh = t.wave.size() % 16 == 0;
+        if (!fresh && used + ns * lanes > max_slots) {
+            while (t.wave.size() % 16) t.wave.push_back(0);  // close the chunk
+            continue;
+        }
+        if (fresh) {
+            if (!t.wave.empty()) t.chunk_s.push_back((int32_t)t.slot_k.size());
+            used = 0;
+        }
+        for (int v : {pos, lanes, used, (int)entries}) t.wave.push_back(v);
+        for (int q = 0; q < ns; ++q)
+            for (int i = 0; i < lanes; ++i) {
+                const auto& k = ks[(size_t)t.fn[(size_t)(pos + i)]];
+                t.slot_k.push_back(q < (int)k.size() ? k[(size_t)q] : 0);
+            }
+        for (int z = 0; z < nz; ++z)
+            for (int i = 0; i < lanes; ++i) {
+                const size_t b = (size_t)t.fn[(size_t)(pos + i)];
+                const bool in = z < (int)rows[b].size();
+                for (int q = 0; q < t.zw; ++q) {
+                    uint32_t w = 0;
+                    if (in && q < (int)rows[b][(size_t)z].f.size()) {
+                        const uint32_t f = rows[b][(size_t)z].f[(size_t)q];
+                        const auto it = std::find(ks[b].begin(), ks[b].end(), (int32_t)(f & 0x7fff));
+                        w = (f & 0x7fff) | (1u << 13) | (f & 0x8000) |
+                            ((uint32_t)(it - ks[b].begin()) | (f & 0x8000)) << 16;
+                    }
+                    t.ztab.push_back(w);
+                }
+                for (int q = 0; q < nc; ++q) t.vals.push_back(in ? rows[b][(size_t)z].v[q] : 0.0);
+            }
+        entries += (int64_t)nz * lanes;
+        used += ns * lanes;
+        t.max_chunk_slots = std::max(t.max_chunk_slots, used);
+        pos += lanes;
+    }
+    if (pk->nB > 0) {
+        while (t.wave.size() % 16) t.wave.push_back(0);
+        t.chunk_s.push_back((int32_t)t.slot_k.size());
     }
     return t;
 }

@@ -62,3 +62,20 @@ def test_batched_cotangents(cuda):
     (g,) = torch.autograd.grad(E, ct, eye, is_grads_batched=True, retain_graph=True)
     one = torch.stack([torch.autograd.grad(E, ct, v, retain_graph=True)[0] for v in eye])
     assert torch.allclose(g, one, rtol=1e-12, atol=1e-14)
+
+
+@pytest.mark.parametrize("args,kw", [((1, 4, 2), {}), ((3, 6, 4), {}), ((4, 8, 4), {}), ((5, 5, 3), {}),
+                                     ((3, 5, 3), {"prop": "EuclideanVector", "species": 2})])
+def test_basis_gradients(cuda, args, kw):
+    """Basis gradients by adjoint weights: fewer functions than a wave and several
+    windows of 256, entries of four and of eight factors, merged (Invariant) and
+    not (vector); against the oracle (1e-10 of the largest value)."""
+    print(f"[gpu] basis gradients {args} {kw}", flush=True)
+    basis, T = basis_for(*args, **kw)
+    off, R, sp = random_batch(5, 3, nspecies=kw.get("species", 0))
+    ev = HIPEvaluator(basis, synth.coefficients(len(basis), 3), device=0)
+    dB = ev.basis_dB(EnvBatch(off, R.T.copy(), sp, device="cuda:0")).cpu().numpy()
+    _, dAA = O.eval_AA_dAA(T, off, R, sp)
+    ref = O.eval_dB(T, dAA)
+    assert dB.size == ref.size
+    assert rel_err(dB.reshape(ref.shape), ref) < 1e-10
