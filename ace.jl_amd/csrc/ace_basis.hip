@@ -64,13 +64,16 @@ __global__ void k_B(int64_t nenv, int nB, int nAA, const int32_t* __restrict__ r
     for (int p = 0; p < NC; ++p) B[i * NC + p] = s[p];
 }
 
-// per-neighbour 1p gradients dphi[j][iA][3] (complex), product_1pbasis.jl:169-221
+// per-neighbour 1p gradients dphi[j][iA][3] (complex), product_1pbasis.jl:169-221:
+// a thread per neighbour, blockIdx.y a share of `per` functions.  A thread's
+// functions follow one another, so a small batch is bound by that chain and is split
+// further: 4,536 neighbours, 139 functions 99 us in 71 waves, 25 in 1,278.
 template <int L>
 __global__ __launch_bounds__(64) void k_dphi(RadialParams rp, int64_t nnbr,
                                              const int32_t* __restrict__ nbr_env,
                                              const double* __restrict__ xyz,
                                              const int8_t* __restrict__ species,
-                                             const int32_t* __restrict__ aspec4, int nA,
+                                             const int32_t* __restrict__ aspec4, int nA, int per,
                                              double2* __restrict__ dphi) {
     constexpr int NP = (L + 1) * (L + 2) / 2;
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -97,7 +100,8 @@ __global__ __launch_bounds__(64) void k_dphi(RadialParams rp, int64_t nnbr,
     alp_eval_ed<L>(rp, S, P, dP);
     const double rinv = 1.0 / (S.r + 2.220446049250313e-16);
     const double rh[3] = {x / S.r, y / S.r, z / S.r};
-    for (int iA = 0; iA < nA; ++iA) {
+    const int i1 = min(nA, ((int)blockIdx.y + 1) * per);
+    for (int iA = blockIdx.y * per; iA < i1; ++iA) {
         const int amu = aspec4[4 * iA], n = aspec4[4 * iA + 1] - 1, l = aspec4[4 * iA + 2],
                   mm = aspec4[4 * iA + 3];
         double2* out = dphi + (j * nA + iA) * 3;
@@ -784,21 +788,17 @@ extern "C" int ace_basis_B(ace_ctx* ctx, int64_t nenv, const int32_t* off, const
     return 0;
 }
 
+// rows: (mu, n, l, m) of each function, all of them (aspec4) or the pooled ones
 template <int L>
-static void launch_dphi(ace_ctx* ctx, hipStream_t st, int64_t nnbr, const double* xyz,
-                        const int8_t* species) {
-    hipLaunchKernelGGL(k_dphi<L>, dim3((unsigned)((nnbr + 63) / 64)), dim3(64), 0, st, radial_params(ctx),
-                       nnbr, ctx->nbr_env.p, xyz, ctx->nspecies > 0 ? species : nullptr, ctx->aspec4.p,
-                       ctx->nA, ctx->dphi.p);
-}
-
-template <int L>
-static void launch_dphi_pool(ace_ctx* ctx, hipStream_t st, int64_t nnbr, const double* xyz,
-                             const int8_t* species) {
-    // the pooled (m >= 0) functions: pool rows are (mu, n, l, m) like aspec rows
-    hipLaunchKernelGGL(k_dphi<L>, dim3((unsigned)((nnbr + 63) / 64)), dim3(64), 0, st, radial_params(ctx),
-                       nnbr, ctx->nbr_env.p, xyz, ctx->nspecies > 0 ? species : nullptr, ctx->pool.p,
-                       ctx->npool, ctx->dphi.p);
+static void launch_dphi(ace_ctx* ctx, hipStream_t st, int64_t nnbr, const double* xyz, const int8_t* species,
+                        const int32_t* rows, int n) {
+    const int64_t nblk = (nnbr + 63) / 64;
+    // shares of eight functions or more, while there are fewer than eight waves per compute unit
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>((n + 7) / 8, 8 * ctx->ncu / nblk));
+    const int per = (int)((n + want - 1) / want);
+    hipLaunchKernelGGL(k_dphi<L>, dim3((unsigned)nblk, (unsigned)((n + per - 1) / per)), dim3(64), 0, st,
+                       radial_params(ctx), nnbr, ctx->nbr_env.p, xyz, ctx->nspecies > 0 ? species : nullptr, rows, n,
+                       per, ctx->dphi.p);
 }
 
 // Basis gradients through per-environment adjoint weights (k_dBw): 0, or 1
@@ -833,7 +833,8 @@ static int basis_dB_weights(ace_ctx* ctx, hipStream_t st, int64_t nenv, const in
     if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false)) return -1;
     hipLaunchKernelGGL(k_nbr_env, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, off,
                        ctx->nbr_env.p);
-    DISPATCH_L(ctx->L, launch_dphi_pool, ctx, st, nnbr, xyz, species);
+    // the pooled (m >= 0) functions: pool rows are (mu, n, l, m) like aspec rows
+    DISPATCH_L(ctx->L, launch_dphi, ctx, st, nnbr, xyz, species, ctx->pool.p, ctx->npool);
     HIP_TRY(hipGetLastError());
     DbArgs a;
     a.wave = reinterpret_cast<const int4*>(ctx->db_wave.p);
@@ -889,7 +890,7 @@ extern "C" int ace_basis_dB(ace_ctx* ctx, int64_t nenv, const int32_t* off, cons
         return -1;
     hipLaunchKernelGGL(k_nbr_env, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, off,
                        ctx->nbr_env.p);
-    DISPATCH_L(ctx->L, launch_dphi, ctx, st, nnbr, xyz, species);
+    DISPATCH_L(ctx->L, launch_dphi, ctx, st, nnbr, xyz, species, ctx->aspec4.p, ctx->nA);
     HIP_TRY(hipGetLastError());
     const int64_t n1 = nnbr * ctx->nAA;
     hipLaunchKernelGGL(k_dAA, dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, st, nnbr, ctx->nA, ctx->nAA,
