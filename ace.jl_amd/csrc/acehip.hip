@@ -1265,10 +1265,13 @@ static bool use_slots(const ace_ctx* ctx, int64_t nenv, bool forces) {
 //   Up to one workgroup per CU: as many parts as the CUs take (256 order-4
 //   environments: 8 parts 0.026 ms, 2 parts 0.062, 1 part 0.110).
 //   More tiles than CUs: energies alone by the rounds' length; with forces
-//   two parts or more, whose tail tiles fill the last round at any tile
-//   count (100,000 environments: 2 parts with 64 tail tiles 1.48 ms, without
-//   1.51, 1 part 1.47 to 1.51, 3 parts 1.56; each part's G share is written
-//   and summed apart).
+//   a split whose tail tiles fill the last round at any tile count, or whole
+//   tiles: each part's G share is written and summed apart (the forces read
+//   about 40 clocks' worth per pooled value and share more).  Order 4, 139
+//   pooled values, whole tiles against two parts with their tail, whole call:
+//   24,700 environments (3.02 rounds) 0.654 and 0.599 ms, 30,011 (3.66) 0.681
+//   and 0.693, 41,400 (5.05) 0.958 and 0.927, 55,296 (6.75) 1.149 and 1.203,
+//   100,000 (12.2) 2.085 and 2.129, 131,072 (16.0) 2.616 and 2.747.
 // Batches that fit the allocation-free entry point take a split whose shares
 // fit it too, so that both entry points give the same bits.
 static int pair_shape(ace_ctx* ctx, int64_t nenv, bool forces, int& P, int64_t& nhi) {
@@ -1288,6 +1291,12 @@ static int pair_shape(ace_ctx* ctx, int64_t nenv, bool forces, int& P, int64_t& 
                 best = c;
                 P = q;
             }
+        }
+        if (forces && ntile > ctx->ncu) {
+            // the tail leaves half a workgroup's time uneven
+            const double r = (double)ntile / ctx->ncu;
+            const double split = r * (P * clocks(P) + (P - 1) * 40.0 * ctx->npool) + 0.5 * clocks(P);
+            if (std::ceil(r) * clocks(1) < split) P = 1;
         }
     }
     nhi = 0;

@@ -55,3 +55,24 @@ def test_pair_kernel(cuda, args, species, nenv):
     E, dE = ev.energy_forces(b)
     assert rel_err(E.cpu().numpy()[:n], -2.0 * E0) < 1e-12
     assert rel_err(dE.cpu().numpy().T[:off[n]], -2.0 * g0) < 1e-10
+
+
+@pytest.mark.parametrize("rounds,extra", [(1, 1), (4, 0), (4, 5)])
+def test_whole_tiles_or_a_split(cuda, rounds, extra):
+    """More tiles than compute units: whole tiles where their rounds are full,
+    a split or whole tiles past that, the same sums either way (1e-13)."""
+    ncu = torch.cuda.get_device_properties(0).multi_processor_count
+    nenv = 32 * ncu * rounds + extra
+    print(f"[gpu] pair kernel whole tiles or a split, {nenv} environments", flush=True)
+    basis, _ = basis_for(4, 5, 3)
+    off, R, sp = synth.random_envs(nenv, "fixed5", 11)
+    ev = HIPEvaluator(basis, synth.coefficients(len(basis), 3), device=0)
+    b = EnvBatch(off, R.T.copy(), sp, device="cuda:0")
+    E, dE = ev.energy_forces(b)
+    if extra == 0:
+        assert ev.last_dag_shape()[:2] == (1, 0)
+    E, dE = E.cpu().numpy(), dE.cpu().numpy()
+    for parts in (1, 2):
+        ev.set_parts(parts)
+        E1, dE1 = ev.energy_forces(b)
+        assert rel_err(E, E1.cpu().numpy()) < 1e-13 and rel_err(dE, dE1.cpu().numpy()) < 1e-13
