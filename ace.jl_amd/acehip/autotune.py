@@ -18,7 +18,7 @@ library's own choice (parts 0) at the widest workgroup stays where no shape is
 more than 1 % faster: the pair and slot kernels have workgroups of their own
 and leave the waves a matter of noise, which the surrogate's fallback, on the
 segment kernel, is not indifferent to (4 waves and 1 part instead of 16 and the
-automatic parts: 7.9 ms a step against 5.5).
+automatic parts: 7.9 ms a step against 4.6).
 Results are cached per (basis size, batch size, mode).
 """
 from __future__ import annotations

@@ -108,9 +108,10 @@ class HIPEvaluator:
 
     def last_dag_shape(self):
         """Product-DAG launch of the last call: (parts per tile, tail tiles,
-        kernel: 0 the pair kernel, or the segment kernel on 64-environment
-        tiles, 1 the segment kernel on narrower ones, else the
-        run interpreter's environments per tile)."""
+        kernel: 0 the pair or slot kernel, or the segment kernel on
+        64-environment tiles, 1 the segment kernel on narrower ones or the
+        slot kernel in its place, else the run interpreter's environments per
+        tile)."""
         p, t, k = C.c_int(), C.c_int64(), C.c_int()
         _lib.check(self.lib.ace_last_dag_shape(self.ctx, C.byref(p), C.byref(t), C.byref(k)))
         return p.value, t.value, k.value
@@ -136,9 +137,9 @@ class HIPEvaluator:
         _lib.check(self.lib.ace_set_pool_shape(self.ctx, int(chunk), int(envs_per_wave)))
 
     def set_kernel(self, mode: int = 0):
-        """Product-DAG kernel: 0 the pair kernel or the record-segment
-        kernel, whichever takes the basis (default), 1 the run interpreter always, 2 the per-record
-        dispatch kernel over the same records (comparison)."""
+        """Product-DAG kernel: 0 the pair, slot or record-segment kernel,
+        whichever takes the basis (default), 1 the run interpreter always,
+        2 the per-record dispatch kernel over the same records (comparison)."""
         _lib.check(self.lib.ace_set_kernel(self.ctx, int(mode)))
 
     def set_tail_parts(self, ntail: int = -1):

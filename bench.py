@@ -23,14 +23,12 @@ sys.path.insert(0, os.path.join(ROOT, "ace.jl_amd"))
 METRIC = "env/s energy+forces: plain FP64 vs surrogate at ≤1 meV/atom MAE"
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-# HBM bytes per product-DAG launch on this workload (100k environments, 16-wave
-# tiles split over 3 workgroups), from rocprofv3 --pmc FETCH_SIZE and
-# WRITE_SIZE runs of this script, scaled by the factors a 256 MiB device copy
-# gives the same counters (2.0 for FETCH_SIZE, 1.0 for WRITE_SIZE): 418.2 MB
-# read (the three workgroups of a tile each load its A+ rows, mostly from the
-# XCD's L2 after the first) + 269.7 MB written.  Only valid for the default
-# --nenv; re-measured whenever the kernel changes.
-DAG_TRAFFIC_BYTES = {100_000: 687.9e6}
+# HBM bytes per product-DAG launch on this workload (100k environments, whole
+# tiles), from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs of this script,
+# scaled by the factors a 256 MiB device copy gives the same counters (2.0 for
+# FETCH_SIZE, 1.0 for WRITE_SIZE): 227.7 MB read + 223.2 MB written.  Only valid
+# for the default --nenv; re-measured whenever the kernel changes.
+DAG_TRAFFIC_BYTES = {100_000: 450.9e6}
 WORKLOAD_NAMES = {
     1: "plain ACE energy+forces, 1000 envs x 12 neighbours, order 3, degree 6, Lmax 4, Invariant, FP64",
     2: "plain ACE energy+forces, 100k envs, nX~Poisson(30) clipped [5,80], order 4, degree 12, Lmax 6, "
@@ -81,7 +79,7 @@ def executed_flops(pack, forces=True, kernel=0):
     4 per leaf, 6 per new prefix product, 8 per run."""
     import numpy as np
     cplx = bool(getattr(pack, "classed", 0))
-    if pair_kernel(pack, kernel):
+    if pair_kernel(pack, kernel) or slot_kernel(pack, kernel):
         return None
     if kernel not in (0, 1):
         w = pack.work_counts(forces)
@@ -96,9 +94,15 @@ def executed_flops(pack, forces=True, kernel=0):
 
 def pair_kernel(pack, kernel):
     """Whether the pair kernel took the benchmark's calls (Invariant,
-    correlation order 4, at most 159 pooled values): its programs are the
+    correlation order 4 to 7, at most 159 pooled values): its programs are the
     library's own, so their operations are not counted here."""
-    return kernel == 0 and pack.prop == 0 and pack.maxorder == 4 and len(pack.pool) <= 159
+    return kernel == 0 and pack.prop == 0 and 4 <= pack.maxorder <= 7 and len(pack.pool) <= 159
+
+
+def slot_kernel(pack, kernel):
+    """Whether the slot kernel took them (class-split EuclideanVector, order
+    3, at most 319 pooled values), likewise."""
+    return (kernel in (0, 1) and bool(getattr(pack, "classed", 0)) and pack.maxorder == 3 and len(pack.pool) <= 319)
 
 
 def _segment_records(pack, forces):
@@ -125,7 +129,7 @@ def lds_read_bytes(pack, forces=True, kernel=0):
     tiles (ET < 64) each environment costs 64 / ET lanes.  None for the other
     kernels."""
     import numpy as np
-    if kernel not in (0, 1) or pair_kernel(pack, kernel):
+    if kernel not in (0, 1) or pair_kernel(pack, kernel) or slot_kernel(pack, kernel):
         return None
     d, nl, et = _segment_records(pack, forces)
     lanes = 64.0 / et if kernel == 1 else 1.0
@@ -136,6 +140,8 @@ def dag_kernel_name(pack, code):
     """The product-DAG kernel of ace_last_dag_shape's code."""
     if pair_kernel(pack, code):
         return "k_pairs (quadratic form in products of two pooled values, 32-environment tiles)"
+    if slot_kernel(pack, code):
+        return "k_slots (panels of gradient slots over shared products, 32-environment tiles)"
     if code == 0:
         return "k_dags (kind-sorted record segments, 64-environment tiles)"
     if code == 1:

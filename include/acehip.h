@@ -232,20 +232,23 @@ int ace_set_tail_parts(ace_ctx* ctx, int ntail);
 
 /* The product-DAG launch of the last evaluation call: workgroups per tile,
  * the number of tail tiles that ran one more part, and the kernel (0: the
- * pair kernel on 32-environment tiles or the segment kernel on
- * 64-environment tiles, 1: the segment kernel on narrower tiles; 64, 32
- * or 16: the run interpreter with that many environments per tile).
+ * pair kernel or the slot kernel on 32-environment tiles, or the segment
+ * kernel on 64-environment tiles, 1: the segment kernel on narrower tiles or
+ * the slot kernel in its place; 64, 32 or 16: the run interpreter with that
+ * many environments per tile).
  * Instrumentation; no counterpart in the reference. */
 int ace_last_dag_shape(ace_ctx* ctx, int* parts, int64_t* tail_tiles, int* kernel);
 
 /* Product-DAG kernel choice: 0 (default) the pair kernel for Invariant bases of
- * correlation order 4 with at most 159 pooled values (order 3: energies, and
- * batches of one tile per compute unit), else the
- * record-segment kernel where the basis allows it (Invariant or class-split EuclideanVector programs,
- * correlation order <= 4, at most 320 pooled values), else the run
- * interpreter; 1 the run interpreter always; 2 the per-record dispatch kernel
- * over the same records where they exist.  A tuning and testing knob of this
- * implementation; no counterpart in the reference. */
+ * correlation order 4 to 7 with at most 159 pooled values (order 3: energies,
+ * and batches of one tile per compute unit); the slot kernel for class-split
+ * EuclideanVector bases of order 3 with at most 319 pooled values; else the
+ * record-segment kernel where the basis allows it (Invariant or class-split
+ * EuclideanVector programs, correlation order <= 8 with at most 160 pooled
+ * values, <= 4 with at most 512), else the run interpreter; 1 the run
+ * interpreter always; 2 the per-record dispatch kernel over the same records
+ * where they exist.  A tuning and testing knob of this implementation; no
+ * counterpart in the reference. */
 int ace_set_kernel(ace_ctx* ctx, int mode);
 
 /* Pooling launch shape: neighbours staged per chunk (8, 16 or 32; 0 = 16)
@@ -275,8 +278,10 @@ int ace_energy_forces(ace_ctx* ctx, int64_t nenv, const int32_t* env_offsets,
  * caller passes nnbr = env_offsets[nenv] (the offsets are not validated).
  * The scratch (pooled values, adjoint, energy shares, neighbour map) lives
  * in a fixed 64 MiB device array, one per device for the life of the
- * process: a batch that needs more is rejected with an error (at the
- * order-4 degree-12 basis about 12,000 environments of 30 neighbours fit).
+ * process, and the further gradient shares of a split launch in 160 MiB behind
+ * it: a batch that needs more than the 64 MiB with one share is rejected with
+ * an error (at the order-4 degree-12 basis about 12,000 environments of 30
+ * neighbours fit), and any other takes a split whose shares fit.
  * Every call on one device shares that array, so calls that overlap on one
  * device (other contexts or streams included) race. */
 int ace_energy_forces_noalloc(ace_ctx* ctx, int64_t nenv, const int32_t* env_offsets, int64_t nnbr,
@@ -370,9 +375,10 @@ int ace_surr_energy_forces(ace_ctx* ctx, int64_t nenv, const int32_t* env_offset
  * executed leaf/run counts per environment. */
 int ace_last_timing(ace_ctx* ctx, double* dag_ms, double* pool_ms, double* force_ms);
 
-/* Host-side validation of env_offsets (non-decreasing, starting at 0) and
- * species (known categories) before every evaluation call: on (default) or
- * off for callers that validated their buffers once. */
+/* Validation of env_offsets (non-decreasing, starting at 0) and species
+ * (known categories) by a kernel before every evaluation call, which waits
+ * for its answer: on (default) or off for callers that validated their
+ * buffers once. */
 int ace_set_validation(ace_ctx* ctx, int on);
 
 const char* ace_last_error(void);
