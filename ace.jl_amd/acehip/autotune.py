@@ -13,12 +13,12 @@ Free shape parameters, all timed on the caller's batch:
   choice, which also gives the tiles of the last round one more part than the
   rest.
 
-Each shape is run once untimed, then ``reps`` times; the fastest is kept.  The
-library's own choice (parts 0) at the widest workgroup stays where no shape is
-more than 1 % faster: the pair and slot kernels have workgroups of their own
-and leave the waves a matter of noise, which the surrogate's fallback, on the
-segment kernel, is not indifferent to (4 waves and 1 part instead of 16 and the
-automatic parts: 7.9 ms a step against 4.6).
+Each shape is run once untimed, then ``reps`` times; the fastest is kept, but
+the library's own parts (0) and the widest workgroup stay where nothing is more than
+1 % faster: the pair and slot kernels have workgroups of their own and leave
+the waves a matter of noise, to which the surrogate's fallback, on the segment
+kernel, is not indifferent (4 waves and 1 part instead of 16 and the automatic parts:
+7.9 ms a step against 4.6).
 Results are cached per (basis size, batch size, mode).
 """
 from __future__ import annotations
@@ -89,8 +89,9 @@ def tune(ev, batch, forces: bool = True, reps: int = 3, candidates=None, parts=N
             ev.set_parts(P)
             results[(W, P)] = _time_call(fn, reps)
     Wbest, Pbest = min(results, key=results.get)
-    if results.get((max(cands), 0), float("inf")) <= 1.01 * results[(Wbest, Pbest)]:
-        Wbest, Pbest = max(cands), 0
+    for W, P in ((max(cands), Pbest), (max(cands), 0)):
+        if results.get((W, P), float("inf")) <= 1.01 * results[min(results, key=results.get)]:
+            Wbest, Pbest = W, P
     ev.set_tile(Wbest)
     ev.set_parts(Pbest)
     _CACHE[key] = ((Wbest, Pbest), results, pool)

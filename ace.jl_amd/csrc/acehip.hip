@@ -1271,7 +1271,10 @@ static bool use_slots(const ace_ctx* ctx, int64_t nenv, bool forces) {
 //   pooled values, whole tiles against two parts with their tail, whole call:
 //   24,700 environments (3.02 rounds) 0.654 and 0.599 ms, 30,011 (3.66) 0.681
 //   and 0.693, 41,400 (5.05) 0.958 and 0.927, 55,296 (6.75) 1.149 and 1.203,
-//   100,000 (12.2) 2.085 and 2.129, 131,072 (16.0) 2.616 and 2.747.
+//   100,000 (12.2) 2.085 and 2.129, 131,072 (16.0) 2.616 and 2.747.  The model
+//   favours whole tiles a little (36,000, 0.975 of the split by the model, 0.825
+//   and 0.806), so they must be 6 % shorter by it; 100,000 (0.945) thereby keep
+//   their split.
 // Batches that fit the allocation-free entry point take a split whose shares
 // fit it too, so that both entry points give the same bits.
 static int pair_shape(ace_ctx* ctx, int64_t nenv, bool forces, int& P, int64_t& nhi) {
@@ -1296,7 +1299,7 @@ static int pair_shape(ace_ctx* ctx, int64_t nenv, bool forces, int& P, int64_t& 
             // the tail leaves half a workgroup's time uneven
             const double r = (double)ntile / ctx->ncu;
             const double split = r * (P * clocks(P) + (P - 1) * 40.0 * ctx->npool) + 0.5 * clocks(P);
-            if (std::ceil(r) * clocks(1) < split) P = 1;
+            if (std::ceil(r) * clocks(1) < 0.94 * split) P = 1;
         }
     }
     nhi = 0;
