@@ -659,8 +659,8 @@ __global__ void k_nbr_env(int64_t nenv, const int32_t* __restrict__ off, int32_t
 static int basis_A_internal(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* xyz,
                             const int8_t* species, int64_t nnbr, hipStream_t st) {
     const int64_t estride = ((nenv + 63) / 64) * 64;
-    if (ctx->Aplus.ensure((size_t)ctx->npool * estride)) return -1;
-    if (ctx->Afull.ensure((size_t)nenv * ctx->nA)) return -1;
+    if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing)) return -1;
+    if (ctx->Afull.ensure((size_t)nenv * ctx->nA, ctx->capturing)) return -1;
     if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false)) return -1;
     const int64_t n = nenv * ctx->nA;
     hipLaunchKernelGGL(k_expandA, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, nenv, ctx->nA,
@@ -682,7 +682,7 @@ extern "C" int ace_basis_A(ace_ctx* ctx, int64_t nenv, const int32_t* off, const
 }
 
 static int basis_AA_internal(ace_ctx* ctx, int64_t nenv, hipStream_t st) {
-    if (ctx->AA.ensure((size_t)nenv * ctx->nAA)) return -1;
+    if (ctx->AA.ensure((size_t)nenv * ctx->nAA, ctx->capturing)) return -1;
     const int64_t n = nenv * ctx->nAA;
     hipLaunchKernelGGL(k_AA, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, nenv, ctx->nA, ctx->nAA,
                        ctx->maxorder, ctx->orders.p, ctx->iAA2iA.p, ctx->Afull.p, ctx->AA.p);
@@ -770,7 +770,7 @@ extern "C" int ace_basis_B(ace_ctx* ctx, int64_t nenv, const int32_t* off, const
     {
         const int64_t estride = ((nenv + 63) / 64) * 64;
         if (bt_fits(ctx, false)) {
-            if (ctx->Aplus.ensure((size_t)ctx->npool * estride)) return -1;
+            if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing)) return -1;
             if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false)) return -1;
             return launch_bt<false>(ctx, st, nenv, estride, B_out);
         }
@@ -827,8 +827,8 @@ static int basis_dB_weights(ace_ctx* ctx, hipStream_t st, int64_t nenv, const in
         ctx->db_ready = true;
     }
     const int64_t estride = ((nenv + 63) / 64) * 64;
-    if (ctx->Aplus.ensure((size_t)ctx->npool * estride) || ctx->nbr_env.ensure(nnbr) ||
-        ctx->dphi.ensure((size_t)nnbr * ctx->npool * 3))
+    if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing) || ctx->nbr_env.ensure(nnbr, ctx->capturing) ||
+        ctx->dphi.ensure((size_t)nnbr * ctx->npool * 3, ctx->capturing))
         return -1;
     if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false)) return -1;
     hipLaunchKernelGGL(k_nbr_env, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, off,
@@ -885,8 +885,8 @@ extern "C" int ace_basis_dB(ace_ctx* ctx, int64_t nenv, const int32_t* off, cons
     if (rc <= 0) return rc;
     // bases whose tables exceed the weight kernel's LDS: dAA per neighbour
     if (basis_A_internal(ctx, nenv, off, xyz, species, nnbr, st)) return -1;
-    if (ctx->nbr_env.ensure(nnbr) || ctx->dphi.ensure((size_t)nnbr * ctx->nA * 3) ||
-        ctx->dAA.ensure((size_t)nnbr * ctx->nAA * 3))
+    if (ctx->nbr_env.ensure(nnbr, ctx->capturing) || ctx->dphi.ensure((size_t)nnbr * ctx->nA * 3, ctx->capturing) ||
+        ctx->dAA.ensure((size_t)nnbr * ctx->nAA * 3, ctx->capturing))
         return -1;
     hipLaunchKernelGGL(k_nbr_env, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, off,
                        ctx->nbr_env.p);
@@ -917,7 +917,8 @@ extern "C" int ace_adjoint_EVAL_D(ace_ctx* ctx, int64_t nenv, const int32_t* off
     hipStream_t st = (hipStream_t)stream;
     const int64_t estride = ((nenv + 63) / 64) * 64;
     if (bt_fits(ctx, true)) {
-        if (ctx->Aplus.ensure((size_t)ctx->npool * estride) || ctx->Wplus.ensure((size_t)ctx->npool * estride))
+        if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing) ||
+            ctx->Wplus.ensure((size_t)ctx->npool * estride, ctx->capturing))
             return -1;
         if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false) ||
             launch_poolw_any(ctx, st, nenv, off, xyz, w, nnbr, species, estride))
@@ -925,8 +926,9 @@ extern "C" int ace_adjoint_EVAL_D(ace_ctx* ctx, int64_t nenv, const int32_t* off
         return launch_bt<true>(ctx, st, nenv, estride, dB_out);
     }
     if (basis_A_internal(ctx, nenv, off, xyz, species, nnbr, st)) return -1;
-    if (ctx->Wplus.ensure((size_t)ctx->npool * estride) || ctx->Wfull.ensure((size_t)nenv * ctx->nA) ||
-        ctx->AA.ensure((size_t)nenv * ctx->nAA))
+    if (ctx->Wplus.ensure((size_t)ctx->npool * estride, ctx->capturing) ||
+        ctx->Wfull.ensure((size_t)nenv * ctx->nA, ctx->capturing) ||
+        ctx->AA.ensure((size_t)nenv * ctx->nAA, ctx->capturing))
         return -1;
     if (launch_poolw_any(ctx, st, nenv, off, xyz, w, nnbr, species, estride)) return -1;
     const int64_t n = nenv * ctx->nA;
@@ -985,8 +987,11 @@ extern "C" int ace_weighted_rows(ace_ctx* ctx, int64_t nrow, int64_t ncol, const
     const int64_t per = std::max<int64_t>(1, (nrow + want - 1) / want);
     const int nshare = (int)((nrow + per - 1) / per);
     if (per >= ((int64_t)1 << 31)) return set_err("ace_weighted_rows: too many rows");
-    if (ctx->wrows.ensure((size_t)std::max(1, nshare) * ncol)) return -1;
     hipStream_t st = (hipStream_t)stream;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(st, &cap));
+    ctx->capturing = cap != hipStreamCaptureStatusNone;
+    if (ctx->wrows.ensure((size_t)std::max(1, nshare) * ncol, ctx->capturing)) return -1;
     if (nshare > 0)
         hipLaunchKernelGGL(k_wrows, dim3((unsigned)gx, (unsigned)nshare), dim3(256), 0, st, nrow, ncol, (int)per, w, B,
                            ctx->wrows.p);

@@ -390,6 +390,7 @@ struct ace_ctx {
     // timing
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool timing_valid = false;
+    bool capturing = false;  // the present call is being captured into a graph
     bool validate = true;
     ~ace_ctx() {
         if (h_words) (void)hipHostFree(h_words);

@@ -166,9 +166,9 @@ extern "C" int ace_surr_features(ace_ctx* ctx, int64_t nenv, const int32_t* off,
     if (!xmean || !xinvstd || !E2) return set_err("ace_surr_features: null argument");
     hipStream_t st = (hipStream_t)stream;
     const int64_t estride = ((nenv + 63) / 64) * 64;
-    if (ctx->Aplus.ensure((size_t)ctx->npool * estride)) return -1;
+    if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing)) return -1;
     // the neighbour map is written for the force kernel of the following call
-    if (ctx->flat_force && nnbr > 0 && ctx->nbr_env.ensure(nnbr)) return -1;
+    if (ctx->flat_force && nnbr > 0 && ctx->nbr_env.ensure(nnbr, ctx->capturing)) return -1;
     if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), ctx->flat_force))
         return -1;
     hipLaunchKernelGGL(k_feat, dim3((unsigned)((nenv + 63) / 64)), dim3(64), 0, st, feat_args(ctx), nenv,
@@ -200,7 +200,7 @@ extern "C" int ace_surr_energy_forces(ace_ctx* ctx, int64_t nenv, const int32_t*
     HIP_TRY(hipGetLastError());
     const bool forces = dE != nullptr;
     if (forces) {
-        if (ctx->Gbuf.ensure((size_t)std::max(1, ctx->ngslots) * estride)) return -1;
+        if (ctx->Gbuf.ensure((size_t)std::max(1, ctx->ngslots) * estride, ctx->capturing)) return -1;
         const size_t fg_lds = (size_t)ctx->nfeat * FG_PAD * sizeof(double);
         set_func_lds((const void*)k_feat_grad, fg_lds);
         hipLaunchKernelGGL(k_feat_grad, dim3((unsigned)ntile), dim3(256), fg_lds, st, feat_args(ctx), nenv,

@@ -1423,7 +1423,8 @@ int check_common(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* x
     HIP_TRY(hipSetDevice(ctx->device));
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing((hipStream_t)stream, &cap));
-    if (cap != hipStreamCaptureStatusNone) {
+    ctx->capturing = cap != hipStreamCaptureStatusNone;
+    if (ctx->capturing) {
         // stream capture (hipGraph): no host reads; the neighbour count comes
         // from the eager call on the same batch that must precede the capture
         // (it also sizes every scratch buffer)
@@ -1666,7 +1667,7 @@ static int run_path(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double
     if (!E_out) return set_err("null E_out");
     const int64_t estride = ((nenv + 63) / 64) * 64;
     const bool forces = dE != nullptr;
-    if (ctx->Aplus.ensure((size_t)ctx->npool * estride)) return -1;
+    if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing)) return -1;
     size_t gslots = (size_t)std::max(1, ctx->ngslots) * gslot_width(ctx), eslots = (size_t)MAX_PARTS * (ctx->classed ? 6 : 1);
     if (use_pairs(ctx, nenv, forces)) {
         int P = 0;
@@ -1678,9 +1679,9 @@ static int run_path(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double
         gslots = std::max(gslots, (size_t)ctx->slots[0].host.nslots);
         eslots = std::max(eslots, (size_t)6 * slot_shape(ctx, nenv, forces).P_hi);
     }
-    if (forces && ctx->Gbuf.ensure(gslots * estride)) return -1;
-    if ((ctx->seg_et > 0 || ctx->rec_et > 0) && ctx->Epart.ensure(eslots * estride)) return -1;
-    if (forces && ctx->flat_force && nnbr > 0 && ctx->nbr_env.ensure(nnbr)) return -1;
+    if (forces && ctx->Gbuf.ensure(gslots * estride, ctx->capturing)) return -1;
+    if ((ctx->seg_et > 0 || ctx->rec_et > 0) && ctx->Epart.ensure(eslots * estride, ctx->capturing)) return -1;
+    if (forces && ctx->flat_force && nnbr > 0 && ctx->nbr_env.ensure(nnbr, ctx->capturing)) return -1;
     return eval_path(ctx, (hipStream_t)stream, nenv, off, xyz, nnbr, species, E_out, dE, ctx_buffers(ctx));
 }
 

@@ -1,12 +1,13 @@
 // Host helpers shared by the translation units of libacehip.so: the
 // thread-local error message behind ace_last_error(), the HIP_TRY macro and
-// a grow-only device buffer.
+// the grow-only buffer on device memory.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <string>
+
+#include "grow_buf.hpp"
 
 // last error message of the calling thread (one instance per process)
 inline thread_local std::string g_err;
@@ -23,27 +24,17 @@ inline int set_err(const std::string& s) {
             return set_err(std::string(#expr) + ": " + hipGetErrorString(e_));    \
     } while (0)
 
-template <typename T>
-struct DevBuf {
-    T* p = nullptr;
-    size_t n = 0;
-    ~DevBuf() {
-        if (p) (void)hipFree(p);
-    }
-    int ensure(size_t count) {
-        if (count <= n) return 0;
-        if (p) {
-            (void)hipFree(p);
-            p = nullptr;
-            n = 0;
-        }
-        HIP_TRY(hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)));
-        n = count;
+struct HipMemory {
+    static int alloc(void** p, size_t bytes) {
+        HIP_TRY(hipMalloc(p, bytes));
         return 0;
     }
-    int upload(const T* h, size_t count) {
-        if (ensure(count)) return -1;
-        if (count) HIP_TRY(hipMemcpy(p, h, count * sizeof(T), hipMemcpyHostToDevice));
+    static void release(void* p) { (void)hipFree(p); }
+    static int copy(void* p, const void* host, size_t bytes) {
+        HIP_TRY(hipMemcpy(p, host, bytes, hipMemcpyHostToDevice));
         return 0;
     }
 };
+
+template <typename T>
+using DevBuf = acehost::GrowBuf<T, HipMemory>;

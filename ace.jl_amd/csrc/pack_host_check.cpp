@@ -8,6 +8,7 @@
 
 #include "basis_host.hpp"
 #include "compile_host.hpp"
+#include "grow_buf.hpp"
 #include "nbrlist_host.hpp"
 #include "pack_host.hpp"
 #include "pairs_host.hpp"
@@ -316,4 +317,42 @@ extern "C" int acehost_class(const ace_pack* pk, const double* c, double* u, dou
         for (int q = 0; q < 6; ++q) u[6 * i + q] = pc.cv.u[i][q];
     for (int q = 0; q < 3; ++q) e0[q] = cf.e0[2 * q];
     return 0;
+}
+
+// Calls of sizes[n], those with captured[i] set recorded in a graph: how many
+// of the blocks that the graphs point to are live after the last call, of how
+// many graphs; *blocks the blocks alive then, *left those alive once the
+// buffer is gone.
+namespace {
+struct CheckMemory {
+    static std::set<void*>& live() {
+        static std::set<void*> s;
+        return s;
+    }
+    static int alloc(void** p, size_t bytes) {
+        live().insert(*p = new char[bytes]);
+        return 0;
+    }
+    static void release(void* p) {
+        live().erase(p);
+        delete[] static_cast<char*>(p);
+    }
+};
+}  // namespace
+extern "C" int acehost_grow_buf(const int64_t* sizes, const int32_t* captured, int n, int* graphs, int* blocks,
+                                int* left) {
+    int ok = 0;
+    {
+        acehost::GrowBuf<double, CheckMemory> buf;
+        std::vector<void*> used;
+        for (int i = 0; i < n; ++i) {
+            if (buf.ensure((size_t)sizes[i], captured[i] != 0)) return -1;
+            if (captured[i]) used.push_back(buf.p);
+        }
+        for (void* p : used) ok += CheckMemory::live().count(p) ? 1 : 0;
+        *graphs = (int)used.size();
+        *blocks = (int)CheckMemory::live().size();
+    }
+    *left = (int)CheckMemory::live().size();
+    return ok;
 }

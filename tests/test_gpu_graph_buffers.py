@@ -1,0 +1,55 @@
+"""A captured call keeps its scratch (gpu): after eager calls on smaller batches
+that need more room (their tiles are split further), each replay still gives
+the eager result, bit for bit, with other memory handed out in between."""
+import pytest
+import torch
+
+from acehip import synth
+from acehip.evaluator import EnvBatch, HIPEvaluator
+from helpers import basis_for
+
+pytestmark = pytest.mark.gpu
+
+
+def _capture(run):
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        run()
+    torch.cuda.current_stream().wait_stream(s)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        run()
+    return g
+
+
+@pytest.mark.parametrize("args,kw,wid,captured,others", [
+    ((4, 12, 6), {}, 2, 8192, (5000, 6000)),  # the pair kernel's G shares
+    ((3, 10, 5), {"prop": "EuclideanVector", "species": 2}, 4, 16384, (8193,)),  # the slot kernel's energy shares
+], ids=["pairs", "slots"])
+def test_replay_after_smaller_eager_batches(cuda, args, kw, wid, captured, others):
+    print(f"[gpu] capture {captured} envs, evaluate {others}, replay", flush=True)
+    basis, _ = basis_for(*args, **kw)
+    ev = HIPEvaluator(basis, synth.coefficients(len(basis), wid), device=0, waves=16)
+    ev.set_validation(False)
+
+    def batch(n, seed):
+        off, R, sp = synth.workload_envs(wid, nenv=n, seed=seed)
+        return EnvBatch(off, R.T.copy(), sp, device="cuda:0")
+
+    b = batch(captured, 11)
+    E0, dE0 = ev.energy_forces(b)
+    E, dE = torch.empty_like(E0), torch.empty_like(dE0)
+    g = _capture(lambda: ev.energy_forces(b, E, dE))
+    for i, n in enumerate(others + (None,) * 2):
+        if n is not None:
+            ev.energy_forces(batch(n, 20 + i))
+        hog = [torch.full((1 << 24,), float("nan"), dtype=torch.float64, device="cuda:0") for _ in range(2)]
+        E.zero_()
+        dE.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(E, E0) and torch.equal(dE, dE0), n
+        assert all(bool(h.isnan().all()) for h in hog)
+        del hog
