@@ -875,7 +875,13 @@ extern "C" int ace_nbrlist_forces(ace_nbrlist* nl, int64_t natoms, const int32_t
     const int64_t ngrp = ((int64_t)n + FA_ATOMS - 1) / FA_ATOMS;
     const int per = (int)((ngrp + FA_BLOCKS - 1) / FA_BLOCKS);
     const int nblk = (int)((ngrp + per - 1) / per);
-    if (virial && nl->vpart.ensure((size_t)nblk * 9)) return -1;
+    if (virial) {
+        // a graph keeps its block: fewer atoms may take more workgroups (32,768
+        // 2,048, 40,000 1,250)
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(st, &cap));
+        if (nl->vpart.ensure((size_t)nblk * 9, cap != hipStreamCaptureStatusNone)) return -1;
+    }
     hipLaunchKernelGGL(k_nbr_forces, dim3((unsigned)nblk), dim3(256), 0, st, n, per, env_offsets, rev, nnbr, dE_dr, xyz, F,
                        virial ? nl->vpart.p : nullptr);
     HIP_TRY(hipGetLastError());

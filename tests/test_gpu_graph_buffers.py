@@ -1,10 +1,13 @@
-"""A captured call keeps its scratch (gpu): after eager calls on smaller batches
+"""A captured call keeps its scratch (gpu), of a context and of a neighbour
+list: after eager calls on smaller batches
 that need more room (their tiles are split further), each replay still gives
 the eager result, bit for bit, with other memory handed out in between."""
+import numpy as np
 import pytest
 import torch
 
 from acehip import synth
+from acehip.atoms import NeighbourList
 from acehip.evaluator import EnvBatch, HIPEvaluator
 from helpers import basis_for
 
@@ -53,3 +56,33 @@ def test_replay_after_smaller_eager_batches(cuda, args, kw, wid, captured, other
         assert torch.equal(E, E0) and torch.equal(dE, dE0), n
         assert all(bool(h.isnan().all()) for h in hog)
         del hog
+
+
+def test_replay_of_forces_after_fewer_atoms(cuda):
+    """The virial's shares: 32,768 atoms take more workgroups than 40,000."""
+    print("[gpu] capture the forces of 40,000 atoms, then 32,768 on the same list", flush=True)
+    rng = np.random.default_rng(3)
+
+    def listed(n):
+        a = (8.0 * n) ** (1.0 / 3.0)  # about four neighbours within 2
+        nl = NeighbourList(0).build(rng.uniform(0.0, a, size=(n, 3)), a * np.eye(3), [1, 1, 1], 2.0)
+        return nl, torch.tensor(rng.normal(size=(3, nl.nnbr)), device="cuda:0")
+
+    nl, g = listed(40000)
+    few, gf = listed(32768)
+    few.h, own = nl.h, few.h  # the other list's arrays through the same handle
+    F0, W0 = nl.forces(g, virial=True)
+    F, W = torch.empty_like(F0), torch.empty_like(W0)
+    graph = _capture(lambda: nl._forces(g, F, W))
+    try:
+        for rep in range(4):
+            few.forces(gf, virial=True)
+            hog = torch.full((1 << 20,), float("nan"), dtype=torch.float64, device="cuda:0")
+            F.zero_()
+            W.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(F, F0) and torch.equal(W, W0), rep
+            assert bool(hog.isnan().all())
+    finally:
+        few.h = own
