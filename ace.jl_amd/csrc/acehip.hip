@@ -1659,6 +1659,14 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
     return 0;
 }
 
+// Energy shares (doubles per environment) that a call's kernel may write.
+static size_t energy_slots(const ace_ctx* ctx, int64_t nenv, bool forces) {
+    const size_t n = (size_t)MAX_PARTS * (ctx->classed ? 6 : 1);
+    if (use_pairs(ctx, nenv, forces)) return std::max<size_t>(n, acehost::PAIR_MAXP + 1);
+    if (use_slots(ctx, nenv, forces)) return std::max(n, (size_t)6 * slot_shape(ctx, nenv, forces).P_hi);
+    return n;
+}
+
 static int run_path(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* xyz,
                     const int8_t* species, double* E_out, double* dE, void* stream) {
     int64_t nnbr = 0;
@@ -1668,17 +1676,17 @@ static int run_path(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double
     const int64_t estride = ((nenv + 63) / 64) * 64;
     const bool forces = dE != nullptr;
     if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing)) return -1;
-    size_t gslots = (size_t)std::max(1, ctx->ngslots) * gslot_width(ctx), eslots = (size_t)MAX_PARTS * (ctx->classed ? 6 : 1);
+    size_t gslots = (size_t)std::max(1, ctx->ngslots) * gslot_width(ctx);
     if (use_pairs(ctx, nenv, forces)) {
         int P = 0;
         int64_t nhi = 0;
         if (pair_shape(ctx, nenv, forces, P, nhi)) return -1;
         gslots = std::max(gslots, (size_t)(P + (nhi > 0)) * ctx->npool);
-        eslots = std::max(eslots, (size_t)(P + (nhi > 0)));
     } else if (use_slots(ctx, nenv, forces)) {
         gslots = std::max(gslots, (size_t)ctx->slots[0].host.nslots);
-        eslots = std::max(eslots, (size_t)6 * slot_shape(ctx, nenv, forces).P_hi);
     }
+    // for energies and for forces: after either call, the other can be captured
+    const size_t eslots = std::max(energy_slots(ctx, nenv, false), energy_slots(ctx, nenv, true));
     if (forces && ctx->Gbuf.ensure(gslots * estride, ctx->capturing)) return -1;
     if ((ctx->seg_et > 0 || ctx->rec_et > 0) && ctx->Epart.ensure(eslots * estride, ctx->capturing)) return -1;
     if (forces && ctx->flat_force && nnbr > 0 && ctx->nbr_env.ensure(nnbr, ctx->capturing)) return -1;

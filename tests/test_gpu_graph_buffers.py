@@ -86,3 +86,35 @@ def test_replay_of_forces_after_fewer_atoms(cuda):
             assert bool(hog.isnan().all())
     finally:
         few.h = own
+
+
+@pytest.mark.parametrize("args,kw,wid,sizes", [
+    ((4, 12, 6), {}, 2, (1500, 9000)),
+    # the slot kernel's energies over more workgroups than its forces: 6 against 3, 7 against 6
+    ((3, 10, 5), {"prop": "EuclideanVector"}, 4, (64, 700)),
+    ((3, 10, 5), {"prop": "EuclideanVector", "species": 2}, 4, (3300,)),
+], ids=["pairs", "slots", "slots2"])
+def test_energies_captured_after_forces(cuda, args, kw, wid, sizes):
+    """One eager call on the batch precedes a capture, in either mode: the call
+    with forces also makes the room for the energies alone."""
+    basis, _ = basis_for(*args, **kw)
+    c = synth.coefficients(len(basis), wid)
+    for n in sizes:
+        print(f"[gpu] energies of {n} envs captured after an eager call with forces", flush=True)
+        off, R, sp = synth.workload_envs(wid, nenv=n, seed=31)
+        b = EnvBatch(off, R.T.copy(), sp if kw.get("species") else None, device="cuda:0")
+        E0 = HIPEvaluator(basis, c, device=0, waves=16).energy(b)
+        ev = HIPEvaluator(basis, c, device=0, waves=16)
+        ev.set_validation(False)
+        E = torch.empty_like(E0)
+        ev.energy_forces(b)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            ev.energy(b, E)
+        for rep in range(3):
+            E.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(E, E0), (n, rep)
+            ev.energy_forces(b)
