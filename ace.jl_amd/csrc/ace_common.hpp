@@ -28,6 +28,7 @@
 #include "pack_host.hpp"
 #include "pairs_host.hpp"
 #include "slots_host.hpp"
+#include "tail_host.hpp"
 
 #define ACE_LMAX 10
 #define ACE_NPMAX ((ACE_LMAX + 1) * (ACE_LMAX + 2) / 2)

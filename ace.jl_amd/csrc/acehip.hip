@@ -1161,40 +1161,6 @@ extern "C" int ace_set_params(ace_ctx* ctx, const double* c, int64_t nB) {
     return upload_coeffs(ctx, c);
 }
 
-// Tail tiles for the automatic parts choice.  The grid runs in rounds of ncu
-// workgroups of equal length d.  Giving the last n tiles P + 1 parts fills the
-// partial last round with shorter workgroups of length dh (segment kernel:
-// 1/(P + 1) of the tile's work plus 8 % for re-staging and thinner task lists,
-// measured 0.200 ms per workgroup with 4 parts against 0.246 ms with 3 at 100k
-// environments).  The makespan of a greedy dispatch of such workgroups onto
-// ncu units is flat over a range of n; take the middle of that range.
-static int64_t choose_tail(int64_t ntile, int P, int ncu, double d, double dh) {
-    std::vector<double> h((size_t)ncu);
-    auto makespan = [&](int64_t nhi) {
-        // the P-part workgroups: full rounds, then r units busy one more
-        const int64_t w = (ntile - nhi) * P, f = w / ncu, r = w % ncu;
-        for (int i = 0; i < ncu; ++i) h[(size_t)i] = (i < r ? f + 1 : f) * d;
-        std::make_heap(h.begin(), h.end(), std::greater<double>());
-        for (int64_t k = 0; k < nhi * (P + 1); ++k) {
-            std::pop_heap(h.begin(), h.end(), std::greater<double>());
-            h.back() += dh;
-            std::push_heap(h.begin(), h.end(), std::greater<double>());
-        }
-        return *std::max_element(h.begin(), h.end());
-    };
-    const int64_t nmax = std::min<int64_t>(ntile, ncu);
-    std::vector<double> ms((size_t)nmax + 1);
-    double best = 1e300;
-    for (int64_t n = 0; n <= nmax; ++n) {
-        ms[(size_t)n] = makespan(n);
-        best = std::min(best, ms[(size_t)n]);
-    }
-    std::vector<int64_t> ties;
-    for (int64_t n = 0; n <= nmax; ++n)
-        if (ms[(size_t)n] <= best * (1.0 + 1e-9)) ties.push_back(n);
-    return ties[ties.size() / 2];
-}
-
 // The segment kernel's parts per tile when the caller leaves the choice: the
 // grid runs in rounds of ncu workgroups, and the last round may be nearly
 // empty; splitting each tile's tasks over P workgroups shortens the rounds.
@@ -1316,7 +1282,7 @@ static int pair_shape(ace_ctx* ctx, int64_t nenv, bool forces, int& P, int64_t& 
         auto it = ctx->tail_cache.find(key);
         if (it == ctx->tail_cache.end()) {
             if (ctx->tail_cache.size() >= 64) ctx->tail_cache.clear();
-            it = ctx->tail_cache.emplace(key, choose_tail(ntile, P, ctx->ncu, clocks(P), clocks(P + 1))).first;
+            it = ctx->tail_cache.emplace(key, acehost::choose_tail(ntile, P, ctx->ncu, clocks(P), clocks(P + 1))).first;
         }
         nhi = it->second;
     }
@@ -1608,7 +1574,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
             auto it = ctx->tail_cache.find(key);
             if (it == ctx->tail_cache.end()) {
                 if (ctx->tail_cache.size() >= 64) ctx->tail_cache.clear();
-                it = ctx->tail_cache.emplace(key, choose_tail(ntile, P, ctx->ncu, 1.0 / P, 1.08 / (P + 1))).first;
+                it = ctx->tail_cache.emplace(key, acehost::choose_tail(ntile, P, ctx->ncu, 1.0 / P, 1.08 / (P + 1))).first;
             }
             nhi = it->second;
         }

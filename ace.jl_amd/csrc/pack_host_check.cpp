@@ -13,6 +13,7 @@
 #include "pack_host.hpp"
 #include "pairs_host.hpp"
 #include "slots_host.hpp"
+#include "tail_host.hpp"
 
 extern "C" int acehost_validate(const ace_pack* pk, char* msg, int len) {
     std::string e = acehost::validate_pack(pk);
@@ -355,4 +356,8 @@ extern "C" int acehost_grow_buf(const int64_t* sizes, const int32_t* captured, i
     }
     *left = (int)CheckMemory::live().size();
     return ok;
+}
+
+extern "C" int64_t acehost_choose_tail(int64_t ntile, int P, int ncu, double d, double dh) {
+    return acehost::choose_tail(ntile, P, ncu, d, dh);
 }
