@@ -1346,14 +1346,26 @@ extern "C" void ace_ctx_destroy(ace_ctx* ctx) {
     delete ctx;
 }
 
+// Bytes from p to the end of its allocation, as far as the runtime knows it.
+static size_t bytes_behind(const void* p) {
+    hipDeviceptr_t base = nullptr;
+    size_t n = 0;
+    if (hipMemGetAddressRange(&base, &n, const_cast<void*>(p)) != hipSuccess) {
+        (void)hipGetLastError();
+        return SIZE_MAX;
+    }
+    return (size_t)((const char*)base + n - (const char*)p);
+}
+
 // Bounds of every kernel, checked on the device: w[0], w[1] the first and the
-// last offset, with `all` w[2] whether some offset decreases (w is pinned host
-// memory, read after the stream has been waited for).  usable: the number of
-// neighbours k_check_species may read.  One workgroup, so that one launch
+// last offset, with `all` w[2] whether some offset decreases (1) or the last
+// exceeds the nspecies bytes there are (2) (w is pinned host memory, read after
+// the stream has been waited for).  usable: the number of neighbours
+// k_check_species may read.  One workgroup, so that one launch
 // answers; 20,011 offsets take 6 us, copying them to the host and looping
 // there took 45.
-__global__ __launch_bounds__(1024) void k_check(int64_t nenv, const int32_t* __restrict__ off, bool all, int32_t* w,
-                                                int32_t* usable) {
+__global__ __launch_bounds__(1024) void k_check(int64_t nenv, const int32_t* __restrict__ off, bool all,
+                                                size_t nspecies, int32_t* w, int32_t* usable) {
     int bad = 0;
     if (all) {
 #pragma unroll 8
@@ -1362,6 +1374,7 @@ __global__ __launch_bounds__(1024) void k_check(int64_t nenv, const int32_t* __r
     }
     if (threadIdx.x == 0) {
         const int32_t first = off[0], last = off[nenv];
+        bad = (bad ? 1 : 0) | (last > 0 && (size_t)last > nspecies ? 2 : 0);
         w[0] = first;
         w[1] = last;
         w[2] = bad;
@@ -1407,9 +1420,13 @@ int check_common(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* x
     hipStream_t st = (hipStream_t)stream;
     volatile int32_t* const w = ctx->h_words;
     const bool all = ctx->validate, sp = all && species && ctx->nspecies > 0;
+    // arrays that end before what the batch claims, where the runtime can tell
+    if (all && bytes_behind(off) < ((size_t)nenv + 1) * sizeof(int32_t))
+        return set_err("env_offsets is shorter than nenv + 1");
+    const size_t nsp = sp ? bytes_behind(species) : SIZE_MAX;
     w[2] = 0;
     w[3] = 0;
-    hipLaunchKernelGGL(k_check, dim3(1), dim3(all && nenv > 64 ? 1024 : 64), 0, st, nenv, off, all, ctx->d_words,
+    hipLaunchKernelGGL(k_check, dim3(1), dim3(all && nenv > 64 ? 1024 : 64), 0, st, nenv, off, all, nsp, ctx->d_words,
                        ctx->usable.p);
     if (sp)
         hipLaunchKernelGGL(k_check_species, dim3((unsigned)std::min<int64_t>(512, (nenv + 7) / 8)), dim3(256), 0, st,
@@ -1417,7 +1434,8 @@ int check_common(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* x
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
     if (w[0] != 0 || w[1] < 0) return set_err("env_offsets must start at 0 and be non-negative");
-    if (w[2]) return set_err("env_offsets must be non-decreasing");
+    if (w[2] & 1) return set_err("env_offsets must be non-decreasing");
+    if (w[2]) return set_err("species is shorter than env_offsets[nenv]");
     if (w[3]) return set_err("species index out of range (unknown category)");
     ctx->batch_off = off;
     ctx->batch_nenv = nenv;
