@@ -336,14 +336,17 @@ __global__ __launch_bounds__(256) void k_nbr_rev(int natoms, const int32_t* __re
     const int t = xcd_share(blockIdx.x, gridDim.x) * 4 + wave;
     if (t >= natoms) return;
     const int i = atoms[t];
-    const int m0 = off[i], m1 = off[i + 1];
+    // entries are counted without a sign: a list may end at 2^31 - 1, and the
+    // steps of 64 and the lanes past its end go beyond
+    const uint32_t m0 = off[i], m1 = off[i + 1];
     const int sub = lane & 15;
-    for (int mb = m0; mb < m1; mb += 64) {
-        const int cnt = min(64, m1 - mb);
+    for (uint32_t mb = m0; mb < m1; mb += 64) {
+        const int cnt = (int)min(64u, m1 - mb);
         const bool mine = lane < cnt;
-        int qa = 0, qb = 0, s0 = 0, s1 = 0, s2 = 0;
+        uint32_t qa = 0, qb = 0;
+        int s0 = 0, s1 = 0, s2 = 0;
         if (mine) {
-            const int64_t m = mb + lane;
+            const int64_t m = (int64_t)mb + lane;
             const int j = nbr_j[m];
             s0 = -shift[m];
             s1 = -shift[nnbr + m];
@@ -355,12 +358,12 @@ __global__ __launch_bounds__(256) void k_nbr_rev(int natoms, const int32_t* __re
 #pragma unroll 2
         for (int e = 0; e < cnt; e += 4) {
             const int src = e + (lane >> 4);  // lanes past the last entry search an empty list
-            const int q0 = __shfl(qa, src), q1 = __shfl(qb, src);
-            for (int p = 0; __any(q0 + p < q1); p += 64) {
+            const uint32_t q0 = __shfl(qa, src), q1 = __shfl(qb, src);
+            for (uint32_t p = 0; __any(q0 + p < q1); p += 64) {
                 bool is[4];
 #pragma unroll
                 for (int h = 0; h < 4; ++h) {
-                    const int q = q0 + p + 16 * h + sub;
+                    const uint32_t q = q0 + p + 16 * h + sub;
                     is[h] = q < q1 && nbr_j[q] == i;
                 }
                 uint64_t hits[4];
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(256) void k_nbr_rev(int natoms, const int32_t* __re
 #pragma unroll
                     for (int h = 3; h >= 0; --h) {
                         const uint32_t f = (uint32_t)(hits[h] >> (16 * g)) & 0xffffu;
-                        if (f) found = qa + p + 16 * h + __ffs((int)f) - 1;
+                        if (f) found = (int)(qa + p + 16 * h + __ffs((int)f) - 1);
                     }
                 }
             }
@@ -381,20 +384,20 @@ __global__ __launch_bounds__(256) void k_nbr_rev(int natoms, const int32_t* __re
         const bool ok = !mine || (found >= 0 && shift[f] == s0 && shift[nnbr + f] == s1 && shift[2 * nnbr + f] == s2);
         for (uint64_t bad = __ballot(!ok); bad; bad &= bad - 1) {
             const int l = __ffsll((unsigned long long)bad) - 1;
-            const int q1 = __builtin_amdgcn_readlane(qb, l);
+            const uint32_t q1 = __builtin_amdgcn_readlane(qb, l);
             const int t0 = __builtin_amdgcn_readlane(s0, l), t1 = __builtin_amdgcn_readlane(s1, l),
                       t2 = __builtin_amdgcn_readlane(s2, l);
             int at = -1;
-            for (int q = __builtin_amdgcn_readlane(qa, l); q < q1 && at < 0; q += 64) {
-                const int64_t p = q + lane;
+            for (uint32_t q = __builtin_amdgcn_readlane(qa, l); q < q1 && at < 0; q += 64) {
+                const uint32_t p = q + lane;
                 const bool is = p < q1 && nbr_j[p] == i && shift[p] == t0 && shift[nnbr + p] == t1 &&
                                 shift[2 * nnbr + p] == t2;
                 const uint64_t hit = __ballot(is);
-                if (hit) at = q + __ffsll((unsigned long long)hit) - 1;
+                if (hit) at = (int)(q + __ffsll((unsigned long long)hit) - 1);
             }
             if (lane == l) found = at;
         }
-        if (mine) rev[mb + lane] = found;
+        if (mine) rev[(int64_t)mb + lane] = found;
         if (__any(mine && found < 0) && lane == 0) atomicOr(flag, 2);
     }
 }
@@ -442,9 +445,10 @@ __global__ __launch_bounds__(256) void k_nbr_forces(int natoms, int per, const i
     double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int64_t q = g0; q < g0 + per; ++q) {
         const int64_t k = q * FA_ATOMS + (tid >> 4);
-        const int m0 = k < n ? off[k] : 0, m1 = k < n ? off[k + 1] : 0;
+        // unsigned, as in k_nbr_rev
+        const uint32_t m0 = k < n ? max(off[k], 0) : 0, m1 = k < n ? max(off[k + 1], 0) : 0;
         double f[3] = {0, 0, 0};
-        for (int mb = m0 + sub; mb < m1; mb += 64) {
+        for (uint32_t mb = m0 + sub; mb < m1; mb += 64) {
             int r[4];
             double gm[4][3], gr[4][3], x[4][3];
 #pragma unroll
