@@ -78,6 +78,14 @@ __device__ __forceinline__ int xcd_share(int b, int n) {
     return x * q + min(x, r) + (b >> 3);
 }
 
+// Workgroups of 256 threads, `first` on, in launches of fewer than 2^32 threads
+// each (what a launch takes): launch(first, workgroups).
+template <typename F>
+void in_launches(int64_t nwg, F launch) {
+    constexpr int64_t most = ((int64_t)1 << 24) - 1;
+    for (int64_t w = 0; w < nwg; w += most) launch((int)w, dim3((unsigned)std::min(most, nwg - w)));
+}
+
 // The atoms' data in bin order, so that the search reads a row of bins as one
 // stretch of memory.
 __global__ __launch_bounds__(256) void k_nbr_gather(int n, const int32_t* __restrict__ bin_atoms,
@@ -106,7 +114,7 @@ __global__ __launch_bounds__(256) void k_nbr_gather(int n, const int32_t* __rest
 // thread per atom, whose lanes diverged at every hit and stored 4 or 8 bytes
 // to a line of their own.
 template <bool FILL>
-__global__ __launch_bounds__(256) void k_nbr_search(NbrArgs a, int32_t* __restrict__ cnt,
+__global__ __launch_bounds__(256) void k_nbr_search(NbrArgs a, int first, int32_t* __restrict__ cnt,
                                                     const int32_t* __restrict__ off, int64_t nnbr,
                                                     int32_t* __restrict__ env_off, int32_t* __restrict__ nbr_j,
                                                     int32_t* __restrict__ shift, double* __restrict__ xyz,
@@ -115,8 +123,9 @@ __global__ __launch_bounds__(256) void k_nbr_search(NbrArgs a, int32_t* __restri
     __shared__ int2 ring[4][FILL ? 128 : 1];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
-    const int t = xcd_share(blockIdx.x, gridDim.x) * 4 + wave;
-    if (t >= a.natoms) return;  // whole waves; the kernel has no barrier
+    const int64_t tw = ((int64_t)first + xcd_share(blockIdx.x, gridDim.x)) * 4 + wave;
+    const int t = (int)tw;
+    if (tw >= a.natoms) return;  // whole waves; the kernel has no barrier
     const int64_t n = a.natoms;
     const int i = a.bin_atoms[t];
     const int b = a.bin[i];
@@ -327,13 +336,13 @@ __global__ __launch_bounds__(256) void k_nbr_scan(int n, const int32_t* __restri
 // those loads: checking every match where it was found took 214 us for 55,296
 // atoms of 54 neighbours, this 143; one thread per entry, with a search for its
 // atom and a scan of the list one entry after the other, 422.
-__global__ __launch_bounds__(256) void k_nbr_rev(int natoms, const int32_t* __restrict__ atoms,
+__global__ __launch_bounds__(256) void k_nbr_rev(int natoms, int first, const int32_t* __restrict__ atoms,
                                                  const int32_t* __restrict__ off, const int32_t* __restrict__ nbr_j,
                                                  const int32_t* __restrict__ shift, int64_t nnbr,
                                                  int32_t* __restrict__ rev, int32_t* __restrict__ flag) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
-    const int t = xcd_share(blockIdx.x, gridDim.x) * 4 + wave;
+    const int64_t t = ((int64_t)first + xcd_share(blockIdx.x, gridDim.x)) * 4 + wave;
     if (t >= natoms) return;
     const int i = atoms[t];
     // entries are counted without a sign: a list may end at 2^31 - 1, and the
@@ -403,12 +412,12 @@ __global__ __launch_bounds__(256) void k_nbr_rev(int natoms, const int32_t* __re
 }
 
 // New relative positions of the entries: 16 lanes per atom.
-__global__ __launch_bounds__(256) void k_nbr_update(int natoms, NbrArgs a, const double* __restrict__ pos,
+__global__ __launch_bounds__(256) void k_nbr_update(int natoms, int first, NbrArgs a, const double* __restrict__ pos,
                                                     const int32_t* __restrict__ off, const int32_t* __restrict__ nbr_j,
                                                     const int32_t* __restrict__ shift, int64_t nnbr,
                                                     double* __restrict__ xyz) {
     const int64_t n = natoms;
-    const int64_t i = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    const int64_t i = ((int64_t)first + blockIdx.x) * 16 + (threadIdx.x >> 4);
     if (i >= n) return;
     // entries outside the offsets belong to the first and the last atom
     const int64_t m0 = i == 0 ? 0 : max(off[i], 0), m1 = i == n - 1 ? nnbr : min((int64_t)off[i + 1], nnbr);
@@ -811,9 +820,11 @@ extern "C" int ace_nbrlist_build(ace_nbrlist* nl, int64_t natoms, const double* 
     hipLaunchKernelGGL(k_nbr_gather, dim3(nblk), dim3(256), 0, st, n, (const int32_t*)nl->bin_atoms.p,
                        (const double*)nl->pw.p, pos, (const int32_t*)nl->wrap.p, nl->sp.p, nl->sx.p, nl->sw.p);
     const NbrArgs a = grid_args(nl, cell);
-    const unsigned nwg = (unsigned)(((int64_t)n + 3) / 4);
-    hipLaunchKernelGGL(k_nbr_search<false>, dim3(nwg), dim3(256), 0, st, a, nl->cnt.p, nullptr, (int64_t)0, nullptr,
-                       nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+    const int64_t nwg = ((int64_t)n + 3) / 4;
+    in_launches(nwg, [&](int first, dim3 grid) {
+        hipLaunchKernelGGL(k_nbr_search<false>, grid, dim3(256), 0, st, a, first, nl->cnt.p, nullptr, (int64_t)0,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+    });
     hipLaunchKernelGGL(k_nbr_scan_sum, dim3(nscan), dim3(256), 0, st, n, (const int32_t*)nl->cnt.p, nl->bsum.p);
     hipLaunchKernelGGL(k_nbr_scan, dim3(nscan), dim3(256), 0, st, n, (const int32_t*)nl->cnt.p,
                        (const int64_t*)nl->bsum.p, nl->off.p, &nl->dmail.p->total);
@@ -827,12 +838,17 @@ extern "C" int ace_nbrlist_build(ace_nbrlist* nl, int64_t natoms, const double* 
                 " neighbour entries (*nnbr_out holds the size needed)");
         return ACE_ERR_CAPACITY;
     }
-    hipLaunchKernelGGL(k_nbr_search<true>, dim3(nwg), dim3(256), 0, st, a, nullptr, (const int32_t*)nl->off.p, total,
-                       env_offsets, nbr_j, shift, xyz, atom_species, nbr_species, flag);
+    in_launches(nwg, [&](int first, dim3 grid) {
+        hipLaunchKernelGGL(k_nbr_search<true>, grid, dim3(256), 0, st, a, first, nullptr, (const int32_t*)nl->off.p,
+                           total, env_offsets, nbr_j, shift, xyz, atom_species, nbr_species, flag);
+    });
     HIP_TRY(hipGetLastError());
     if (rev && total > 0) {
-        hipLaunchKernelGGL(k_nbr_rev, dim3(nwg), dim3(256), 0, st, n, (const int32_t*)nl->bin_atoms.p,
-                           (const int32_t*)nl->off.p, (const int32_t*)nbr_j, (const int32_t*)shift, total, rev, flag);
+        in_launches(nwg, [&](int first, dim3 grid) {
+            hipLaunchKernelGGL(k_nbr_rev, grid, dim3(256), 0, st, n, first, (const int32_t*)nl->bin_atoms.p,
+                               (const int32_t*)nl->off.p, (const int32_t*)nbr_j, (const int32_t*)shift, total, rev,
+                               flag);
+        });
         HIP_TRY(hipGetLastError());
     }
     if (read_back()) return -1;
@@ -853,8 +869,10 @@ extern "C" int ace_nbrlist_update(ace_nbrlist* nl, int64_t natoms, const double*
     HIP_TRY(hipSetDevice(nl->device));
     NbrArgs a{};
     for (int q = 0; q < 9; ++q) a.cell[q] = cell[q];
-    hipLaunchKernelGGL(k_nbr_update, dim3((unsigned)((natoms + 15) / 16)), dim3(256), 0, (hipStream_t)stream,
-                       (int)natoms, a, pos, env_offsets, nbr_j, shift, nnbr, xyz);
+    in_launches((natoms + 15) / 16, [&](int first, dim3 grid) {
+        hipLaunchKernelGGL(k_nbr_update, grid, dim3(256), 0, (hipStream_t)stream, (int)natoms, first, a, pos,
+                           env_offsets, nbr_j, shift, nnbr, xyz);
+    });
     HIP_TRY(hipGetLastError());
     return 0;
 }

@@ -1,9 +1,13 @@
 """Neighbour lists near the entry points' limits (gpu): 2^31 - 48 entries, where
-steps of 64 entries pass the largest 32-bit number."""
+steps of 64 entries pass the largest 32-bit number, and more than 2^26 atoms,
+whose waves are more threads than one launch takes."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
+from acehip._lib import check
 from acehip.atoms import NeighbourList
 
 pytestmark = pytest.mark.gpu
@@ -43,4 +47,61 @@ def test_entries_up_to_the_limit(cuda):
     want = (dE[:, e] - dE[:, nl.rev[e].long()]).view(3, len(atoms), k).sum(2)
     assert torch.equal(F[:, atoms], want)
     del dE, F, nl
+    torch.cuda.empty_cache()
+
+
+def test_more_atoms_than_one_launch_takes(cuda):
+    """2^26 sites of a cubic lattice of spacing 1 without neighbours within 0.9,
+    and five atoms half-way between two of them."""
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GiB of device memory")
+    n0, dims = 1 << 26, (512, 512, 256)
+    print(f"[gpu] {n0 + 5} atoms", flush=True)
+    i = torch.arange(n0, device="cuda:0")
+    site = torch.stack([i // (dims[1] * dims[2]), i // dims[2] % dims[1], i % dims[2]]).double()
+    near = torch.tensor([0, 12345678, n0 // 2, n0 - 1000, n0 - 1], device="cuda:0")
+    step = torch.tensor([[0.5], [0.0], [0.0]], dtype=torch.float64, device="cuda:0")
+    pos = torch.cat([site, site[:, near] + step], 1).contiguous()
+    del i, site
+    nl = NeighbourList(0).build(pos, np.diag(np.array(dims, dtype=float)), [1, 1, 1], 0.9)
+    other = (near + dims[1] * dims[2]) % n0  # the next site along x
+    assert nl.nnbr == 20
+    cnt = torch.zeros(n0 + 5, dtype=torch.int64, device="cuda:0")
+    cnt[n0:] = 2
+    for s in (near, other):
+        cnt[s] += 1
+    assert torch.equal((nl.offsets[1:] - nl.offsets[:-1]).long(), cnt)
+    i = torch.repeat_interleave(torch.arange(n0 + 5, device="cuda:0"), cnt)
+    assert torch.equal(nl.nbr_j[-10:].long().view(5, 2).sort(1).values, torch.stack([near, other], 1).sort(1).values)
+    rev = nl.rev.long()
+    assert torch.equal(nl.nbr_j[rev].long(), i) and torch.equal(nl.shift[:, rev], -nl.shift)
+    assert torch.equal(nl.xyz.abs()[0], torch.full((20,), 0.5, dtype=torch.float64, device="cuda:0"))
+    assert not nl.xyz[1:].any()
+    nl.update(pos + 0.25 * torch.arange(n0 + 5, device="cuda:0").eq(n0 + 4))
+    assert torch.equal(nl.xyz[:, -2:].abs().sum(0).sort().values,
+                       torch.tensor([0.75, 1.25], dtype=torch.float64, device="cuda:0"))
+    del pos, cnt, i, nl
+    torch.cuda.empty_cache()
+
+
+def test_update_of_more_atoms_than_one_launch_takes(cuda):
+    """2^28 + 32 atoms at 16 threads each; the last has the only two entries."""
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GiB of device memory")
+    n = (1 << 28) + 32
+    print(f"[gpu] update of {n} atoms", flush=True)
+    pos = torch.zeros((3, n), dtype=torch.float64, device="cuda:0")
+    pos[:, 5] = 1.0
+    pos[0, n - 1] = 4.0
+    off = torch.zeros(n + 1, dtype=torch.int32, device="cuda:0")
+    off[n] = 2
+    nl = NeighbourList(0)
+    j = torch.tensor([5, 7], dtype=torch.int32, device="cuda:0")
+    shift = torch.tensor([[0, 1], [0, 0], [0, 0]], dtype=torch.int32, device="cuda:0")
+    xyz = torch.full((3, 2), float("nan"), dtype=torch.float64, device="cuda:0")
+    cell = (C.c_double * 9)(10.0, 0, 0, 0, 10.0, 0, 0, 0, 10.0)
+    p = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    check(nl.lib.ace_nbrlist_update(nl.h, n, p(pos), cell, 2, p(off), p(j), p(shift), p(xyz), nl._stream(None)))
+    assert torch.equal(xyz, torch.tensor([[-3.0, 6.0], [1.0, 0.0], [1.0, 0.0]], dtype=torch.float64, device="cuda:0"))
+    del pos, off, nl
     torch.cuda.empty_cache()
