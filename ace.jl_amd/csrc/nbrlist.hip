@@ -128,6 +128,11 @@ __global__ __launch_bounds__(256) void k_nbr_search(NbrArgs a, int first, int32_
     if (tw >= a.natoms) return;  // whole waves; the kernel has no barrier
     const int64_t n = a.natoms;
     const int i = a.bin_atoms[t];
+    // positions that are refused may all lie in one bin
+    if (!FILL && (*flag & 12)) {
+        if (lane == 0) cnt[i] = 0;
+        return;
+    }
     const int b = a.bin[i];
     const int bx = b % a.nb[0], by = (b / a.nb[0]) % a.nb[1], bz = b / (a.nb[0] * a.nb[1]);
     const double pix = a.sp[t], piy = a.sp[n + t], piz = a.sp[2 * n + t];
@@ -782,8 +787,8 @@ extern "C" int ace_nbrlist_build(ace_nbrlist* nl, int64_t natoms, const double* 
     HIP_TRY(hipGetLastError());
     // The bins of a cell that is periodic along all axes do not depend on the
     // positions: only open axes wait for their extents here.  Positions found
-    // invalid above are wrapped to some bin and match nothing, or are searched
-    // in vain; the next read back refuses them.
+    // invalid above are wrapped to some bin and not searched; the next read back
+    // refuses them.
     const bool open = !(geo.pbc[0] && geo.pbc[1] && geo.pbc[2]);
     if (open) {
         hipLaunchKernelGGL(k_nbr_minmax, dim3(1), dim3(256), 0, st, (int)nblk, (const double*)nl->bmm.p,
@@ -823,7 +828,7 @@ extern "C" int ace_nbrlist_build(ace_nbrlist* nl, int64_t natoms, const double* 
     const int64_t nwg = ((int64_t)n + 3) / 4;
     in_launches(nwg, [&](int first, dim3 grid) {
         hipLaunchKernelGGL(k_nbr_search<false>, grid, dim3(256), 0, st, a, first, nl->cnt.p, nullptr, (int64_t)0,
-                           nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+                           nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, flag);
     });
     hipLaunchKernelGGL(k_nbr_scan_sum, dim3(nscan), dim3(256), 0, st, n, (const int32_t*)nl->cnt.p, nl->bsum.p);
     hipLaunchKernelGGL(k_nbr_scan, dim3(nscan), dim3(256), 0, st, n, (const int32_t*)nl->cnt.p,

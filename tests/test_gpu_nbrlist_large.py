@@ -1,13 +1,15 @@
 """Neighbour lists near the entry points' limits (gpu): 2^31 - 48 entries, where
 steps of 64 entries pass the largest 32-bit number, and more than 2^26 atoms,
-whose waves are more threads than one launch takes."""
+whose waves are more threads than one launch takes; and many positions that
+are not finite."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
 import torch
 
-from acehip._lib import check
+from acehip._lib import AceError, check
 from acehip.atoms import NeighbourList
 
 pytestmark = pytest.mark.gpu
@@ -105,3 +107,22 @@ def test_update_of_more_atoms_than_one_launch_takes(cuda):
     assert torch.equal(xyz, torch.tensor([[-3.0, 6.0], [1.0, 0.0], [1.0, 0.0]], dtype=torch.float64, device="cuda:0"))
     del pos, off, nl
     torch.cuda.empty_cache()
+
+
+def test_positions_gone_bad_are_refused_at_once(cuda):
+    """They all fall into one bin, where a search would compare each of the
+    three million with every other (over ten seconds)."""
+    n = 3_000_000
+    print(f"[gpu] {n} positions that are not numbers", flush=True)
+    nl = NeighbourList(0)
+    cell = 150.0 * np.eye(3)
+    for value, text in ((float("nan"), "finite"), (1e12, "too far outside")):
+        bad = torch.full((3, n), value, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        with pytest.raises(AceError, match=text):
+            nl.build(bad, cell, [1, 1, 1], 5.0)
+        assert time.perf_counter() - t < 2.0
+    # the list still works
+    x = torch.tensor([[1.0, 2.0], [1.0, 1.0], [1.0, 1.0]], dtype=torch.float64, device="cuda:0")
+    assert nl.build(x, cell, [1, 1, 1], 5.0).nnbr == 2
