@@ -31,6 +31,7 @@ from __future__ import annotations
 
 import numpy as np
 import torch
+import torch.autograd.forward_ad as fwAD
 
 from .evaluator import EnvBatch, HIPEvaluator
 
@@ -40,13 +41,19 @@ def _env_of(offsets: torch.Tensor, nnbr: int) -> torch.Tensor:
     return torch.bucketize(torch.arange(nnbr, device=offsets.device), offsets[1:].long(), right=True)
 
 
-def _weighted(ev, gE, B):
-    """sum_env gE[env] B[env]: the library's kernel for plain tensors; where a
-    graph is being recorded through gE, or gE is a wrapped one (vmap), torch's."""
-    rows = getattr(ev, "weighted_rows", None)
+def _plain(t: torch.Tensor) -> bool:
+    """Whether t is no more than its memory: no subclass, no wrapper (vmap), no
+    tangent of forward-mode derivatives, no pending negation, no implicit zeros."""
     F = torch._C._functorch
-    if (rows is None or (gE.requires_grad and torch.is_grad_enabled()) or F.is_functorch_wrapped_tensor(gE)
-            or F.is_legacy_batchedtensor(gE)):
+    return (type(t) is torch.Tensor and not F.is_functorch_wrapped_tensor(t) and not F.is_legacy_batchedtensor(t)
+            and fwAD.unpack_dual(t).tangent is None and not t.is_neg() and not t._is_zerotensor())
+
+
+def _weighted(ev, gE, B):
+    """sum_env gE[env] B[env]: the library's kernel for plain tensors; for
+    others, and where a graph is being recorded through gE, torch's."""
+    rows = getattr(ev, "weighted_rows", None)
+    if rows is None or (gE.requires_grad and torch.is_grad_enabled()) or not _plain(gE):
         return gE @ B
     return rows(gE, B)
 
