@@ -116,6 +116,13 @@ class HIPEvaluator:
         _lib.check(self.lib.ace_last_dag_shape(self.ctx, C.byref(p), C.byref(t), C.byref(k)))
         return p.value, t.value, k.value
 
+    def last_dag_kernel(self):
+        """Product-DAG kernel of the last call: "interpreter", "records",
+        "segments", "pairs" or "slots" (None before the first)."""
+        k = C.c_int()
+        _lib.check(self.lib.ace_last_dag_kernel(self.ctx, C.byref(k)))
+        return None if k.value < 0 else ("interpreter", "records", "segments", "pairs", "slots")[k.value]
+
     def __del__(self):
         ctx = getattr(self, "ctx", None)
         if ctx:

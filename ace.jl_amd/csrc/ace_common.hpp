@@ -370,7 +370,8 @@ struct ace_ctx {
     int64_t batch_nenv = -1, batch_nnbr = 0;
     int last_parts = 1;
     int64_t last_tail = 0;  // tiles of the last call that ran one more part
-    int last_kernel = 0;    // product-DAG kernel of the last call: 0 records, else the interpreter's tile width
+    int last_kernel = 0;    // tiles of the last call's product-DAG kernel, as ace_last_dag_shape reports them
+    int last_dag = -1;      // and the kernel (ACE_DAG_..)
     int nrec = 0;           // program records (0: the run interpreter evaluates every call)
     unsigned char* scratch = nullptr;  // device address of this device's allocation-free scratch array
     // scratch

@@ -1154,6 +1154,12 @@ extern "C" int ace_last_dag_shape(ace_ctx* ctx, int* parts, int64_t* tail_tiles,
     return 0;
 }
 
+extern "C" int ace_last_dag_kernel(ace_ctx* ctx, int* kernel) {
+    if (!ctx || !kernel) return set_err("ace_last_dag_kernel: null argument");
+    *kernel = ctx->last_dag;
+    return 0;
+}
+
 extern "C" int ace_set_params(ace_ctx* ctx, const double* c, int64_t nB) {
     if (!ctx || !c) return set_err("ace_set_params: null argument");
     if (nB != ctx->nB) return set_err("ace_set_params: len(c) != len(basis)");
@@ -1563,6 +1569,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
         ctx->last_parts = P;
         ctx->last_tail = nhi;
         ctx->last_kernel = 0;
+        ctx->last_dag = ACE_DAG_PAIRS;
     } else if (use_slots(ctx, nenv, forces)) {
         const acehost::SlotShape sh = slot_shape(ctx, nenv, forces);
         if (launch_slots(ctx, st, nenv, estride, forces, sh, ws)) return -1;
@@ -1572,6 +1579,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
         ctx->last_parts = sh.P;
         ctx->last_tail = sh.nhi;
         ctx->last_kernel = ctx->seg_et == 64 ? 0 : 1;  // as the segment kernel's tiles
+        ctx->last_dag = ACE_DAG_SLOTS;
     } else if (use_records) {
         const int ET = rec_et;
         const int NE = ctx->classed ? 6 : 1;
@@ -1581,6 +1589,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
         const int P = ctx->parts > 0 ? ctx->parts : segment_parts(ctx, ntile, ntask_mode, wc->W);
         ctx->last_parts = P;
         ctx->last_kernel = ET == 64 ? 0 : 1;  // 1: narrower tiles
+        ctx->last_dag = ctx->rec_dispatch ? ACE_DAG_RECORDS : ACE_DAG_SEGMENTS;
         // tail tiles with P + 1 parts (P >= 2, so every tile sums shares in k_esum)
         int64_t nhi = 0;
         if (ctx->tail >= 0) {
@@ -1633,6 +1642,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
         }
     } else {
         ctx->last_parts = 1;
+        ctx->last_dag = ACE_DAG_INTERPRETER;
         if (launch_dag_interp(ctx, st, a, nenv, estride, ws, E_out)) return -1;
     }
     HIP_TRY(hipGetLastError());

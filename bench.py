@@ -65,11 +65,12 @@ def algorithmic_flops(pack, forces=True):
     return fe + float(np.sum(6 * c + 4 * o2))
 
 
-def executed_flops(pack, forces=True, kernel=0):
-    """FLOPs the product-DAG kernel executes per environment.
+def executed_flops(pack, forces=True, kernel="segments", tiles=0):
+    """FLOPs the product-DAG kernel executes per environment (None for the pair
+    and the slot kernel, whose programs are the library's own).
 
-    Segment kernel (kernel code 0 / 1: 64- / 32-environment tiles), per record
-    (a run's leaves cut into records of at most 8, 4 above correlation order
+    Segment kernel (tiles 0 / 1: 64 / fewer environments), per record (a run's
+    leaves cut into records of at most 8, 4 above correlation order
     4) of depth d with s leaves: 4 per leaf, less 2 for the first (a
     multiply), 8 for the complex coefficients of class-split EuclideanVector
     programs (less 4); the whole prefix product, 6 per factor after the first;
@@ -79,30 +80,17 @@ def executed_flops(pack, forces=True, kernel=0):
     4 per leaf, 6 per new prefix product, 8 per run."""
     import numpy as np
     cplx = bool(getattr(pack, "classed", 0))
-    if pair_kernel(pack, kernel) or slot_kernel(pack, kernel):
+    if kernel in ("pairs", "slots"):
         return None
-    if kernel not in (0, 1):
+    if kernel == "interpreter":
         w = pack.work_counts(forces)
         per_leaf = 8.0 if cplx else 4.0
         return per_leaf * w["leaves"] + 6.0 * w["prefix_mults"] + 8.0 * w["runs"]
     d, nl, et = _segment_records(pack, forces)
-    lanes = 64.0 / et if kernel == 1 else 1.0
+    lanes = 64.0 / et if tiles == 1 else 1.0
     per_leaf = 8.0 if cplx else 4.0
     rec = per_leaf * nl - per_leaf / 2 + 6.0 * np.maximum(d - 1, 0) + np.where(d > 0, 8.0, 2.0)
     return float(lanes * np.sum(rec))
-
-
-def pair_kernel(pack, kernel):
-    """Whether the pair kernel took the benchmark's calls (Invariant,
-    correlation order 4 to 7, at most 159 pooled values): its programs are the
-    library's own, so their operations are not counted here."""
-    return kernel == 0 and pack.prop == 0 and 4 <= pack.maxorder <= 7 and len(pack.pool) <= 159
-
-
-def slot_kernel(pack, kernel):
-    """Whether the slot kernel took them (class-split EuclideanVector, order
-    3, at most 319 pooled values), likewise."""
-    return (kernel in (0, 1) and bool(getattr(pack, "classed", 0)) and pack.maxorder == 3 and len(pack.pool) <= 319)
 
 
 def _segment_records(pack, forces):
@@ -123,30 +111,31 @@ def _segment_records(pack, forces):
     return d, nl, et
 
 
-def lds_read_bytes(pack, forces=True, kernel=0):
+def lds_read_bytes(pack, forces=True, kernel="segments", tiles=0):
     """LDS bytes the segment kernel reads per environment: every record reads
     its d prefix factors and s leaves, 16 bytes each per lane; on narrower
     tiles (ET < 64) each environment costs 64 / ET lanes.  None for the other
     kernels."""
     import numpy as np
-    if kernel not in (0, 1) or pair_kernel(pack, kernel) or slot_kernel(pack, kernel):
+    if kernel not in ("segments", "records"):
         return None
     d, nl, et = _segment_records(pack, forces)
-    lanes = 64.0 / et if kernel == 1 else 1.0
+    lanes = 64.0 / et if tiles == 1 else 1.0
     return float(16.0 * lanes * np.sum(d + nl))
 
 
-def dag_kernel_name(pack, code):
-    """The product-DAG kernel of ace_last_dag_shape's code."""
-    if pair_kernel(pack, code):
+def dag_kernel_name(kernel, tiles):
+    """The product-DAG kernel that ran (ace_last_dag_kernel) and its tiles
+    (ace_last_dag_shape's code)."""
+    if kernel == "pairs":
         return "k_pairs (quadratic form in products of two pooled values, 32-environment tiles)"
-    if slot_kernel(pack, code):
+    if kernel == "slots":
         return "k_slots (panels of gradient slots over shared products, 32-environment tiles)"
-    if code == 0:
-        return "k_dags (kind-sorted record segments, 64-environment tiles)"
-    if code == 1:
-        return "k_dags (kind-sorted record segments, tiles of fewer than 64 environments)"
-    return f"k_dag run interpreter ({code}-environment tiles)"
+    if kernel == "interpreter":
+        return f"k_dag run interpreter ({tiles}-environment tiles)"
+    of = "64-environment tiles" if tiles == 0 else "tiles of fewer than 64 environments"
+    return (f"k_dags (kind-sorted record segments, {of})" if kernel == "segments"
+            else f"k_dagr (per-record dispatch, {of})")
 
 
 def cpu_model() -> str:
@@ -397,10 +386,11 @@ def main():
         torch.cuda.synchronize()
 
     pk = ev.pack
-    dag_parts, dag_tail, dag_kernel = ev.last_dag_shape()
+    dag_parts, dag_tail, dag_tiles = ev.last_dag_shape()
+    dag_kernel = ev.last_dag_kernel()
     f_alg = algorithmic_flops(pk, True)
-    f_exe = executed_flops(pk, True, dag_kernel)
-    lds_env = lds_read_bytes(pk, True, dag_kernel)
+    f_exe = executed_flops(pk, True, dag_kernel, dag_tiles)
+    lds_env = lds_read_bytes(pk, True, dag_kernel, dag_tiles)
     dag_avg = float(np.mean(dag_ms))
     achieved = f_alg * b.nenv / (dag_avg * 1e-3) / 1e12
     achieved_exe = None if f_exe is None else f_exe * b.nenv / (dag_avg * 1e-3) / 1e12
@@ -437,7 +427,7 @@ def main():
                      "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
                      "traffic": DAG_TRAFFIC_BYTES.get(b.nenv) if headline else None,
                      "traffic_source": TRAFFIC_SOURCE if headline and b.nenv in DAG_TRAFFIC_BYTES else None,
-                     "kernel": dag_kernel_name(pk, dag_kernel),
+                     "kernel": dag_kernel_name(dag_kernel, dag_tiles),
                      "kernel_ms": round(dag_avg, 4), "dag_parts": dag_parts, "dag_tail_tiles": dag_tail,
                      "flops_per_env_algorithmic": f_alg, "flops_per_env_executed": f_exe,
                      "executed_tflops": None if f_exe is None else round(achieved_exe, 3),

@@ -239,6 +239,15 @@ int ace_set_tail_parts(ace_ctx* ctx, int ntail);
  * Instrumentation; no counterpart in the reference. */
 int ace_last_dag_shape(ace_ctx* ctx, int* parts, int64_t* tail_tiles, int* kernel);
 
+/* Which product-DAG kernel the last evaluation call launched (-1: none yet).
+ * Instrumentation; no counterpart in the reference. */
+#define ACE_DAG_INTERPRETER 0 /* the run interpreter */
+#define ACE_DAG_RECORDS 1     /* the per-record dispatch kernel (ace_set_kernel 2) */
+#define ACE_DAG_SEGMENTS 2    /* the record-segment kernel */
+#define ACE_DAG_PAIRS 3       /* the pair kernel */
+#define ACE_DAG_SLOTS 4       /* the slot kernel */
+int ace_last_dag_kernel(ace_ctx* ctx, int* kernel);
+
 /* Product-DAG kernel choice: 0 (default) the pair kernel for Invariant bases of
  * correlation order 4 to 7 with at most 159 pooled values (order 3: energies,
  * and batches of one tile per compute unit); the slot kernel for class-split
