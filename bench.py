@@ -23,12 +23,14 @@ sys.path.insert(0, os.path.join(ROOT, "ace.jl_amd"))
 METRIC = "env/s energy+forces: plain FP64 vs surrogate at ≤1 meV/atom MAE"
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-# HBM bytes per product-DAG launch on this workload (100k environments, whole
-# tiles), from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs of this script,
-# scaled by the factors a 256 MiB device copy gives the same counters (2.0 for
-# FETCH_SIZE, 1.0 for WRITE_SIZE): 227.7 MB read + 223.2 MB written.  Only valid
-# for the default --nenv; re-measured whenever the kernel changes.
-DAG_TRAFFIC_BYTES = {100_000: 450.9e6}
+# HBM bytes per product-DAG launch on the headline workload, by environments,
+# parts per tile and whether the last tiles take one part more: rocprofv3 --pmc
+# FETCH_SIZE and WRITE_SIZE runs of this script, scaled by the factors a 256 MiB
+# device copy gives the same counters (2.0 for FETCH_SIZE, 1.0 for WRITE_SIZE).
+# Whole tiles 227.7 MB read + 223.2 MB written; two parts, each of which loads
+# A+ and writes a share of G, with a finer tail 276.6 + 453.7.  Re-measured
+# whenever the kernel changes; other shapes were not measured.
+DAG_TRAFFIC_BYTES = {(100_000, 1, False): 450.9e6, (100_000, 2, True): 730.3e6}
 WORKLOAD_NAMES = {
     1: "plain ACE energy+forces, 1000 envs x 12 neighbours, order 3, degree 6, Lmax 4, Invariant, FP64",
     2: "plain ACE energy+forces, 100k envs, nX~Poisson(30) clipped [5,80], order 4, degree 12, Lmax 6, "
@@ -109,6 +111,11 @@ def _segment_records(pack, forces):
     nl = np.minimum(ch, np.repeat(rn, nrec) - ch * q)
     et = min(64, (160 * 1024) // (16 * len(pack.pool)))   # the library's tile width
     return d, nl, et
+
+
+def dag_traffic(kernel, nenv, parts, tail_tiles):
+    """HBM bytes of the pair kernel's launch, None where that shape was not measured."""
+    return DAG_TRAFFIC_BYTES.get((nenv, parts, tail_tiles > 0)) if kernel == "pairs" else None
 
 
 def lds_read_bytes(pack, forces=True, kernel="segments", tiles=0):
@@ -388,6 +395,7 @@ def main():
     pk = ev.pack
     dag_parts, dag_tail, dag_tiles = ev.last_dag_shape()
     dag_kernel = ev.last_dag_kernel()
+    traffic = dag_traffic(dag_kernel, b.nenv, dag_parts, dag_tail) if headline else None
     f_alg = algorithmic_flops(pk, True)
     f_exe = executed_flops(pk, True, dag_kernel, dag_tiles)
     lds_env = lds_read_bytes(pk, True, dag_kernel, dag_tiles)
@@ -425,8 +433,7 @@ def main():
         "roofline": {"bound": "fp64-vector", "compute": "FP64 vector ALU (no MFMA); MI355X FP64 vector peak",
                      "achieved": round(achieved, 3), "peak": FP64_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
-                     "traffic": DAG_TRAFFIC_BYTES.get(b.nenv) if headline else None,
-                     "traffic_source": TRAFFIC_SOURCE if headline and b.nenv in DAG_TRAFFIC_BYTES else None,
+                     "traffic": traffic, "traffic_source": TRAFFIC_SOURCE if traffic else None,
                      "kernel": dag_kernel_name(dag_kernel, dag_tiles),
                      "kernel_ms": round(dag_avg, 4), "dag_parts": dag_parts, "dag_tail_tiles": dag_tail,
                      "flops_per_env_algorithmic": f_alg, "flops_per_env_executed": f_exe,

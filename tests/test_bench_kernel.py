@@ -30,3 +30,11 @@ def test_names():
                                                       ("segments", 1), ("records", 0), ("interpreter", 32))]
     assert [n.split()[0] for n in names] == ["k_pairs", "k_slots", "k_slots", "k_dags", "k_dags", "k_dagr", "k_dag"]
     assert names[3] != names[4] and "32" in names[6]
+
+
+def test_traffic_is_that_of_the_launch():
+    whole, split = bench.dag_traffic("pairs", 100_000, 1, 0), bench.dag_traffic("pairs", 100_000, 2, 102)
+    assert 0 < whole < split  # a split writes its shares of G
+    for k, n, parts, tail in (("pairs", 100_000, 2, 0), ("pairs", 100_000, 3, 5), ("pairs", 50_000, 1, 0),
+                              ("segments", 100_000, 1, 0)):
+        assert bench.dag_traffic(k, n, parts, tail) is None
