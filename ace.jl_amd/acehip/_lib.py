@@ -63,7 +63,7 @@ class AcePack(C.Structure):
 
 
 # every symbol declared in include/acehip.h
-EXPORTS = ("ace_ctx_create", "ace_ctx_create_jl", "ace_compile_check", "ace_last_dag_shape", "ace_last_dag_kernel", "ace_set_kernel", "ace_set_pool_shape", "ace_set_params", "ace_set_tile", "ace_set_parts", "ace_set_tail_parts", "ace_energy",
+EXPORTS = ("ace_ctx_create", "ace_ctx_create_jl", "ace_compile_check", "ace_last_dag_shape", "ace_last_dag_kernel", "ace_last_dag_work", "ace_set_kernel", "ace_set_pool_shape", "ace_set_params", "ace_set_tile", "ace_set_parts", "ace_set_tail_parts", "ace_energy",
            "ace_energy_forces", "ace_basis_A", "ace_basis_AA", "ace_basis_B",
            "ace_basis_dB", "ace_surr_features", "ace_surr_energy_forces",
            "ace_last_timing", "ace_set_validation", "ace_last_error",
@@ -95,6 +95,7 @@ def load(path: str | None = None):
     lib.ace_ctx_create_jl.argtypes = [C.POINTER(AceJlBasis), C.c_int, _f64p, C.c_int64, C.POINTER(vp)]
     lib.ace_compile_check.argtypes = [C.POINTER(AceJlBasis), _i64p]
     lib.ace_last_dag_kernel.argtypes = [vp, C.POINTER(C.c_int)]
+    lib.ace_last_dag_work.argtypes = [vp, C.POINTER(C.c_double), C.POINTER(C.c_double)]
     lib.ace_last_dag_shape.argtypes = [vp, C.POINTER(C.c_int), C.POINTER(C.c_int64), C.POINTER(C.c_int)]
     lib.ace_set_params.argtypes = [vp, _f64p, C.c_int64]
     lib.ace_set_tile.argtypes = [vp, C.c_int]

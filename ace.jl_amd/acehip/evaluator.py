@@ -123,6 +123,13 @@ class HIPEvaluator:
         _lib.check(self.lib.ace_last_dag_kernel(self.ctx, C.byref(k)))
         return None if k.value < 0 else ("interpreter", "records", "segments", "pairs", "slots")[k.value]
 
+    def last_dag_work(self):
+        """(FP64 operations, bytes loaded from LDS) per environment of the last
+        call's launch of the pair or the slot kernel; None for the others."""
+        f, b = C.c_double(), C.c_double()
+        _lib.check(self.lib.ace_last_dag_work(self.ctx, C.byref(f), C.byref(b)))
+        return (f.value, b.value) if f.value > 0 else None
+
     def __del__(self):
         ctx = getattr(self, "ctx", None)
         if ctx:

@@ -372,6 +372,8 @@ struct ace_ctx {
     int64_t last_tail = 0;  // tiles of the last call that ran one more part
     int last_kernel = 0;    // tiles of the last call's product-DAG kernel, as ace_last_dag_shape reports them
     int last_dag = -1;      // and the kernel (ACE_DAG_..)
+    bool last_forces = false;
+    double last_mean_parts = 1.0;  // pair kernel: workgroups per tile
     int nrec = 0;           // program records (0: the run interpreter evaluates every call)
     unsigned char* scratch = nullptr;  // device address of this device's allocation-free scratch array
     // scratch

@@ -1160,6 +1160,23 @@ extern "C" int ace_last_dag_kernel(ace_ctx* ctx, int* kernel) {
     return 0;
 }
 
+extern "C" int ace_last_dag_work(ace_ctx* ctx, double* flops, double* lds_bytes) {
+    if (!ctx || !flops || !lds_bytes) return set_err("ace_last_dag_work: null argument");
+    *flops = 0.0;
+    *lds_bytes = 0.0;
+    const int m = ctx->last_forces ? 0 : 1;
+    if (ctx->last_dag == ACE_DAG_PAIRS) {
+        const acehost::DagWork w = acehost::pair_work(ctx->pairs[m].host, ctx->last_forces, ctx->last_mean_parts);
+        *flops = w.flops;
+        *lds_bytes = w.lds;
+    } else if (ctx->last_dag == ACE_DAG_SLOTS) {
+        const acehost::SlotWork w = acehost::slot_work(ctx->slots[m].host, ctx->last_forces);
+        *flops = w.flops;
+        *lds_bytes = w.lds;
+    }
+    return 0;
+}
+
 extern "C" int ace_set_params(ace_ctx* ctx, const double* c, int64_t nB) {
     if (!ctx || !c) return set_err("ace_set_params: null argument");
     if (nB != ctx->nB) return set_err("ace_set_params: len(c) != len(basis)");
@@ -1556,6 +1573,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
     if (ctx->rec_dispatch && ctx->rec_et == 0 && !ctx->force_interp)
         return set_err("ace_set_kernel mode 2: per-record dispatch needs records (correlation order <= 4, npool <= 320)");
     ctx->last_tail = 0;
+    ctx->last_forces = forces;
     if (use_pairs(ctx, nenv, forces)) {
         int P = 0;
         int64_t nhi = 0;
@@ -1570,6 +1588,7 @@ static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* 
         ctx->last_tail = nhi;
         ctx->last_kernel = 0;
         ctx->last_dag = ACE_DAG_PAIRS;
+        ctx->last_mean_parts = P + (double)nhi / ((nenv + 31) / 32);
     } else if (use_slots(ctx, nenv, forces)) {
         const acehost::SlotShape sh = slot_shape(ctx, nenv, forces);
         if (launch_slots(ctx, st, nenv, estride, forces, sh, ws)) return -1;

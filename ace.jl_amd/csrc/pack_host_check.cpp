@@ -1,6 +1,7 @@
 // CPU test shim over pack_host.hpp and compile_host.hpp: the host-side pack
 // logic and the program compiler of libacehip.so built without HIP (tests
 // build it with the address sanitizer, and plain for the larger bases).
+#include <algorithm>
 #include <complex>
 #include <cstring>
 #include <map>
@@ -360,4 +361,41 @@ extern "C" int acehost_grow_buf(const int64_t* sizes, const int32_t* captured, i
 
 extern "C" int64_t acehost_choose_tail(int64_t ntile, int P, int ncu, double d, double dh) {
     return acehost::choose_tail(ntile, P, ncu, d, dh);
+}
+
+// What the pair kernel (classed packs: the slot kernel) executes per
+// environment: FP64 operations, LDS bytes; and the columns of all panels, the
+// panels, the rows of all panels (slots: steps, pieces, rows).
+extern "C" int acehost_dag_work(const ace_pack* pk, int forces, double* out) {
+    if (!acehost::validate_pack(pk).empty()) return -1;
+    const acehost::PackCopy pc = acehost::copy_pack(pk);
+    const int np = pk->npool;
+    const std::vector<int32_t> pool(pk->pool, pk->pool + 4 * (size_t)np);
+    if (pk->classed) {
+        acehost::SlotProgram sp;
+        if (!acehost::slot_program(pc, pool, std::vector<int32_t>(pk->gslot_ptr, pk->gslot_ptr + np + 1),
+                                   std::vector<int32_t>(pk->gslot_list, pk->gslot_list + pk->gslot_ptr[np]),
+                                   std::vector<int32_t>(pk->gslot_class, pk->gslot_class + pk->ngslots), forces != 0, sp)
+                 .empty())
+            return 1;
+        const acehost::SlotWork w = acehost::slot_work(sp, forces != 0);
+        out[0] = w.flops;
+        out[1] = w.lds;
+        out[2] = (double)(sp.codes.size() / 8 - 3);
+        out[3] = sp.pieces();
+        out[4] = forces ? sp.nslots : 0;
+        return 0;
+    }
+    acehost::PairForm pf;
+    acehost::PairProgram pp;
+    if (!acehost::pair_form(pc, pool, 159, pf).empty() ||
+        !acehost::pair_program(pf, forces != 0, forces ? 1024 : 512, np, 96, pp).empty())
+        return 1;
+    const acehost::DagWork w = acehost::pair_work(pp, forces != 0, 1.0);
+    out[0] = w.flops;
+    out[1] = w.lds;
+    out[2] = (double)(pp.coef.size() - 64) / acehost::PAIR_ROWS;
+    out[3] = (double)std::count_if(pp.panel.begin(), pp.panel.end(), [](int32_t p) { return p >= 0; });
+    out[4] = (double)pf.virt.size();
+    return 0;
 }

@@ -590,6 +590,39 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
     return "";
 }
 
+// What k_pairs executes per environment with `parts` workgroups per tile, as its
+// code has it: FP64 vector operations and bytes that loads take from LDS (the
+// atomic additions to G are neither).  A lane has half an environment.  Order 4,
+// degree 12, whole tiles: 337,990 operations; the counter
+// SQ_INSTS_VALU_FLOPS_FP64 gives 337,984.
+struct DagWork {
+    double flops = 0, lds = 0;
+};
+inline DagWork pair_work(const PairProgram& pp, bool forces, double parts) {
+    DagWork w;
+    for (int32_t at : pp.panel) {
+        if (at < 0) continue;
+        const uint32_t cnt = pp.words[(size_t)at];
+        for (int k = 0; k < 3; ++k) {
+            const int nq = k == 0 ? 4 : k == 1 ? 2 : 1;
+            const double n = cnt >> (10 * k) & (k < 2 ? 1023u : 4095u);
+            // per column a multiplication and a multiply-add, then one multiply-add per row
+            w.flops += n * nq * (3.0 + 2.0 * PAIR_ROWS);
+            w.lds += n * (16.0 + 16.0 * nq);
+        }
+        // per row: both products, and the energy
+        w.flops += PAIR_ROWS * (forces ? 8.0 : 5.0);
+        w.lds += PAIR_ROWS * 32.0;
+    }
+    const double nvirt = (double)pp.virt.size() / 2, nback = (double)pp.back.size() / 2;
+    const double npool = (double)pp.back_ptr.size() - 1;
+    w.flops += parts * (nvirt * 3.0 + (forces ? nback * 4.0 : 0.0));
+    w.lds += parts * (nvirt * 32.0 + (forces ? nback * 32.0 + npool * 8.0 : 0.0));
+    w.flops *= 2.0;
+    w.lds *= 2.0;
+    return w;
+}
+
 // The program's coefficients from those of the leaves.
 inline void pair_coefs(PairProgram& pp, const std::vector<double>& leaf) {
     std::fill(pp.coef.begin(), pp.coef.end(), 0.0);

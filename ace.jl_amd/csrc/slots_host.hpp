@@ -311,6 +311,30 @@ inline SlotShape slot_shape(const SlotProgram& sp, int64_t ntile, int ncu, int p
     return best;
 }
 
+// What k_slots executes per environment, as its code has it: FP64 vector
+// operations and bytes that loads take from LDS.  Two lanes have an environment.
+struct SlotWork {
+    double flops = 0, lds = 0;
+};
+inline SlotWork slot_work(const SlotProgram& sp, bool forces) {
+    SlotWork w;
+    for (int p = 0; p < sp.pieces(); ++p) {
+        const uint32_t* hd = sp.hdr.data() + (size_t)SLOT_HDR * p;
+        // a step: two products of two values, four multiply-adds per row and product
+        w.flops += (double)(hd[1] + hd[2] + hd[3]) * (2.0 * 6.0 + 2.0 * 8.0 * SLOT_ROWS);
+        w.lds += (double)(hd[1] + hd[2] + hd[3]) * 4.0 * 16.0;
+        if (forces) w.flops += 3.0 * 4.0 * SLOT_ROWS;
+        for (int r = 0; r < SLOT_ROWS; ++r) {
+            if (hd[4 + r] == ~0u) continue;
+            w.flops += 6.0 + 2.0 + (forces ? 1.0 : 0.0);  // the slot's share of Q, the half-waves' sum
+            w.lds += 16.0;
+        }
+    }
+    w.flops *= 2.0;
+    w.lds *= 2.0;
+    return w;
+}
+
 // The program's coefficients from those of the leaves and the tasks' constants
 // (complex numbers).
 inline void slot_coefs(SlotProgram& sp, const Coeffs& cf) {

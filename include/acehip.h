@@ -248,6 +248,12 @@ int ace_last_dag_shape(ace_ctx* ctx, int* parts, int64_t* tail_tiles, int* kerne
 #define ACE_DAG_SLOTS 4       /* the slot kernel */
 int ace_last_dag_kernel(ace_ctx* ctx, int* kernel);
 
+/* What that launch executed per environment of a full tile, as the kernel's
+ * code has it: FP64 vector operations and bytes loaded from LDS.  For the pair
+ * and the slot kernel, whose programs are the library's own; else 0 and 0.
+ * Instrumentation; no counterpart in the reference. */
+int ace_last_dag_work(ace_ctx* ctx, double* flops, double* lds_bytes);
+
 /* Product-DAG kernel choice: 0 (default) the pair kernel for Invariant bases of
  * correlation order 4 to 7 with at most 159 pooled values (order 3: energies,
  * and batches of one tile per compute unit); the slot kernel for class-split

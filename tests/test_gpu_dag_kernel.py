@@ -26,10 +26,13 @@ CASES = [
 
 
 def _run(ev, b):
-    ev.energy_forces(b)
-    k = ev.last_dag_kernel()
-    ev.energy(b)
-    return k, ev.last_dag_kernel()
+    got = []
+    for run in (ev.energy_forces, ev.energy):
+        run(b)
+        got.append(ev.last_dag_kernel())
+        work = ev.last_dag_work()  # counted by the library for the kernels with programs of their own
+        assert (work is not None) == (got[-1] in ("pairs", "slots")) and (work is None or min(work) > 0)
+    return tuple(got)
 
 
 @pytest.mark.parametrize("args,kw,nenv,forces,energy", CASES)
