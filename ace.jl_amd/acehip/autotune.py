@@ -14,11 +14,12 @@ Free shape parameters, all timed on the caller's batch:
   rest.
 
 Each shape is run once untimed, then ``reps`` times; the fastest is kept, but
-the library's own parts (0) and the widest workgroup stay where nothing is more than
-1 % faster: the pair and slot kernels have workgroups of their own and leave
-the waves a matter of noise, to which the surrogate's fallback, on the segment
-kernel, is not indifferent (4 waves and 1 part instead of 16 and the automatic parts:
-7.9 ms a step against 4.6).
+the library's own parts (0) and the widest workgroup stay where nothing is
+more than 1 % faster.  The pair and the slot kernel have workgroups of their
+own: where one of them runs, the waves are not timed and the widest workgroup
+is set, for the calls that use the segment kernel even so (the surrogate's
+fallback: 4.6 ms a step with 16 waves, 7.9 with 4, which 1 % of noise in the
+pair kernel's times had let through).
 Results are cached per (basis size, batch size, mode).
 """
 from __future__ import annotations
@@ -83,11 +84,13 @@ def tune(ev, batch, forces: bool = True, reps: int = 3, candidates=None, parts=N
     records = ev.last_dag_shape()[2] in (0, 1)
     pcands = list(parts) if parts else ([0, 1, 2, 3, 4] if records else [1])
     results = {}
-    for W in cands:
-        for P in pcands:
+    for P in pcands:
+        for W in sorted(cands, reverse=True):
             ev.set_tile(W)
             ev.set_parts(P)
             results[(W, P)] = _time_call(fn, reps)
+            if ev.last_dag_kernel() in ("pairs", "slots"):
+                break
     Wbest, Pbest = min(results, key=results.get)
     for W, P in ((max(cands), Pbest), (max(cands), 0)):
         if results.get((W, P), float("inf")) <= 1.01 * results[min(results, key=results.get)]:

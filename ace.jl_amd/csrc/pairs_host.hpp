@@ -593,7 +593,7 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
 // What k_pairs executes per environment with `parts` workgroups per tile, as its
 // code has it: FP64 vector operations and bytes that loads take from LDS (the
 // atomic additions to G are neither).  A lane has half an environment.  Order 4,
-// degree 12, whole tiles: 337,990 operations; the counter
+// degree 12, whole tiles: 337,926 operations; the counter
 // SQ_INSTS_VALU_FLOPS_FP64 gives 337,984.
 struct DagWork {
     double flops = 0, lds = 0;
