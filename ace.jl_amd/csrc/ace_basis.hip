@@ -70,7 +70,6 @@ __global__ void k_B(int64_t nenv, int nB, int nAA, const int32_t* __restrict__ r
 // further: 4,536 neighbours, 139 functions 99 us in 71 waves, 25 in 1,278.
 template <int L>
 __global__ __launch_bounds__(64) void k_dphi(RadialParams rp, int64_t nnbr,
-                                             const int32_t* __restrict__ nbr_env,
                                              const double* __restrict__ xyz,
                                              const int8_t* __restrict__ species,
                                              const int32_t* __restrict__ aspec4, int nA, int per,
@@ -797,7 +796,7 @@ static void launch_dphi(ace_ctx* ctx, hipStream_t st, int64_t nnbr, const double
     const int64_t want = std::max<int64_t>(1, std::min<int64_t>((n + 7) / 8, 8 * ctx->ncu / nblk));
     const int per = (int)((n + want - 1) / want);
     hipLaunchKernelGGL(k_dphi<L>, dim3((unsigned)nblk, (unsigned)((n + per - 1) / per)), dim3(64), 0, st,
-                       radial_params(ctx), nnbr, ctx->nbr_env.p, xyz, ctx->nspecies > 0 ? species : nullptr, rows, n,
+                       radial_params(ctx), nnbr, xyz, ctx->nspecies > 0 ? species : nullptr, rows, n,
                        per, ctx->dphi.p);
 }
 
@@ -827,12 +826,10 @@ static int basis_dB_weights(ace_ctx* ctx, hipStream_t st, int64_t nenv, const in
         ctx->db_ready = true;
     }
     const int64_t estride = ((nenv + 63) / 64) * 64;
-    if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing) || ctx->nbr_env.ensure(nnbr, ctx->capturing) ||
+    if (ctx->Aplus.ensure((size_t)ctx->npool * estride, ctx->capturing) ||
         ctx->dphi.ensure((size_t)nnbr * ctx->npool * 3, ctx->capturing))
         return -1;
     if (launch_pool_any(ctx, st, nenv, off, xyz, nnbr, species, estride, ctx_buffers(ctx), false)) return -1;
-    hipLaunchKernelGGL(k_nbr_env, dim3((unsigned)((nenv + 255) / 256)), dim3(256), 0, st, nenv, off,
-                       ctx->nbr_env.p);
     // the pooled (m >= 0) functions: pool rows are (mu, n, l, m) like aspec rows
     DISPATCH_L(ctx->L, launch_dphi, ctx, st, nnbr, xyz, species, ctx->pool.p, ctx->npool);
     HIP_TRY(hipGetLastError());
