@@ -261,29 +261,21 @@ __global__ __launch_bounds__(1024) void k_pairs(PairArgs a, int64_t nenv, const 
     PairInt* ps = (PairInt*)(uintptr_t)(tail ? a.seq_hi : a.seq) + (tail ? a.seq_ptr_hi : a.seq_ptr)[part];
     const int nround = ps[0];
     ++ps;
-    int po[acehost::PAIR_SLOTS], nt = ps[0];
-#pragma unroll
-    for (int q = 0; q < acehost::PAIR_SLOTS; ++q) po[q] = ps[1 + q * NW + wave];
+    int po = ps[1 + wave], nt = ps[0];
     for (int ri = 0; ri < nround; ++ri) {
         ps += acehost::PAIR_SEQ;
-        const int ntn = ps[0];
-        int pn[acehost::PAIR_SLOTS];
-#pragma unroll
-        for (int q = 0; q < acehost::PAIR_SLOTS; ++q) pn[q] = ps[1 + q * NW + wave];
-        PairSums sums[acehost::PAIR_SLOTS];
-#pragma unroll
-        for (int q = 0; q < acehost::PAIR_SLOTS; ++q) evaluate(po[q], sums[q]);
+        const int ntn = ps[0], pn = ps[1 + wave];
+        PairSums sums;
+        evaluate(po, sums);
         if (FORCES) {
             // the panel's turn: nt barriers in all, its sums after turn + 1 of them
-            static_assert(acehost::PAIR_SLOTS == 1, "one panel's sums are kept");
-            const int pre = sums[0].turn >= 0 ? sums[0].turn + 1 : nt;
+            const int pre = sums.turn >= 0 ? sums.turn + 1 : nt;
             for (int s = 0; s < pre; ++s) __syncthreads();
-            if (sums[0].turn >= 0) scatter(sums[0]);
+            if (sums.turn >= 0) scatter(sums);
             for (int s = pre; s < nt; ++s) __syncthreads();
         }
         nt = ntn;
-#pragma unroll
-        for (int q = 0; q < acehost::PAIR_SLOTS; ++q) po[q] = pn[q];
+        po = pn;
     }
     __syncthreads();
     if (FORCES) {

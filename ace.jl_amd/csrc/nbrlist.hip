@@ -47,8 +47,6 @@ struct NbrArgs {
     double rc2;
     int nb[3], R[3], pbc[3];
     int natoms;
-    const double* pw;          // wrapped positions [3][natoms]
-    const int32_t* wrap;       // wrap counts [3][natoms]
     const int32_t* bin;        // [natoms]
     const int32_t* bin_start;  // [nbins + 1]
     const int32_t* bin_atoms;  // [natoms]
@@ -698,8 +696,6 @@ static NbrArgs grid_args(ace_nbrlist* nl, const double* cell) {
         a.pbc[d] = g.pbc[d];
     }
     a.natoms = nl->natoms;
-    a.pw = nl->pw.p;
-    a.wrap = nl->wrap.p;
     a.bin = nl->bin.p;
     a.bin_start = nl->bin_start.p;
     a.bin_atoms = nl->bin_atoms.p;

@@ -45,9 +45,8 @@ namespace acehost {
 
 constexpr int PAIR_ROWS = 8;     // rows per panel
 constexpr int PAIR_WAVES = 16;   // waves per workgroup
-constexpr int PAIR_SLOTS = 1;    // panels per wave and round
-constexpr int PAIR_SEQ = 1 + PAIR_SLOTS * PAIR_WAVES;  // words of a round: turns, panels [slot][wave]
-constexpr int PAIR_HDR = 4 + 2 * PAIR_ROWS;  // header words of a panel
+constexpr int PAIR_SEQ = 1 + PAIR_WAVES;  // words of a round: turns, panels [wave]
+constexpr int PAIR_HDR = 4 + 2 * PAIR_ROWS;  // header words of a panel (the fourth is not used)
 constexpr int PAIR_MAXP = 8;     // workgroups a tile's rounds can be split over (and one more for tail tiles)
 // Words of a record of nq columns: the shared factor, nq factors.
 constexpr int pair_rec_words(int nq) { return 1 + nq; }
@@ -58,7 +57,7 @@ constexpr int pair_rec_cost(int nq) { return 6 + 12 * nq; }
 constexpr uint32_t PAIR_BACK_IN = 1, PAIR_BACK_OUT = 2;
 
 // One mode's program.  Panel words: [records of 4 | of 2 << 10 | of 1 << 20
-// columns, rows | turn << 8, first coefficient, cost of the records], then per
+// columns, rows | turn << 8, first coefficient, 0], then per
 // row the LDS offsets of its two factors (bit 0 of the second: the second
 // factor is conjugated), then the records: LDS offset of the shared factor (bit 0:
 // conjugated), the offsets of the other factors.  Coefficients of a panel's
@@ -66,7 +65,7 @@ constexpr uint32_t PAIR_BACK_IN = 1, PAIR_BACK_OUT = 2;
 struct PairProgram {
     std::vector<uint32_t> words;
     std::vector<double> coef;
-    std::vector<int32_t> panel;  // [round][slot][wave] first word of the panel, -1: none
+    std::vector<int32_t> panel;  // [round][wave] first word of the panel, -1: none
     std::vector<int32_t> turns;  // [round] sub-phases in which the panels add to G
     std::vector<double> cost;    // [round] clocks of a workgroup, estimated
     // term c[leaf] * scale of coef[at]
@@ -312,7 +311,6 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
     struct Panel {
         std::vector<int32_t> rows, cols;
         double cost = 0;
-        int rec_cost = 0;
         std::vector<int32_t> targets;
         int nrec[3] = {0, 0, 0};
         struct Rec {
@@ -440,8 +438,8 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
             }
         }
         // vector instructions: the records, and per row the products of the scatter
-        for (const auto& r : pn.recs) pn.rec_cost += pair_rec_cost(r.nq);
-        pn.cost = 20.0 + (forces ? 18.0 : 8.0) * pn.rows.size() + pn.rec_cost;
+        pn.cost = 20.0 + (forces ? 18.0 : 8.0) * pn.rows.size();
+        for (const auto& r : pn.recs) pn.cost += pair_rec_cost(r.nq);
         for (int32_t p : pn.rows)
             for (int k : {(int)pf.halves[(size_t)p].a, (int)pf.halves[(size_t)p].d})
                 if (k != npool) pn.targets.push_back(k);
@@ -459,7 +457,7 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
             if (hit[(size_t)k]) return false;
         return true;
     };
-    constexpr int NP = PAIR_SLOTS * PAIR_WAVES;
+    constexpr int NP = PAIR_WAVES;
     constexpr size_t WINDOW = 6 * PAIR_WAVES;
     constexpr int TURNS = 6;  // turns a round is given before it gets more
     while (first < panels.size()) {
@@ -498,18 +496,13 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
             std::stable_sort(got.begin(), got.end(), [&](const auto& x, const auto& y) {
                 return panels[(size_t)x.first].cost > panels[(size_t)y.first].cost;
             });
-            double sum[PAIR_WAVES] = {0}, simd[4] = {0, 0, 0, 0};
-            int n[PAIR_WAVES] = {0};
+            double simd[4] = {0, 0, 0, 0};
             for (const auto& x : got) {
                 int b = -1;
-                for (int w = 0; w < PAIR_WAVES; ++w)
-                    if (n[w] < PAIR_SLOTS &&
-                        (b < 0 || std::make_pair(simd[w & 3], sum[w]) < std::make_pair(simd[b & 3], sum[b])))
-                        b = w;
-                slots[n[b] * PAIR_WAVES + b] = x.first;
-                turn_of[n[b] * PAIR_WAVES + b] = x.second;
-                ++n[b];
-                sum[b] += panels[(size_t)x.first].cost;
+                for (int w = 0; w < NP; ++w)
+                    if (slots[w] < 0 && (b < 0 || simd[w & 3] < simd[b & 3])) b = w;
+                slots[b] = x.first;
+                turn_of[b] = x.second;
                 simd[b & 3] += panels[(size_t)x.first].cost;
             }
         }
@@ -526,7 +519,6 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
             hd[0] = (uint32_t)pn.nrec[0] | (uint32_t)pn.nrec[1] << 10 | (uint32_t)pn.nrec[2] << 20;
             hd[1] = (uint32_t)pn.rows.size() | (uint32_t)turn_of[w] << 8;
             hd[2] = (uint32_t)out.coef.size();
-            hd[3] = (uint32_t)pn.rec_cost;
             for (int r = 0; r < PAIR_ROWS; ++r) {
                 // absent rows: the constant's (their h is zero)
                 const PairForm::Half h = r < (int)pn.rows.size() ? pf.halves[(size_t)pn.rows[(size_t)r]]
