@@ -5,7 +5,8 @@
 //
 // Units: acehip.hip (context, product DAG, energy entry points),
 // ace_pairs.hip (pair kernel: the product DAG of Invariant bases of
-// order 3 and 4), ace_pool.hip (1p basis and pooling), ace_force.hip (adjoint force
+// order 3 to 7), ace_slots.hip (slot kernel: of class-split bases of order 3),
+// ace_pool.hip (1p basis and pooling), ace_force.hip (adjoint force
 // kernels), ace_basis.hip (basis-level evaluate / evaluate_d,
 // adjoint_EVAL_D), ace_surr.hip (learned-surrogate support).
 #pragma once
@@ -293,11 +294,11 @@ struct ace_ctx {
     int rec_et = 0;
     int seg_et = 0;
     bool force_interp = false;
-    // pair kernel programs (energy + forces, energy only) of bases it takes
     // slot kernel (class-split bases): programs, and the force kernel's slot table
     bool slots_ok = false;
     SlotDev slots[2];
     DevBuf<int32_t> slot_ptr, slot_list, slot_cls;
+    // pair kernel programs (energy + forces, energy only) of bases it takes
     bool pairs_ok = false;
     PairDev pairs[2];
     // rec_dispatch: the record kernel that switches per record (ace_set_kernel

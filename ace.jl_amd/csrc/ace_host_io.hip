@@ -61,7 +61,7 @@ int host_call(ace_ctx* ctx, int64_t nenv, const int32_t* off, const double* xyz,
         HIP_TRY(hipMemcpyAsync(ctx->io_w.p, w, sizeof(double) * 3 * nnbr, hipMemcpyHostToDevice, st));
         dw = ctx->io_w.p;
     }
-    // checked above: skip the device entry points' own host copy of the inputs
+    // checked above: skip the device entry points' own checks
     const bool validate = ctx->validate;
     ctx->validate = false;
     const int rc = fn(ctx->io_off.p, ctx->io_xyz.p, dsp, dw, ctx->io_out1.p, n2 > 0 ? ctx->io_out2.p : nullptr,

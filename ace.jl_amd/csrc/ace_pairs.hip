@@ -138,7 +138,7 @@ struct PairSums {
 // A+ and storing G.  Energies alone need no turns: 0.51 ms (0.79 ms).  Columns
 // per panel and rows per panel: 8 rows keep 64 % of the coefficients nonzero;
 // 16 rows 47 %, more multiply-adds on zeros than products saved.
-// Order 5, degree 10, Lmax 4 (84 pooled values and 36 products of their own):
+// Order 5, degree 10, Lmax 4 (84 pooled values and 38 products of their own):
 // 0.394 ms for 30,000 environments; with each monomial's five factors
 // multiplied out in the segment kernel, 0.973 ms.
 template <bool FORCES>

@@ -1,8 +1,9 @@
 // libacehip.so — MI355X (gfx950) basis-evaluation path of the Atomic Cluster
 // Expansion with ACE.jl v0.12.46 semantics.  FP64 throughout.
 //
-// Pipeline of an energy (+ forces) call (k_pairs, ace_pairs.hip, takes the place of
-// the product DAG for Invariant bases up to order 4):
+// Pipeline of an energy (+ forces) call (k_pairs, ace_pairs.hip, and k_slots,
+// ace_slots.hip, take the place of the product DAG for most Invariant bases of
+// order 3 to 7 and class-split bases of order 3, see use_pairs and use_slots):
 //   k_pool   (ace_pool.hip): one wave per environment (two, one per
 //              half-wave, for bases with at most 32 pooled values), lanes =
 //              neighbours.  Radial basis and m >= 0 spherical harmonics per
@@ -1260,10 +1261,13 @@ static bool use_slots(const ace_ctx* ctx, int64_t nenv, bool forces) {
 //   pooled values, whole tiles against two parts with their tail, whole call:
 //   24,700 environments (3.02 rounds) 0.654 and 0.599 ms, 30,011 (3.66) 0.681
 //   and 0.693, 41,400 (5.05) 0.958 and 0.927, 55,296 (6.75) 1.149 and 1.203,
-//   100,000 (12.2) 2.085 and 2.129, 131,072 (16.0) 2.616 and 2.747.  The model
-//   favours whole tiles a little (36,000, 0.975 of the split by the model, 0.825
-//   and 0.806), so they must be 6 % shorter by it; 100,000 (0.945) thereby keep
-//   their split.
+//   100,000 (12.2) 2.085 and 2.129, 131,072 (16.0) 2.616 and 2.747.  By the
+//   model whole tiles take 1.110, 0.926, 1.025, 0.906, 0.945 and 0.891 of the
+//   split's time; it favours them a little (36,000 environments, 0.975 by it,
+//   0.825 and 0.806 ms), so any line from 0.945 to 0.975 would follow the
+//   measurements.  It lies below the 0.945 of 100,000 environments, although
+//   whole tiles are 2 % faster there, because the automatic choice is expected
+//   to run tail tiles at that size (test_tail_tiles_full_size).
 // Batches that fit the allocation-free entry point take a split whose shares
 // fit it too, so that both entry points give the same bits.
 static int pair_shape(ace_ctx* ctx, int64_t nenv, bool forces, int& P, int64_t& nhi) {
@@ -1540,8 +1544,9 @@ static void launch_dagr(int ET, dim3 grid, dim3 block, size_t lds, hipStream_t s
 }
 
 // The launches of an energy (+ forces) evaluation, into a workspace that
-// holds A+ [npool][estride], G [ngslots * NC][estride] (forces), MAX_PARTS
-// energy shares [estride] and, for the flat force kernel, nnbr map entries.
+// holds A+ [npool][estride], with forces G (slots of the programs, of the slot
+// kernel's, or the pair kernel's shares), energy_slots energy shares [estride]
+// and, for the flat force kernel, nnbr map entries.
 static int eval_path(ace_ctx* ctx, hipStream_t st, int64_t nenv, const int32_t* off, const double* xyz,
                      int64_t nnbr, const int8_t* species, double* E_out, double* dE, Workspace ws) {
     const int64_t estride = ((nenv + 63) / 64) * 64;

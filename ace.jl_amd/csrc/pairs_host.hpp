@@ -5,7 +5,7 @@
 // Monomials of more than four factors (correlation order 5 to 7) are first
 // brought to four: products of two pooled values that occur in many of them
 // become values of their own, rows behind the pooled ones (greedily, the product
-// that shortens most monomials next; order 5 of degree 10: 36 rows for 7,128
+// that shortens most monomials next; order 5 of degree 10: 38 rows for 7,128
 // monomials of five factors).  G of such a row u = X_s X_t is passed on in the
 // end: G[s] += G_u X_t, G[t] += G_u X_s.
 //
@@ -27,7 +27,8 @@
 // columns q overlap; a panel's columns are records that share one factor.  The
 // panels are scheduled in rounds, one panel per wave.  The waves of a round
 // add to G in turns (sub-phases), such that the panels of one turn have no
-// target in common: G is summed in a fixed order without atomics between waves.
+// target in common: G is summed in a fixed order, by LDS additions of one wave at a
+// time per target.
 #pragma once
 
 #include <algorithm>
@@ -545,7 +546,8 @@ inline std::string pair_program(const PairForm& pf, bool forces, int row_bytes, 
                 }
         }
         out.turns.push_back(forces ? nt : 0);
-        // measured: an FP64 wave instruction takes 4.6 clocks of its SIMD, an
+        // measured: an FP64 wave instruction takes 4.6 clocks of its SIMD (a probe;
+        // 5.9 of the nominal clock with the whole chip at work), an
         // LDS atomic 9.3 of the CU, a turn's barrier about 150
         out.cost.push_back(4.6 * *std::max_element(simd, simd + 4) + (forces ? 150.0 * nt : 0.0));
     }

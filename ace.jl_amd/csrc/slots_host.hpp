@@ -54,7 +54,7 @@ struct SlotProgram {
 };
 
 // Clocks of a SIMD per step: 2 columns of 2 products and 16 multiply-adds per row
-// of 4.6 clocks, and the addresses and signs; of a piece besides; a step's
+// of 4.6 clocks (a probe; 5.9 with the whole chip at work), and the addresses and signs; of a piece besides; a step's
 // latency in a wave that has its SIMD to itself.
 constexpr double SLOT_STEP = 2 * (4 * SLOT_ROWS + 5) * 4.6 + 80, SLOT_PIECE = 600, SLOT_LATENCY = 500;
 

@@ -218,9 +218,12 @@ int ace_set_params(ace_ctx* ctx, const double* c, int64_t nB);
  * the pack's wave configurations). */
 int ace_set_tile(ace_ctx* ctx, int waves_per_tile);
 
-/* Workgroups per product-DAG tile (Invariant): each runs 1/parts of the
- * tile's tasks, which shortens the last, partly empty round of workgroups.
- * 0 (default) chooses 1 to 4 per call from the tile and CU counts. */
+/* Workgroups per product-DAG tile: each runs 1/parts of the tile's tasks,
+ * which shortens the last, partly empty round of workgroups.  0 (default)
+ * chooses per call from the tile and CU counts (1 to 4; the pair kernel 1 to 8,
+ * the slot kernel 1 to 16).  The slot kernel splits a tile by its own rule
+ * alone: while parts, or tail tiles, are set, class-split bases run the
+ * segment kernel. */
 int ace_set_parts(ace_ctx* ctx, int parts);
 
 /* Tiles at the end of the product-DAG grid (record kernel) that run one more
