@@ -112,20 +112,23 @@ class _OfParams(torch.autograd.Function):
 
 class _OfPositions(torch.autograd.Function):
     """Site energies as a function of xyz.  The pullback is a function of c and
-    gE in turn; c reaches it as the tensor itself (held in ``c_graph``), not as an input, so
-    that a gradient in c does not run this node."""
+    gE in turn; c reaches it as the other node saved it (``params``, None where
+    c needs no gradient), not as an input, so that a gradient in c does not run
+    this node."""
 
     @staticmethod
-    def forward(ctx, xyz, c, E, ev, b, dE, c_graph):
-        ctx.ev, ctx.b, ctx.c_graph = ev, b, c_graph
+    def forward(ctx, xyz, c, E, ev, b, dE, params):
+        ctx.ev, ctx.b, ctx.params = ev, b, params
         ctx.save_for_backward(c, dE)
         return E.view_as(E)
 
     @staticmethod
     def backward(ctx, gE):
-        _, dE = ctx.saved_tensors
+        c, dE = ctx.saved_tensors
         ev, b = ctx.ev, ctx.b
-        g = _Pullback.apply(ctx.c_graph[0], gE.contiguous(), ev, b, dE, _env_of(b.offsets, b.nnbr))
+        if ctx.params is not None and torch.is_grad_enabled():
+            (c,) = ctx.params.saved_tensors  # still there: this node was made later, so it runs first
+        g = _Pullback.apply(c, gE.contiguous(), ev, b, dE, _env_of(b.offsets, b.nnbr))
         return g, None, None, None, None, None, None
 
 
@@ -163,8 +166,8 @@ def site_energies(ev: HIPEvaluator, c: torch.Tensor, offsets, xyz: torch.Tensor,
         ev._autograd_c = c.detach().clone()
     b = EnvBatch(offsets, xyz.detach(), species, device=xyz.device)
     E, dE = ev.energy_forces(b)
-    return _SiteEnergy.apply(_OfParams.apply(c, E, ev, b),
-                             _OfPositions.apply(xyz, c.detach(), E, ev, b, dE, (c,)))
+    of_c = _OfParams.apply(c, E, ev, b)
+    return _SiteEnergy.apply(of_c, _OfPositions.apply(xyz, c.detach(), E, ev, b, dE, of_c.grad_fn))
 
 
 class SiteEnergy(torch.nn.Module):
