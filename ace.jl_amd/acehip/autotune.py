@@ -13,13 +13,15 @@ Free shape parameters, all timed on the caller's batch:
   choice, which also gives the tiles of the last round one more part than the
   rest.
 
-Each shape is run once untimed, then ``reps`` times; the fastest is kept, but
-the library's own parts (0) and the widest workgroup stay where nothing is
-more than 1 % faster.  The pair and the slot kernel have workgroups of their
-own: where one of them runs, the waves are not timed and the widest workgroup
-is set, for the calls that use the segment kernel even so (the surrogate's
-fallback: 4.6 ms a step with 16 waves, 7.9 with 4, which 1 % of noise in the
-pair kernel's times had let through).
+Each shape is run once untimed, then ``reps`` times; the fastest is kept.  On
+the segment kernel the library's own parts (0) and the widest workgroup stay
+where nothing is more than 1 % faster.  The pair and the slot kernel have
+workgroups of their own: where one of them runs, the waves are not timed and
+the widest workgroup is set, for the calls that use the segment kernel even so
+(the surrogate's fallback: 4.6 ms a step with 16 waves, 7.9 with 4, which 1 %
+of noise in the pair kernel's times had let through), and the parts, whose
+times really differ (100,000 order-4 environments: 2.10 ms with whole tiles,
+2.13 with the library's split), are the fastest.
 Results are cached per (basis size, batch size, mode).
 """
 from __future__ import annotations
@@ -83,18 +85,20 @@ def tune(ev, batch, forces: bool = True, reps: int = 3, candidates=None, parts=N
     torch.cuda.synchronize()
     records = ev.last_dag_shape()[2] in (0, 1)
     pcands = list(parts) if parts else ([0, 1, 2, 3, 4] if records else [1])
-    results = {}
+    results, own = {}, set()  # own: shapes of the kernels with workgroups of their own
     for P in pcands:
         for W in sorted(cands, reverse=True):
             ev.set_tile(W)
             ev.set_parts(P)
             results[(W, P)] = _time_call(fn, reps)
             if ev.last_dag_kernel() in ("pairs", "slots"):
+                own.add((W, P))
                 break
     Wbest, Pbest = min(results, key=results.get)
-    for W, P in ((max(cands), Pbest), (max(cands), 0)):
-        if results.get((W, P), float("inf")) <= 1.01 * results[min(results, key=results.get)]:
-            Wbest, Pbest = W, P
+    if (Wbest, Pbest) not in own:
+        for W, P in ((max(cands), Pbest), (max(cands), 0)):
+            if results.get((W, P), float("inf")) <= 1.01 * results[min(results, key=results.get)]:
+                Wbest, Pbest = W, P
     ev.set_tile(Wbest)
     ev.set_parts(Pbest)
     _CACHE[key] = ((Wbest, Pbest), results, pool)

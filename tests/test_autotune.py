@@ -56,6 +56,11 @@ def test_pair_kernel_keeps_the_widest(tuned):
     assert (W, P) == (16, 1) and {w for w, _ in results} == {16}
 
 
+def test_pair_kernel_takes_the_fastest_parts(tuned):
+    W, P, _ = tuned(lambda P: "pairs", lambda W, P: {0: 1.009, 1: 1.0, 2: 1.02, 3: 1.1, 4: 1.2}[P])
+    assert (W, P) == (16, 1)
+
+
 def test_slot_kernel_keeps_its_own_parts(tuned):
     # parts that the caller sets are the segment kernel's, slower here
     W, P, results = tuned(lambda P: "slots" if P == 0 else "segments", lambda W, P: NOISE[W] * (1.0 if P == 0 else 1.5))
@@ -65,3 +70,8 @@ def test_slot_kernel_keeps_its_own_parts(tuned):
 def test_segment_kernel_by_time(tuned):
     W, P, results = tuned(lambda P: "segments", lambda W, P: {4: 1.0, 8: 0.9, 16: 1.1}[W] * (1.0 if P == 2 else 1.05))
     assert (W, P) == (8, 2) and len(results) == 15
+
+
+def test_segment_kernel_keeps_the_librarys_choice_within_one_percent(tuned):
+    W, P, _ = tuned(lambda P: "segments", lambda W, P: 1.009 if (W, P) == (16, 0) else 1.0)
+    assert (W, P) == (16, 0)
